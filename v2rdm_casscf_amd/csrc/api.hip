@@ -23,6 +23,7 @@
 #include "kernels.hpp"
 #include "layout.hpp"
 #include "mlp.hpp"
+#include "redcg.hpp"
 #include "spatial.hpp"
 
 #include <random>
@@ -87,8 +88,11 @@ struct v2g_solver {
     DevBuf<int64_t> d_rowtiles, d_xtiles, d_t2tiles;
     DevBuf<int2> d_g2idx;
     v2g::MapPlan plan;
-    // CG
-    DevBuf<double> r, p, z, Ap, t, partial, scal, jacobi, user_minv, rowpart;
+    // CG: the reduced form of the plain solve (redcg.hpp) and the general form
+    // (preconditioned, flexible, layouts with second-pass rows) work in one slab
+    v2g::RedCG redcg;
+    DevBuf<double> cgmem;
+    DevBuf<double> t, partial, scal, jacobi, user_minv, rowpart;
     bool have_jacobi = false, have_user = false;
     // loop scratch
     DevBuf<double> Ax, Bv, ATy, red;
@@ -165,7 +169,7 @@ struct v2g_solver {
     bool use_graphs = false;
     hipGraphExec_t cg_exec = nullptr;
     const double *cg_exec_y = nullptr, *cg_exec_minv = nullptr;
-    int cg_exec_flex = -1;
+    int cg_exec_kind = -1;                  // 0 plain, 1 flexible, 2 reduced
 
     explicit v2g_solver(const v2g_layout_desc &d);
     ~v2g_solver()
@@ -195,14 +199,23 @@ struct v2g_solver {
     struct CgBufs {
         double *r, *p, *Ap, *t, *partial, *scal, *rowpart;
     };
-    CgBufs own_cg_bufs() { return {r.p, p.p, Ap.p, t.p, partial.p, scal.p, rowpart.p}; }
+    CgBufs own_cg_bufs()
+    {
+        const int64_t n = (L->ncon + 31) / 32 * 32;
+        return {cgmem.p, cgmem.p + n, cgmem.p + 2 * n, t.p, partial.p, scal.p, rowpart.p};
+    }
     // fused iterations: rowpart holds x_tiles squares of A^T p, then three
     // arrays of row_tiles residual partials (the unfused p.Ap partials use the
     // first row_tiles)
     bool fused_cg() const { return V2G_CG_FUSE && plan.t2_tiles == 0 && plan.x_tiles > 0; }
     int64_t rowpart_len() const { return std::max<int64_t>(1, plan.x_tiles + 3 * plan.row_tiles); }
+    // general = true: the final residual stays in own_cg_bufs().r
     int cg(const double *rhs, double *y, double tol, int maxiter, int precond, int flexible,
-           double *res);
+           double *res, bool general = false);
+    int cg_reduced(double *scratch, bool graphs, const double *rhs, double *y, double tol,
+                   int maxiter, double *res);
+    template <class F>
+    hipGraphExec_t cg_graph(double *y, const double *minv, int kind, F enqueue);
     int cg_with(const CgBufs &B, bool graphs, const double *rhs, double *y, double tol, int maxiter,
                 const double *minv, int flexible, double *res);
     void update_xz(double mu, const double *y, const double *c, double *x, double *z,
@@ -290,10 +303,8 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
     }
 
     const int64_t ncon = L->ncon, dimx = L->dimx;
-    r.alloc(ncon);
-    p.alloc(ncon);
-
-    Ap.alloc(ncon);
+    redcg.build({L.get()}, {dl}, d_lay.p);
+    cgmem.alloc(std::max<int64_t>(3 * ((ncon + 31) / 32 * 32), redcg.ok() ? redcg.doubles() : 0));
     t.alloc(dimx);
     partial.alloc(v2g::kPartialArrays * v2g::kRedBlocks);
     rowpart.alloc(rowpart_len());
@@ -580,8 +591,10 @@ double v2g_solver::dot(const double *a, const double *b, int64_t n)
 }
 
 int v2g_solver::cg(const double *rhs, double *y, double tolv, int maxiter, int precond,
-                   int flexible, double *res)
+                   int flexible, double *res, bool general)
 {
+    if (precond == 0 && !flexible && !general && redcg.ok())
+        return cg_reduced(cgmem.p, use_graphs, rhs, y, tolv, maxiter, res);
     const double *minv = nullptr;
     if (precond == 1) { ensure_jacobi(); minv = jacobi.p; }
     else if (precond == 2) {
@@ -591,6 +604,63 @@ int v2g_solver::cg(const double *rhs, double *y, double tolv, int maxiter, int p
         minv = lminv.p;  // the learned diagonal from mlp_infer
     }
     return cg_with(own_cg_bufs(), use_graphs, rhs, y, tolv, maxiter, minv, flexible, res);
+}
+
+// The chunk of kCgChunk iterations that enqueue() puts on the stream, as a graph
+// (kept for the last y, preconditioner and form); null: capture is unsupported
+// here, plain launches from now on
+template <class F>
+hipGraphExec_t v2g_solver::cg_graph(double *y, const double *minv, int kind, F enqueue)
+{
+    if (cg_exec && cg_exec_y == y && cg_exec_minv == minv && cg_exec_kind == kind) return cg_exec;
+    if (cg_exec) { (void)hipGraphExecDestroy(cg_exec); cg_exec = nullptr; }
+    // relaxed mode: the other host threads of a bond scan keep allocating,
+    // copying and synchronizing their own streams while this one captures
+    hipGraph_t g = nullptr;
+    bool ok = hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed) == hipSuccess;
+    if (ok) {
+        enqueue();
+        ok = hipStreamEndCapture(st, &g) == hipSuccess && g;
+    }
+    if (ok) ok = hipGraphInstantiate(&cg_exec, g, nullptr, nullptr, 0) == hipSuccess;
+    if (g) (void)hipGraphDestroy(g);
+    if (!ok) {
+        cg_exec = nullptr;
+        use_graphs = false;
+        (void)hipGetLastError();
+    } else {
+        cg_exec_y = y;
+        cg_exec_minv = minv;
+        cg_exec_kind = kind;
+    }
+    return cg_exec;
+}
+
+// The plain CG in its reduced form, in `scratch` (redcg.doubles() doubles).  The
+// host looks at the convergence test after at most kCgChunk iterations and never
+// enqueues iterations beyond maxiter (rounded up to an even number).
+int v2g_solver::cg_reduced(double *scratch, bool graphs, const double *rhs, double *y, double tolv,
+                           int maxiter, double *res)
+{
+    const v2g::RedBufs B = redcg.carve(scratch);
+    redcg.start(B, rhs, y, tolv, nullptr, nullptr, maxiter, st);
+    double hs[v2g::kRedScal];
+    for (int it = 0;;) {
+        const int n = std::max(2, (std::min(kCgChunk, maxiter - it) + 1) / 2 * 2);
+        hipGraphExec_t exec = nullptr;
+        if (graphs && L->ncon <= kGraphMaxRows && n == kCgChunk)
+            exec = cg_graph(y, nullptr, 2, [&] { redcg.iterate(B, y, kCgChunk, st); });
+        if (exec) HIPCHK(hipGraphLaunch(exec, st));
+        else redcg.iterate(B, y, n, st);
+        it += n;
+        HIPCHK(hipMemcpyAsync(hs, B.scal, sizeof(hs), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        if (hs[v2g::RS_DONE] != 0.0 || it >= maxiter) break;
+    }
+    redcg.finish(B, y, nullptr, st);
+    if (res) *res = hs[v2g::RS_NRM];
+    last_cg_nrm0 = hs[v2g::RS_NRM0];
+    return (int)hs[v2g::RS_ITER];
 }
 
 int v2g_solver::cg_with(const CgBufs &B, bool graphs, const double *rhs, double *y, double tolv,
@@ -633,31 +703,7 @@ int v2g_solver::cg_with(const CgBufs &B, bool graphs, const double *rhs, double 
         }
     };
     hipGraphExec_t exec = nullptr;
-    if (graphs && n <= kGraphMaxRows) {
-        if (!(cg_exec && cg_exec_y == y && cg_exec_minv == minv && cg_exec_flex == flexible)) {
-            if (cg_exec) { (void)hipGraphExecDestroy(cg_exec); cg_exec = nullptr; }
-            // relaxed mode: the other host threads of a bond scan keep allocating,
-            // copying and synchronizing their own streams while this one captures
-            hipGraph_t g = nullptr;
-            bool ok = hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed) == hipSuccess;
-            if (ok) {
-                enqueue_chunk();
-                ok = hipStreamEndCapture(st, &g) == hipSuccess && g;
-            }
-            if (ok) ok = hipGraphInstantiate(&cg_exec, g, nullptr, nullptr, 0) == hipSuccess;
-            if (g) (void)hipGraphDestroy(g);
-            if (!ok) {            // capture unsupported here: stay with plain launches
-                cg_exec = nullptr;
-                use_graphs = false;
-                (void)hipGetLastError();
-            } else {
-                cg_exec_y = y;
-                cg_exec_minv = minv;
-                cg_exec_flex = flexible;
-            }
-        }
-        exec = cg_exec;
-    }
+    if (graphs && n <= kGraphMaxRows) exec = cg_graph(y, minv, flexible ? 1 : 0, enqueue_chunk);
     double hs[v2g::CG_NSLOTS];
     int it = 0;
     for (;;) {
@@ -905,6 +951,7 @@ int v2g_cg_solve(v2g_handle h, const double *rhs, double *y, double tol, int max
     const int it = h->cg(rhs, y, tol, maxiter, precond, flexible, resnorm);
     if (iters) *iters = it;
     HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(h->st));
     API_END
 }
 
@@ -928,6 +975,13 @@ int v2g_cg_solve_noalloc(v2g_handle h, const double *rhs, double *y, double tol,
                                     std::to_string(need) + " doubles of scratch, at most " +
                                     std::to_string(kScratchDoubles) + " (64 MiB) are available");
     double *s = h->scratch_dev;
+    if (precond == 0 && !flexible && h->redcg.ok() && h->redcg.doubles() <= (int64_t)kScratchDoubles) {
+        const int it = h->cg_reduced(s, false, rhs, y, tol, maxiter, resnorm);
+        HIPCHK(hipStreamSynchronize(h->st));
+        if (iters) *iters = it;
+        HIPCHK(hipGetLastError());
+        return 0;
+    }
     v2g_solver::CgBufs B{};
     B.r = s;
     B.p = B.r + up(ncon);
@@ -1099,14 +1153,15 @@ int v2g_bpsdp(v2g_handle h, const v2g_params *prm, const double *c, const double
         }
         if (training)
             HIPCHK(hipMemcpyAsync(h->yprev.p, y, sizeof(double) * ncon, hipMemcpyDeviceToDevice, st));
-        const int iiter = h->cg(h->Bv.p, y, cgtol, prm->cg_maxiter, pc, flex, &res);
+        const int iiter = h->cg(h->Bv.p, y, cgtol, prm->cg_maxiter, pc, flex, &res, training);
         cgtot += iiter;
         // convergence rate of this solve: ln(||r_0|| / ||r||) per iteration
         const double rate = (iiter > 0 && res > 0.0 && h->last_cg_nrm0 > res)
                                 ? std::log(h->last_cg_nrm0 / res) / iiter : -1.0;
         if (training) {
             // the base solve's final residual carries its slowest modes
-            last_loss = h->mlp_train(h->Bv.p, h->r.p, prm->train_batch > 0 ? prm->train_batch : 16384,
+            last_loss = h->mlp_train(h->Bv.p, h->own_cg_bufs().r,
+                                     prm->train_batch > 0 ? prm->train_batch : 16384,
                                      prm->train_steps > 0 ? prm->train_steps : 10,
                                      prm->train_lr > 0 ? prm->train_lr : 2e-3, prm->train_penalty,
                                      rng);
