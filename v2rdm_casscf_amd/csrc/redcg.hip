@@ -9,16 +9,20 @@
 // residual norm: it is summed row by row from c s + B2 u - P mu, never expanded
 // into products of its parts, whose difference would lose the digits of a small
 // residual.  Three launches make an iteration:
-//   direction   beta from the last norms; v, nu, p; t = A^T p on the D entries
-//   residual    alpha from ||A^T p||^2; u, w, mu, om; explicit rows of r and y
-//   norms       one read of s: r.r, r.p and p.p of the self rows
+//   direction   beta from the last norms; v, nu, p; ||A^T p||^2
+//   residual    alpha; u, w, mu, om; explicit rows of r and y
+//   norms       r.r, r.p and p.p of the self rows, one read of s
 // ||p_self||^2 of the next direction follows from the three norms (p' = r + beta p).
 //
-// What bounds it: the norm pass reads s once (212 MB at (50e,50o)); the D2 vectors
-// are read through L2 and the memory-side cache.  Every workgroup re-sums the
-// partials of the pass before (at most kRedMaxBlocks of them, in one order), so
-// alpha and beta are the same bits everywhere without a grid barrier or a launch
-// of their own.
+// What bounds it: at (50e,50o) the bytes of the cells (redrows.hpp), 85 us for each of
+// the three passes, 255 us an iteration against 590 us with the entries in block order
+// (index chains and a divergent branch for every D1 term) and 796 us for the general
+// form; 58 against 74 us at (24e,24o) without symmetry, latency-bound: 23 us at (10e,8o).
+// Norms and residual are two launches because together they need more registers than
+// four workgroups a CU leave (200 us in one, spilling or at three a CU).  Every
+// workgroup re-sums the partials of the pass before (at most kRedMaxBlocks of them, in
+// one order), so alpha and beta are the same bits everywhere without a grid barrier or
+// a launch of their own.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,9 +38,9 @@ namespace {
 
 using namespace rows;
 
-constexpr int kNT = 512;                 // threads per workgroup
+constexpr int kNT = 256;                 // threads per workgroup
 constexpr int kWaves = kNT / 64;
-// workgroups of one launch: four per CU
+// workgroups of one launch: four per CU, what the registers of the passes allow
 constexpr int kRedMaxBlocks = 1024;
 constexpr int kXcds = 8;
 
@@ -69,17 +73,6 @@ __device__ __forceinline__ void block_sums(double (&v)[N], double *sh)
     }
 }
 
-__device__ __forceinline__ int find_segment(const int64_t *__restrict__ t0, int nseg, int64_t b)
-{
-    int lo = 0, hi = nseg;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (t0[mid] <= b) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // workgroup -> problem and place in it; XCD x (workgroups x, x + 8, ...) takes a
 // contiguous eighth, so one L2 serves neighbouring entries
 struct Place {
@@ -103,39 +96,41 @@ __device__ __forceinline__ Place place(const RedProb *prob, const int *blk)
 // runs fn(segment, item, lane) over the tiles of list k that belong to this
 // workgroup: elementwise items one per thread, wavefront items one per wave (all
 // 64 lanes), workgroup items one per tile (all threads)
+// Both orders are fixed, and so are the sums.
 template <class F>
 __device__ __forceinline__ void for_tiles(const Place &pl, int k, F fn)
 {
-    const int nseg = pl.pr->nseg[k];
-    const int64_t *t0 = pl.pr->tile0[k];
-    const int64_t nt = t0[nseg];
-    for (int64_t t = pl.lb; t < nt; t += pl.nb) {
-        const int si = find_segment(t0, nseg, t);
-        const Segment sg = pl.pr->seg[k][si];
-        const int64_t l = t - t0[si];
+    // the lists lead with latency-bound items and end with the cells' streams: every
+    // other workgroup goes through its tiles backwards, so that a CU has both at a time
+    const int nt = pl.pr->ntile[k], mine = pl.lb < nt ? (nt - 1 - pl.lb) / pl.nb + 1 : 0;
+    const RedTile *tiles = pl.pr->tile[k];
+    for (int m = 0; m < mine; m++) {
+        const RedTile &tl = tiles[pl.lb + (pl.lb & 1 ? mine - 1 - m : m) * pl.nb];
+        const Segment &sg = tl.sg;
         if (sg.wave == 0) {
-            const int64_t i = l * kNT + threadIdx.x;
+            const int64_t i = tl.first + threadIdx.x;
             if (i < sg.count) fn(sg, i, 0);
         } else if (sg.wave == 1) {
-            const int64_t i = l * kWaves + (threadIdx.x >> 6);
+            const int64_t i = tl.first + (threadIdx.x >> 6);
             if (i < sg.count) fn(sg, i, (int)(threadIdx.x & 63));
         } else {
-            fn(sg, l, (int)threadIdx.x);
+            fn(sg, tl.first, (int)threadIdx.x);
         }
     }
 }
 
-// the vectors of one problem
+// the vectors of one problem in an iteration of parity par: u0, v0, p0, mu0, nu0 as
+// the iteration before left them, u1, ... as this one leaves them
 struct View {
-    double *g, *u, *w, *v0, *v1, *t, *r, *p0, *p1, *s, *mu, *nu0, *nu1, *om, *ams, *scal;
+    double *g, *t, *w, *u0, *u1, *v0, *v1, *r, *p0, *p1, *s, *mu0, *mu1, *nu0, *nu1, *om, *ams, *scal;
 };
 
 __device__ __forceinline__ View view(const RedBufs &B, const RedProb &p, int prob, int par)
 {
-    // v0 / p0 / nu0: the direction before this iteration, v1 / p1 / nu1: its own
-    return {B.g + p.oD, B.u + p.oD, B.w + p.oD, B.v[par ^ 1] + p.oD, B.v[par] + p.oD, B.t + p.oD,
-            B.r + p.oR, B.p[par ^ 1] + p.oR, B.p[par] + p.oR, B.s + p.oS, B.mu + p.oM,
-            B.nu[par ^ 1] + p.oM, B.nu[par] + p.oM, B.om + p.oM, B.ams + p.oM,
+    const int o = par ^ 1;
+    return {B.g + p.oD, B.t + p.oD, B.w + p.oD, B.u[o] + p.oD, B.u[par] + p.oD, B.v[o] + p.oD,
+            B.v[par] + p.oD, B.r + p.oR, B.p[o] + p.oR, B.p[par] + p.oR, B.s + p.oS, B.mu[o] + p.oM,
+            B.mu[par] + p.oM, B.nu[o] + p.oM, B.nu[par] + p.oM, B.om + p.oM, B.ams + p.oM,
             B.scal + (int64_t)prob * kRedScal};
 }
 
@@ -157,11 +152,98 @@ struct Ptr {
     __device__ __forceinline__ double operator[](int64_t i) const { return a[i]; }
 };
 
-struct GatherD {
-    const double *__restrict__ x;
-    double acc;
-    __device__ __forceinline__ void operator()(int64_t col, double c) { acc += c * x[col]; }
+__device__ __forceinline__ void store_cell(const RedLayout &R, int64_t pos, int64_t cc, int64_t k, double *x,
+                                           const Cell &c)
+{
+#pragma unroll
+    for (int o = 0; o < 4; o++) x[pos + o * cc] = c.ab[o];
+    x[R.nAB + k] = c.aa;
+    x[R.nAB + R.nAA + k] = c.bb;
+}
+
+__device__ __forceinline__ double cell_sq(const Cell &t)
+{
+    return ((t.ab[0] * t.ab[0] + t.ab[1] * t.ab[1]) + (t.ab[2] * t.ab[2] + t.ab[3] * t.ab[3])) +
+           (t.aa * t.aa + t.bb * t.bb);
+}
+
+// The cells of one irrep, one per thread: bases that every thread shares (scalar
+// registers) and one 32-bit byte offset (fewer than 2^30 / 6 cells, redlayout.cc), which
+// spares a 64-bit address per load.
+__device__ __forceinline__ double ld(const double *__restrict__ b, uint32_t off)
+{
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(b) + off);
+}
+
+__device__ __forceinline__ void st(double *__restrict__ b, uint32_t off, double v)
+{
+    *reinterpret_cast<double *>(reinterpret_cast<char *>(b) + off) = v;
+}
+
+struct CellAt {
+    int64_t ab, aa, bb, cc;   // first D2ab / D2aa / D2bb entry of the irrep, cells of the irrep
+    uint32_t off;
+    __device__ __forceinline__ Cell load(const double *__restrict__ x) const
+    {
+        Cell c;
+#pragma unroll
+        for (int o = 0; o < 4; o++) c.ab[o] = ld(x + ab + o * cc, off);
+        c.aa = ld(x + aa, off);
+        c.bb = ld(x + bb, off);
+        return c;
+    }
+    __device__ __forceinline__ void store(double *__restrict__ x, const Cell &c) const
+    {
+#pragma unroll
+        for (int o = 0; o < 4; o++) st(x + ab + o * cc, off, c.ab[o]);
+        st(x + aa, off, c.aa);
+        st(x + bb, off, c.bb);
+    }
 };
+
+// a + f b
+__device__ __forceinline__ Cell cell_axpy(double f, const Cell &b, const Cell &a)
+{
+    Cell c;
+#pragma unroll
+    for (int o = 0; o < 4; o++) c.ab[o] = fma(f, b.ab[o], a.ab[o]);
+    c.aa = fma(f, b.aa, a.aa);
+    c.bb = fma(f, b.bb, a.bb);
+    return c;
+}
+
+__device__ __forceinline__ Cell cell_add(const Cell &a, const Cell &b) { return cell_axpy(1.0, b, a); }
+
+// the record of cell i of an irrep, if its pairs share an orbital (one bit a cell, a
+// wavefront's in one word)
+__device__ __forceinline__ const CellRec *shared_cell(const RedProb &p, const Segment &sg, int64_t i)
+{
+    const int64_t w = sg.aux + __builtin_amdgcn_readfirstlane((int)(i >> 6));
+    const uint64_t b = p.bits[w], m = (uint64_t)1 << (i & 63);
+    return b & m ? p.cell + p.rank[w] + __popcll(b & (m - 1)) : nullptr;
+}
+
+// an entry of the start list's RK_AB / RK_DIAG segments; false: no entry
+__device__ __forceinline__ bool start_entry(const RedLayout &R, const Segment &sg, int64_t i, AbEntry &a)
+{
+    if (sg.kind == RK_DIAG) return diag_ab(R, i, a);
+    a = cell_ab(R, sg.h, i);
+    return true;
+}
+
+__device__ __forceinline__ bool is_ab(const Segment &sg) { return sg.kind == RK_AB || sg.kind == RK_DIAG; }
+
+// slot of a D1 + Q1 row's Q1 part
+__device__ __forceinline__ int64_t q1_slot(const RedLayout &R, const Segment &sg, int64_t i)
+{
+    return R.soff[sg.sub ? SF_Q1B : SF_Q1A] + (sg.start - R.L.xoff[sg.sub ? XB_D1B : XB_D1A][0]) + i;
+}
+
+// the full rows of the explicit rows aligned with cell k of irrep h
+__device__ __forceinline__ int64_t cell_row(const RedLayout &R, const DevLayout &Lo, int j, int h, int64_t k)
+{
+    return (j ? Lo.rowoff[RF_SPIN_ANTI][j - 1][h] : Lo.rowoff[RF_SPIN_D2][0][h]) + (k - R.aa0[h]);
+}
 
 // what the norms of the iteration before say: the stopping rule and the next direction
 struct Eval {
@@ -201,7 +283,7 @@ __device__ __forceinline__ Eval evaluate(const RedBufs &B, const Place &pl, cons
 
 // ---- start of a solve -------------------------------------------------------
 
-// t = (A^T y)_D from the full rows, u = w = v = 0 and the scalars
+// t = (A^T y)_D from the full rows; u, v, w, p, mu, nu, om = 0 and the scalars
 __global__ void __launch_bounds__(kNT, 4)
 k_red_aty(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B,
           const double *__restrict__ y, double tol, const double *__restrict__ tolv,
@@ -216,24 +298,31 @@ k_red_aty(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
         }
         return;
     }
+    const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
     for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
-        if (sg.kind == XS_D1) {
+        if (is_ab(sg)) {
+            AbEntry a;
+            if (start_entry(R, sg, i, a)) V.t[a.pos] = full_at_ab(Lo, a, y);
+        } else if (sg.kind == RK_AA) {
+            const AbEntry a = cell_entry(R, sg.h, i);
+            for (int sp = 0; sp < 2; sp++) V.t[R.nAB + sp * R.nAA + sg.start + i] = full_at_aa(Lo, sp, a, y);
+        } else if (sg.kind == XS_D1) {
             const double a = wave_sum(atu_d1_wave(Lo, sg, i, lane, y));
-            if (lane == 0) {
-                V.t[sg.start + i] = a;
-                V.u[sg.start + i] = V.w[sg.start + i] = V.v0[sg.start + i] = 0.0;
-            }
-        } else if (sg.kind == XS_D2AB || sg.kind == XS_D2AA) {
-            V.t[sg.start + i] = sg.kind == XS_D2AB ? atu_d2ab(Lo, sg, i, y) : atu_d2aa(Lo, sg, i, y);
-            V.u[sg.start + i] = V.w[sg.start + i] = V.v0[sg.start + i] = 0.0;
-        } else if (sg.kind == RK_ROWS) {
+            if (lane == 0) V.t[sg.start + i] = a;
+        } else if (sg.kind == RK_DVEC) {
+            V.u0[i] = V.v0[i] = V.w[i] = V.u1[i] = V.v1[i] = 0.0;
+        } else if (sg.kind == RK_RVEC) {
             V.p0[i] = 0.0;
         } else if (sg.kind == RK_MVEC) {
-            V.mu[i] = V.om[i] = V.nu0[i] = 0.0;
+            V.mu0[i] = V.nu0[i] = V.om[i] = 0.0;
         }
     });
     if (pl.lb == 0 && threadIdx.x == 0) {
+        // the zero that indices without an entry point at
+        V.u0[R.nD] = V.u1[R.nD] = V.v0[R.nD] = V.v1[R.nD] = 0.0;
+        V.r[R.nR] = V.p0[R.nR] = V.p1[R.nR] = 0.0;
+        V.mu0[R.nM] = V.mu1[R.nM] = V.nu0[R.nM] = V.nu1[R.nM] = 0.0;
         double *a = V.scal + RS_A + 6;      // as left by an iteration of parity 1
         a[0] = 0.0;                         // done
         a[1] = 1.0;                         // r.z (the first beta is 0)
@@ -252,15 +341,16 @@ k_red_aty(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
     }
 }
 
-// visits the self rows of one D entry: fn(slot, full row, D2 / D1 part of x minus the
-// maximal-spin part of m)
+// visits the self rows of a start-list item: fn(slot, full row, D2 / D1 part of x
+// minus the maximal-spin part of m)
 template <class X, class M, class F>
 __device__ __forceinline__ void self_slots(const RedLayout &R, const DevLayout &Lo, const Segment &sg,
-                                           int64_t i, const X &x, const M &m, F fn)
+                                           int64_t i, int lane, const X &x, const M &m, F fn)
 {
-    if (sg.kind == XS_D2AB) {
-        const AbEntry a = ab_entry(R.L, sg.h, i);
-        auto one = [&](int f, double o) { fn(R.soff[f][sg.h] + i, self_row_ab(Lo, f, a), o); };
+    if (is_ab(sg)) {
+        AbEntry a;
+        if (!start_entry(R, sg, i, a)) return;
+        auto one = [&](int f, double o) { fn(R.soff[f] + a.pos, self_row_ab(Lo, f, a), o); };
         const SelfAb<X> o(R, a, x);
         if (R.L.q2) one(SF_Q2AB, o.q2);
         if (R.L.g2) {
@@ -275,12 +365,13 @@ __device__ __forceinline__ void self_slots(const RedLayout &R, const DevLayout &
             const D200Ab<X> d(R, a, x);
             for (int k = 0; k < R.nblk_d; k++) one(SF_D0 + k, d.row(R, a, k));
         }
-    } else if (sg.kind == XS_D2AA) {
-        if (R.L.q2)
-            fn(R.soff[sg.sub ? SF_Q2BB : SF_Q2AA][sg.h] + i, Lo.rowoff[RF_Q2AA][sg.sub][sg.h] + i,
-               self_row_aa(R, sg.sub, sg.h, i, x));
-    } else {
-        fn(R.soff[sg.sub ? SF_Q1B : SF_Q1A][sg.h] + i, self_row_d1(Lo, sg.sub, sg.h, i), x[sg.start + i]);
+    } else if (sg.kind == RK_AA) {
+        if (!R.L.q2) return;
+        const AbEntry a = cell_entry(R, sg.h, i);
+        for (int sp = 0; sp < 2; sp++)
+            fn(R.soff[SF_Q2AA + sp] + sg.start + i, Lo.rowoff[RF_Q2AA][sp][sg.h] + i, self_row_aa(R, sp, a, x));
+    } else if (sg.kind == XS_D1 && lane == 0) {
+        fn(q1_slot(R, sg, i), self_row_d1(Lo, sg.sub, sg.h, i), x[sg.start + i]);
     }
 }
 
@@ -297,8 +388,8 @@ k_red_self(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     const DevLayout &Lo = *pl.pr->full;
     const Ptr t{V.t}, ms{y + (R.nM ? Lo.rowoff[RF_MAXSPIN][0][0] : 0)};
     double ss[1] = {0.0};
-    for_tiles(pl, 2, [&](const Segment &sg, int64_t i, int) {
-        self_slots(R, Lo, sg, i, t, ms, [&](int64_t slot, int64_t row, double o) {
+    for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
+        self_slots(R, Lo, sg, i, lane, t, ms, [&](int64_t slot, int64_t row, double o) {
             const double v = rhs[row] - y[row] - o;
             V.s[slot] = v;
             ss[0] += v * v;
@@ -307,7 +398,6 @@ k_red_self(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     block_sums<1>(ss, sh);
     if (threadIdx.x == 0) *part(B, P_RR2, pl.gb) = ss[0];
 }
-
 
 // g = B2^T s, and r = rhs - A (A^T y) on the explicit rows
 __global__ void __launch_bounds__(kNT, 4)
@@ -320,13 +410,26 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     if (V.scal[RS_DONE] != 0.0) return;
     const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
-    const Ptr s{V.s}, ms{y + (R.nM ? Lo.rowoff[RF_MAXSPIN][0][0] : 0)};
+    const Ptr s{V.s}, t{V.t}, ms{y + (R.nM ? Lo.rowoff[RF_MAXSPIN][0][0] : 0)};
     double rr[1] = {0.0};
+    auto row = [&](int64_t k, int64_t full, double at) {
+        const double ri = rhs[full] - at;
+        V.r[k] = ri;
+        rr[0] += ri * ri;
+    };
     for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
-        if (sg.kind == XS_D2AB) {
-            V.g[sg.start + i] = self_at_ab(R, ab_entry(R.L, sg.h, i), s);
-        } else if (sg.kind == XS_D2AA) {
-            V.g[sg.start + i] = self_at_aa(R, sg.sub, sg.h, i, s);
+        if (is_ab(sg)) {
+            AbEntry a;
+            if (start_entry(R, sg, i, a)) V.g[a.pos] = self_at_ab(R, a, s);
+        } else if (sg.kind == RK_AA) {
+            const AbEntry a = cell_entry(R, sg.h, i);
+            const int64_t k = sg.start + i;
+            for (int sp = 0; sp < 2; sp++) V.g[R.nAB + sp * R.nAA + k] = self_at_aa(R, sp, sg.h, a, s);
+            if (R.cells) {
+                double at[3];
+                cell_rows(load_cell(R, a.pos, sg.count, k, t), at);
+                for (int j = 0; j < 3; j++) row(j * R.nAA + k, cell_row(R, Lo, j, sg.h, k), at[j]);
+            }
         } else if (sg.kind == XS_D1) {
             const double a = wave_sum(self_at_d1(R, sg.sub, sg.h, i, lane, s));
             if (lane == 0) V.g[sg.start + i] = a;
@@ -335,39 +438,23 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
             const int pr = R.L.bab[R.L.bab_off[0] + i], k = P0(pr), l = P1(pr);
             double v = ms_row_gram(R, sg.sub, (int)i, lane, ms);
             for (int j = lane; j < R.L.amo; j += 64) {
-                AbEntry a{};
-                a.q = sg.sub ? j : k;
-                a.r = sg.sub ? j : l;
-                a.s = sg.sub ? k : j;
-                a.p = sg.sub ? l : j;
+                const AbEntry a{sg.sub ? l : j, sg.sub ? j : k, sg.sub ? j : l, sg.sub ? k : j, 0};
                 v -= y[self_row_ab(Lo, SF_G2BA, a)];
             }
             v = wave_sum(v);
-            if (lane == 0) {
-                const double ri = rhs[Lo.rowoff[RF_MAXSPIN][sg.sub][0] + i] - v;
-                V.r[sg.start + i] = ri;
-                rr[0] += ri * ri;
-            }
+            if (lane == 0) row(sg.start + i, sg.aux + i, v);
         }
     });
-    for_tiles(pl, 1, [&](const Segment &sg, int64_t i, int lane) {
-        if (sg.kind >= RK_ROWS || sg.kind == RF_MAXSPIN) return;
-        GatherD f{V.t, 0.0};
-        if (sg.wave == 0) {
-            elem_terms(R.L, sg, i, f);
-        } else if (sg.wave == 1) {
-            wave_terms(R.L, sg, i, lane, f);
-            f.acc = wave_sum(f.acc);
-        } else {
-            wave_terms(R.L, sg, i, lane, f, kNT);
-            double a[1] = {f.acc};
-            block_sums<1>(a, sh);
-            f.acc = a[0];
-        }
-        if (sg.wave == 0 || lane == 0) {
-            const double ri = rhs[sg.aux + i] - f.acc;
-            V.r[sg.start + i] = ri;
-            rr[0] += ri * ri;
+    for_tiles(pl, 2, [&](const Segment &sg, int64_t i, int lane) {
+        if (sg.kind == RF_SPIN_D1) {
+            row(sg.start + i, sg.aux + i, t[R.L.xoff[XB_D1A][sg.h] + i] - t[R.L.xoff[XB_D1B][sg.h] + i]);
+        } else if (sg.kind == RF_CONTR) {
+            const double v = wave_sum(long_row(R, sg, i, lane, 64, t));
+            if (lane == 0) row(sg.start + i, sg.aux + i, v);
+        } else if (sg.wave == 2) {
+            double v[1] = {long_row(R, sg, i, lane, kNT, t)};
+            block_sums<1>(v, sh);
+            if (lane == 0) row(sg.start + i, sg.aux + i, v[0]);
         }
     });
     block_sums<1>(rr, sh);
@@ -380,8 +467,11 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
 
 // ---- one iteration ----------------------------------------------------------
 
-// direction: beta and the stopping rule; v, nu, p; t = A^T p on the D entries, the
-// maximal-spin rows of A A^T p, and the sum of t.t and their cross terms
+// direction: beta and the stopping rule; v, nu, p; ||A^T p||^2 (t = A^T p is kept where
+// it is gathered from: listed entries and D1) and the maximal-spin rows of A A^T p
+// FULL: every problem is a singlet with Q2, G2 and spin rows, so no load hides behind a
+// branch; else the flags of each layout decide
+template <bool FULL>
 __global__ void __launch_bounds__(kNT, 4)
 k_red_dir(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B, int par)
 {
@@ -411,40 +501,56 @@ k_red_dir(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
     }
     if (ev.done) return;
     const RedLayout &R = pl.pr->R;
-    const Axpy v{V.u, V.v0, ev.beta}, p{V.r, V.p0, ev.beta}, nu{V.mu, V.nu0, ev.beta};
+    const bool q2 = FULL || R.L.q2, g2 = FULL || R.L.g2, cells = FULL || R.cells;
+    const int nd = FULL ? 1 : R.nblk_d;
+    const Axpy v{V.u0, V.v0, ev.beta}, p{V.r, V.p0, ev.beta}, nu{V.mu0, V.nu0, ev.beta};
     double tt[1] = {0.0};
-    for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
-        if (sg.kind == XS_D2AB) {
-            const int64_t k = sg.start + i;
-            const double t = fma(d, V.g[k], atu_d2ab<false, true>(R.L, sg, i, p)) +
-                             gram_ab(R, ab_entry(R.L, sg.h, i), v, nu);
-            V.t[k] = t;
-            V.v1[k] = v[k];
-            tt[0] += t * t;
-        } else if (sg.kind == XS_D2AA) {
-            const int64_t k = sg.start + i;
-            const double t = fma(d, V.g[k], atu_d2aa<false, true>(R.L, sg, i, p)) +
-                             gram_aa(R, sg.sub, sg.h, i, v);
-            V.t[k] = t;
-            V.v1[k] = v[k];
-            tt[0] += t * t;
+    auto keep = [&](int64_t k, double t) {
+        V.t[k] = t;
+        V.v1[k] = v[k];
+        tt[0] += t * t;
+    };
+    for_tiles(pl, 1, [&](const Segment &sg, int64_t i, int lane) {
+        if (sg.kind == RK_CELLS) {
+            const CellRec *rec = shared_cell(*pl.pr, sg, i);
+            const int64_t k0 = R.aa0[sg.h];
+            const CellAt at{R.ab0[sg.h], R.nAB + k0, R.nAB + R.nAA + k0, sg.count, (uint32_t)i * 8u};
+            const Cell u = at.load(V.u0), v0 = at.load(V.v0), g = at.load(V.g);
+            double pr[3] = {0.0, 0.0, 0.0};
+            if (cells)
+#pragma unroll
+                for (int j = 0; j < 3; j++)
+                    pr[j] = fma(ev.beta, ld(V.p0 + j * R.nAA + k0, at.off), ld(V.r + j * R.nAA + k0, at.off));
+            const Cell vc = cell_axpy(ev.beta, v0, u);
+            Cell t = cell_at(q2, g2, nd, cells, d, g, vc, pr);
+            if (rec) {
+                shared_at(R, *rec, v, nu, p, t);
+                at.store(V.t, t);
+            }
+            tt[0] += cell_sq(t);
+            at.store(V.v1, vc);
+            if (cells)
+#pragma unroll
+                for (int j = 0; j < 3; j++) st(V.p1 + j * R.nAA + k0, at.off, pr[j]);
+        } else if (sg.kind == RK_LIST_AB) {
+            const AbRec a = pl.pr->ab[i];
+            const double t = fma(d, V.g[a.pos], rec_expl_ab(R, a, p)) +
+                             (AbVals(R, a, v).gram(R, a) + (nu[a.m0] + nu[a.m1]));
+            keep(a.pos, t);
         } else if (sg.kind == XS_D1) {
             const int64_t k = sg.start + i;
             const double t = wave_sum(atu_d1_wave<false, true>(R.L, sg, i, lane, p) +
                                       gram_d1(R, sg.sub, sg.h, i, lane, v, nu)) + d * V.g[k];
-            if (lane == 0) {
-                V.t[k] = t;
-                V.v1[k] = v[k];
-                tt[0] += t * t;
-            }
+            if (lane == 0) keep(k, t);
         } else if (sg.kind == RK_ROWS) {
-            V.p1[i] = p[i];
+            V.p1[sg.start + i] = p[sg.start + i];
         } else if (sg.kind == RK_MVEC) {
             V.nu1[i] = nu[i];
         } else {
             // maximal-spin row: (A A^T p) = P^T P p_ms - P^T p_self, and its share
             // of ||A^T p||^2 beyond ||p_self||^2
-            const Axpy ps{V.r + R.L.rowoff[RF_MAXSPIN][0][0], V.p0 + R.L.rowoff[RF_MAXSPIN][0][0], ev.beta};
+            const int64_t m0 = R.L.rowoff[RF_MAXSPIN][0][0];
+            const Axpy ps{V.r + m0, V.p0 + m0, ev.beta};
             const double self = wave_sum(ms_row_self(R, sg.sub, (int)i, lane, d, Ptr{V.s}, v, nu));
             const double gr = wave_sum(ms_row_gram(R, sg.sub, (int)i, lane, ps));
             if (lane == 0) {
@@ -482,44 +588,65 @@ k_red_res(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
         b1[2] = alpha;
     }
     const RedLayout &R = pl.pr->R;
+    const DevLayout &Lo = *pl.pr->full;
+    const Ptr t{V.t};
     double rr[1] = {0.0};
-    for_tiles(pl, 1, [&](const Segment &sg, int64_t i, int lane) {
-        if (sg.kind == RK_DVEC) {
-            const double vi = V.v1[i];
-            V.u[i] = fma(-alpha, vi + V.t[i], V.u[i]);
-            V.w[i] = fma(alpha, vi, V.w[i]);
-            return;
-        }
-        if (sg.kind == RK_MVEC) {
-            const double vi = V.nu1[i];
-            V.mu[i] = fma(-alpha, vi + V.p1[R.L.rowoff[RF_MAXSPIN][0][0] + i], V.mu[i]);
-            V.om[i] = fma(alpha, vi, V.om[i]);
-            return;
-        }
-        double at;
-        if (sg.kind == RF_MAXSPIN) {
-            at = V.ams[sg.sub * (R.nM / 2) + i];
-        } else {
-            GatherD f{V.t, 0.0};
-            if (sg.wave == 0) {
-                elem_terms(R.L, sg, i, f);
-                at = f.acc;
-            } else if (sg.wave == 1) {
-                wave_terms(R.L, sg, i, lane, f);
-                at = wave_sum(f.acc);
-            } else {
-                wave_terms(R.L, sg, i, lane, f, kNT);
-                double s[1] = {f.acc};
-                block_sums<1>(s, sh);
-                at = s[0];
+    auto row = [&](int64_t k, int64_t full, double at) {
+        const double yn = fma(alpha, V.p1[k], y[full]), rn = fma(-alpha, at, V.r[k]);
+        y[full] = yn;
+        V.r[k] = rn;
+        rr[0] = fma(rn, rn, rr[0]);
+    };
+    for_tiles(pl, 2, [&](const Segment &sg, int64_t i, int lane) {
+        if (sg.kind == RK_CELLS) {
+            const CellRec *rec = shared_cell(*pl.pr, sg, i);
+            const int64_t k0 = R.aa0[sg.h];
+            const CellAt at{R.ab0[sg.h], R.nAB + k0, R.nAB + R.nAA + k0, sg.count, (uint32_t)i * 8u};
+            // every load before the first store, so that none waits for another
+            const Cell vc = at.load(V.v1), g = at.load(V.g), u = at.load(V.u0), w = at.load(V.w);
+            double pr[3] = {0.0, 0.0, 0.0}, r[3], yy[3];
+            if (R.cells)
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    pr[j] = ld(V.p1 + j * R.nAA + k0, at.off);
+                    r[j] = ld(V.r + j * R.nAA + k0, at.off);
+                    yy[j] = ld(y + cell_row(R, Lo, j, sg.h, k0), at.off);
+                }
+            Cell tc = cell_at(R.L.q2, R.L.g2, R.nblk_d, R.cells, d, g, vc, pr);
+            if (rec) tc = at.load(V.t);
+            at.store(V.u1, cell_axpy(-alpha, cell_add(vc, tc), u));
+            at.store(V.w, cell_axpy(alpha, vc, w));
+            if (R.cells) {
+                double ct[3];
+                cell_rows(tc, ct);
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const double rn = fma(-alpha, ct[j], r[j]);
+                    rr[0] = fma(rn, rn, rr[0]);
+                    st(V.r + j * R.nAA + k0, at.off, rn);
+                    st(y + cell_row(R, Lo, j, sg.h, k0), at.off, fma(alpha, pr[j], yy[j]));
+                }
             }
-        }
-        if (sg.wave == 0 || lane == 0) {
+        } else if (sg.kind == RK_STEP) {
             const int64_t k = sg.start + i;
-            y[sg.aux + i] = fma(alpha, V.p1[k], y[sg.aux + i]);
-            const double rn = fma(-alpha, at, V.r[k]);
-            V.r[k] = rn;
-            rr[0] = fma(rn, rn, rr[0]);
+            const double v = V.v1[k], u = fma(-alpha, v + V.t[k], V.u0[k]), w = fma(alpha, v, V.w[k]);
+            V.u1[k] = u;
+            V.w[k] = w;
+        } else if (sg.kind == RK_MVEC) {
+            const double v = V.nu1[i], m = V.mu0[i], o = V.om[i];
+            V.mu1[i] = fma(-alpha, v + V.p1[R.L.rowoff[RF_MAXSPIN][0][0] + i], m);
+            V.om[i] = fma(alpha, v, o);
+        } else if (sg.kind == RF_MAXSPIN) {
+            row(sg.start + i, sg.aux + i, V.ams[sg.sub * (R.nM / 2) + i]);
+        } else if (sg.kind == RF_SPIN_D1) {
+            row(sg.start + i, sg.aux + i, t[R.L.xoff[XB_D1A][sg.h] + i] - t[R.L.xoff[XB_D1B][sg.h] + i]);
+        } else if (sg.kind == RF_CONTR) {
+            const double at = wave_sum(long_row(R, sg, i, lane, 64, t));
+            if (lane == 0) row(sg.start + i, sg.aux + i, at);
+        } else if (sg.wave == 2) {
+            double at[1] = {long_row(R, sg, i, lane, kNT, t)};
+            block_sums<1>(at, sh);
+            if (lane == 0) row(sg.start + i, sg.aux + i, at[0]);
         }
     });
     block_sums<1>(rr, sh);
@@ -527,6 +654,7 @@ k_red_res(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
 }
 
 // norms: r.r, r.p, p.p of the self rows, r of this iteration and p its direction
+template <bool FULL>
 __global__ void __launch_bounds__(kNT, 4)
 k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B, int par)
 {
@@ -536,40 +664,98 @@ k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     if (V.scal[RS_A + 6 * par] != 0.0) return;
     const double c = V.scal[RS_B + 3 * par], d = V.scal[RS_A + 6 * par + 2];
     const RedLayout &R = pl.pr->R;
-    const Ptr u{V.u}, v{V.v1}, mu{V.mu}, nu{V.nu1};
+    const bool q2 = FULL || R.L.q2, g2 = FULL || R.L.g2;
+    const int nd = FULL ? 1 : R.nblk_d;
+    const Ptr u{V.u1}, v{V.v1}, mu{V.mu1}, nu{V.nu1};
     double n[3] = {0.0, 0.0, 0.0};
-    auto add = [&](double s, double ru, double pv) {
+    auto self = [&](double s, double ru, double pv) {
         const double r = fma(c, s, ru), p = fma(d, s, pv);
         n[0] = fma(r, r, n[0]);
         n[1] = fma(r, p, n[1]);
         n[2] = fma(p, p, n[2]);
     };
-    for_tiles(pl, 2, [&](const Segment &sg, int64_t i, int) {
-        if (sg.kind == XS_D2AB) {
-            const AbEntry a = ab_entry(R.L, sg.h, i);
-            SelfAb<Ptr> su(R, a, u), sv(R, a, v);
-            const double *s = V.s + i;
-            auto one = [&](int f, double ru, double pv) { add(s[R.soff[f][sg.h]], ru, pv); };
-            if (R.L.q2) one(SF_Q2AB, su.q2, sv.q2);
-            if (R.L.g2) {
-                one(SF_G2AB, su.g1, sv.g1);
-                one(SF_G2BA, su.g2 - ms_part(R, a.p, a.q, a.r, a.s, mu),
-                    sv.g2 - ms_part(R, a.p, a.q, a.r, a.s, nu));
-                one(SF_G2X, su.x, sv.x);
-                one(SF_G2Y, su.x, sv.x);
-                one(SF_G2A, su.ga, sv.ga);
-                one(SF_G2B, su.gb, sv.gb);
+    for_tiles(pl, 3, [&](const Segment &sg, int64_t i, int) {
+        if (sg.kind == RK_CELLS) {
+            const CellRec *rec = shared_cell(*pl.pr, sg, i);
+            const int64_t k0 = R.aa0[sg.h], cc = sg.count;
+            const CellAt at{R.ab0[sg.h], R.nAB + k0, R.nAB + R.nAA + k0, cc, (uint32_t)i * 8u};
+            const uint32_t off = at.off;
+            const Cell uc = at.load(V.u1), vc = at.load(V.v1);
+            const double *s = V.s + at.ab;
+            // rows that a shared orbital does not touch
+            if (g2) {
+#pragma unroll
+                for (int o = 0; o < 4; o++) {
+                    self(ld(s + o * cc + R.soff[SF_G2X], off), uc.ab[o], vc.ab[o]);
+                    self(ld(s + o * cc + R.soff[SF_G2Y], off), uc.ab[o], vc.ab[o]);
+                }
             }
-            if (R.nblk_d) {
-                const D200Ab<Ptr> du(R, a, u), dv(R, a, v);
-                for (int k = 0; k < R.nblk_d; k++) one(SF_D0 + k, du.row(R, a, k), dv.row(R, a, k));
+            for (int b = 0; b < nd; b++) {
+                double cf[4];
+                d200_coef(b, FULL || R.L.singlet, false, false, cf);
+#pragma unroll
+                for (int o = 0; o < 4; o++)
+                    self(ld(s + R.soff[SF_D0 + b] + o * cc, off),
+                         cf[0] * uc.ab[o] + cf[1] * uc.ab[o ^ 1] + cf[2] * uc.ab[o ^ 2] + cf[3] * uc.ab[o ^ 3],
+                         cf[0] * vc.ab[o] + cf[1] * vc.ab[o ^ 1] + cf[2] * vc.ab[o ^ 2] + cf[3] * vc.ab[o ^ 3]);
             }
-        } else if (sg.kind == XS_D2AA) {
-            if (R.L.q2)
-                add(V.s[R.soff[sg.sub ? SF_Q2BB : SF_Q2AA][sg.h] + i],
-                    self_row_aa(R, sg.sub, sg.h, i, u), self_row_aa(R, sg.sub, sg.h, i, v));
-        } else {
-            add(V.s[R.soff[sg.sub ? SF_Q1B : SF_Q1A][sg.h] + i], u[sg.start + i], v[sg.start + i]);
+            if (!rec) {
+                if (q2) {
+#pragma unroll
+                    for (int o = 0; o < 4; o++) self(ld(s + R.soff[SF_Q2AB] + o * cc, off), uc.ab[o], vc.ab[o]);
+                    self(ld(V.s + R.soff[SF_Q2AA] + k0, off), uc.aa, vc.aa);
+                    self(ld(V.s + R.soff[SF_Q2BB] + k0, off), uc.bb, vc.bb);
+                }
+                if (g2) {
+#pragma unroll
+                    for (int o = 0; o < 4; o++) {
+                        const double *so = s + o * cc;
+                        const double x = uc.ab[o], z = vc.ab[o], sg2 = o == 1 || o == 2 ? 1.0 : -1.0;
+                        self(ld(so + R.soff[SF_G2AB], off), -x, -z);
+                        self(ld(so + R.soff[SF_G2BA], off), -x, -z);
+                        self(ld(so + R.soff[SF_G2A], off), sg2 * uc.aa, sg2 * vc.aa);
+                        self(ld(so + R.soff[SF_G2B], off), sg2 * uc.bb, sg2 * vc.bb);
+                    }
+                }
+            }
+        } else if (sg.kind == RK_SHARED) {
+            // the other rows of a cell whose pairs share an orbital, one orientation a thread
+            const int64_t nc = sg.dim;
+            const int o = (int)(i / nc);
+            const CellRec a = pl.pr->cell[i - o * nc];
+            const int64_t ga = R.L.gems_aa[a.flags >> 8], e = a.pos + o * ga * ga, k = a.k;
+            const double f = o == 1 || o == 2 ? 1.0 : -1.0;
+            const SharedAt su(R, a, o, u, mu), sv(R, a, o, v, nu);
+            const double x = u[e], z = v[e], xa = u[R.nAB + k], za = v[R.nAB + k], xb = u[R.nAB + R.nAA + k],
+                         zb = v[R.nAB + R.nAA + k];
+            if (q2) {
+                self(V.s[R.soff[SF_Q2AB] + e], x + su.q2, z + sv.q2);
+                if (o < 2)
+                    self(V.s[R.soff[SF_Q2AA + o] + k], (o ? xb : xa) + shared_q2(R, a, o, u),
+                         (o ? zb : za) + shared_q2(R, a, o, v));
+            }
+            if (g2) {
+                self(V.s[R.soff[SF_G2AB] + e], su.g1 - x, sv.g1 - z);
+                self(V.s[R.soff[SF_G2BA] + e], su.g2 - x, sv.g2 - z);
+                self(V.s[R.soff[SF_G2A] + e], fma(f, xa, su.g1), fma(f, za, sv.g1));
+                self(V.s[R.soff[SF_G2B] + e], fma(f, xb, su.gb), fma(f, zb, sv.gb));
+            }
+        } else if (sg.kind == RK_LIST_AB) {
+            const AbRec a = pl.pr->ab[i];
+            const AbVals su(R, a, u), sv(R, a, v);
+            auto one = [&](int f, double ru, double pv) { self(V.s[R.soff[f] + a.pos], ru, pv); };
+            if (q2) one(SF_Q2AB, su.q2(), sv.q2());
+            if (g2) {
+                one(SF_G2AB, su.g1(), sv.g1());
+                one(SF_G2BA, su.g2() - (mu[a.m0] + mu[a.m1]), sv.g2() - (nu[a.m0] + nu[a.m1]));
+                one(SF_G2X, su.x0, sv.x0);
+                one(SF_G2Y, su.x0, sv.x0);
+                one(SF_G2A, su.ga(a), sv.ga(a));
+                one(SF_G2B, su.gb(a), sv.gb(a));
+            }
+            for (int b = 0; b < nd; b++) one(SF_D0 + b, su.d200(R, a, b), sv.d200(R, a, b));
+        } else {   // the D1 + Q1 rows
+            self(V.s[q1_slot(R, sg, i)], u[sg.start + i], v[sg.start + i]);
         }
     });
     block_sums<3>(n, sh);
@@ -613,8 +799,8 @@ k_red_y(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B
     const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
     const Ptr w{V.w}, om{V.om};
-    for_tiles(pl, 2, [&](const Segment &sg, int64_t i, int) {
-        self_slots(R, Lo, sg, i, w, om, [&](int64_t slot, int64_t row, double o) {
+    for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
+        self_slots(R, Lo, sg, i, lane, w, om, [&](int64_t slot, int64_t row, double o) {
             y[row] += fma(e, V.s[slot], o);
         });
     });
@@ -642,37 +828,43 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
         RedProb &p = prob[q];
         if (!make_red_layout(*L[q], dev[q], p.R, work[q])) return false;
         p.full = d_dev + q;
+        full_ = full_ && p.R.L.q2 && p.R.L.g2 && p.R.cells;
         p.oD = nD_;
         p.oR = nR_;
         p.oS = nS_;
         p.oM = nM_;
-        nD_ += p.R.nD;
-        nR_ += p.R.nR;
+        nD_ += p.R.nD + 1;
+        nR_ += p.R.nR + 1;
         nS_ += p.R.nS;
-        nM_ += p.R.nM;
+        nM_ += p.R.nM + 1;
     }
-    // segments and tile prefixes of every problem's three lists, in one array each
-    std::vector<Segment> segs;
-    std::vector<int64_t> t0;
-    std::vector<size_t> so(3 * np_), to(3 * np_);
+    // the tiles of every problem's three lists, in one array, and the listed entries
+    std::vector<RedTile> tl;
+    std::vector<AbRec> ab;
+    std::vector<CellRec> cell;
+    std::vector<uint64_t> bits;
+    std::vector<uint32_t> rank;
+    std::vector<size_t> to(4 * np_), ao(np_), co(np_), bo(np_);
     for (int q = 0; q < np_; q++) {
         tiles[q] = 1;
-        for (int k = 0; k < 3; k++) {
-            const auto &v = k == 0 ? work[q].p : k == 1 ? work[q].r : work[q].n;
-            so[3 * q + k] = segs.size();
-            to[3 * q + k] = t0.size();
-            prob[q].nseg[k] = (int)v.size();
-            int64_t t = 0;
+        for (int k = 0; k < 4; k++) {
+            const auto &v = k == 0 ? work[q].start : k == 1 ? work[q].dir : k == 2 ? work[q].res : work[q].norm;
+            to[4 * q + k] = tl.size();
             for (const Segment &s : v) {
-                t0.push_back(t);
                 const int64_t per = s.wave == 0 ? kNT : s.wave == 1 ? kWaves : 1;
-                t += (s.count + per - 1) / per;
-                segs.push_back(s);
+                for (int64_t i = 0; i < s.count; i += per) tl.push_back({s, i});
             }
-            t0.push_back(t);
-            tiles[q] = std::max(tiles[q], t);
+            prob[q].ntile[k] = (int)(tl.size() - to[4 * q + k]);
+            tiles[q] = std::max<int64_t>(tiles[q], prob[q].ntile[k]);
         }
         total += tiles[q];
+        ao[q] = ab.size();
+        co[q] = cell.size();
+        bo[q] = bits.size();
+        bits.insert(bits.end(), work[q].bits.begin(), work[q].bits.end());
+        rank.insert(rank.end(), work[q].rank.begin(), work[q].rank.end());
+        ab.insert(ab.end(), work[q].ab.begin(), work[q].ab.end());
+        cell.insert(cell.end(), work[q].cell.begin(), work[q].cell.end());
     }
     // workgroups in proportion to the tiles, at least one a problem
     std::vector<int> blk;
@@ -684,17 +876,30 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     }
     nblk_ = (int)blk.size();
     if (nblk_ > kRedMaxBlocks) throw std::logic_error("reduced CG: more workgroups than partial sums");
-    const size_t sb = sizeof(Segment) * segs.size(), tb = sizeof(int64_t) * t0.size();
-    HIPCHK(hipMalloc(&d_work_, sb + tb));
-    const Segment *ds = static_cast<const Segment *>(d_work_);
-    const int64_t *dt = reinterpret_cast<const int64_t *>(static_cast<char *>(d_work_) + sb);
-    HIPCHK(hipMemcpy(d_work_, segs.data(), sb, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(static_cast<char *>(d_work_) + sb, t0.data(), tb, hipMemcpyHostToDevice));
-    for (int q = 0; q < np_; q++)
-        for (int k = 0; k < 3; k++) {
-            prob[q].seg[k] = ds + so[3 * q + k];
-            prob[q].tile0[k] = dt + to[3 * q + k];
-        }
+    // one allocation, regions on 256-byte boundaries
+    auto room = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t tb = sizeof(RedTile) * tl.size(), abb = sizeof(AbRec) * ab.size(),
+                 cb = sizeof(CellRec) * cell.size(), bb = sizeof(uint64_t) * bits.size(), rb = sizeof(uint32_t) * rank.size();
+    HIPCHK(hipMalloc(&d_work_, room(tb) + room(abb) + room(cb) + room(bb) + room(rb)));
+    char *at = static_cast<char *>(d_work_);
+    auto put = [&](const void *src, size_t n) {
+        char *p = at;
+        if (n) HIPCHK(hipMemcpy(p, src, n, hipMemcpyHostToDevice));
+        at += room(n);
+        return p;
+    };
+    const RedTile *dt = reinterpret_cast<const RedTile *>(put(tl.data(), tb));
+    const AbRec *da = reinterpret_cast<const AbRec *>(put(ab.data(), abb));
+    const CellRec *dc = reinterpret_cast<const CellRec *>(put(cell.data(), cb));
+    const uint64_t *db = reinterpret_cast<const uint64_t *>(put(bits.data(), bb));
+    const uint32_t *dr = reinterpret_cast<const uint32_t *>(put(rank.data(), rb));
+    for (int q = 0; q < np_; q++) {
+        for (int k = 0; k < 4; k++) prob[q].tile[k] = dt + to[4 * q + k];
+        prob[q].ab = da + ao[q];
+        prob[q].cell = dc + co[q];
+        prob[q].bits = db + bo[q];
+        prob[q].rank = dr + bo[q];
+    }
     HIPCHK(hipMalloc(&d_blk_, sizeof(int) * blk.size()));
     HIPCHK(hipMemcpy(d_blk_, blk.data(), sizeof(int) * blk.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&d_prob_, sizeof(RedProb) * prob.size()));
@@ -709,7 +914,7 @@ int64_t up(int64_t n) { return (n + 31) / 32 * 32; }
 
 int64_t RedCG::doubles() const
 {
-    return 6 * up(nD_) + 3 * up(nR_) + up(nS_) + 5 * up(nM_) + kRedParts * kRedMaxBlocks +
+    return 7 * up(nD_) + 3 * up(nR_) + up(nS_) + 6 * up(nM_) + kRedParts * kRedMaxBlocks +
            up((int64_t)np_ * kRedScal);
 }
 
@@ -718,9 +923,9 @@ RedBufs RedCG::carve(double *s) const
     RedBufs B;
     auto take = [&](int64_t n) { double *p = s; s += up(n); return p; };
     B.s = take(nS_);
-    for (double **p : {&B.g, &B.u, &B.w, &B.v[0], &B.v[1], &B.t}) *p = take(nD_);
+    for (double **p : {&B.g, &B.t, &B.w, &B.u[0], &B.u[1], &B.v[0], &B.v[1]}) *p = take(nD_);
     for (double **p : {&B.r, &B.p[0], &B.p[1]}) *p = take(nR_);
-    for (double **p : {&B.mu, &B.nu[0], &B.nu[1], &B.om, &B.ams}) *p = take(nM_);
+    for (double **p : {&B.mu[0], &B.mu[1], &B.nu[0], &B.nu[1], &B.om, &B.ams}) *p = take(nM_);
     B.part = take(kRedParts * kRedMaxBlocks);
     B.scal = take((int64_t)np_ * kRedScal);
     return B;
@@ -738,9 +943,11 @@ void RedCG::start(const RedBufs &B, const double *rhs, const double *y, double t
 void RedCG::iterate(const RedBufs &B, double *y, int n, hipStream_t st) const
 {
     for (int k = 0; k < n; k++) {
-        hipLaunchKernelGGL(k_red_dir, dim3(nblk_), dim3(kNT), 0, st, d_prob_, d_blk_, B, k & 1);
+        hipLaunchKernelGGL(full_ ? k_red_dir<true> : k_red_dir<false>, dim3(nblk_), dim3(kNT), 0, st,
+                           d_prob_, d_blk_, B, k & 1);
         hipLaunchKernelGGL(k_red_res, dim3(nblk_), dim3(kNT), 0, st, d_prob_, d_blk_, B, y, k & 1);
-        hipLaunchKernelGGL(k_red_norm, dim3(nblk_), dim3(kNT), 0, st, d_prob_, d_blk_, B, k & 1);
+        hipLaunchKernelGGL(full_ ? k_red_norm<true> : k_red_norm<false>, dim3(nblk_), dim3(kNT), 0, st,
+                           d_prob_, d_blk_, B, k & 1);
     }
     hipLaunchKernelGGL(k_red_status, dim3(np_), dim3(kNT), 0, st, d_prob_, B);
 }

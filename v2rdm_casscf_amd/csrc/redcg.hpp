@@ -8,19 +8,32 @@
 
 namespace v2g {
 
-// segment kinds of the reduced kernels beside XSegKind / RowFam
+// segment kinds of the reduced kernels beside XS_D1 and RowFam
 enum RedKind : int {
-    RK_ROWS = 100,   // all explicit rows, elementwise (search direction)
-    RK_DVEC,         // all D2 / D1 entries, elementwise
-    RK_MVEC,         // the maximal-spin coefficients, elementwise
+    RK_AB = 100,     // the D2ab entries of an irrep's cells, in position order
+    RK_DIAG,         // the D2ab entries with p == q or r == s
+    RK_AA,           // the cells of an irrep (both like-spin blocks)
+    RK_LIST_AB,      // the D2ab entries with p == q or r == s, by their records
+    RK_CELLS,        // the cells of an irrep
+    RK_ROWS,         // explicit rows not aligned with cells, elementwise
+    RK_DVEC, RK_RVEC, RK_MVEC,   // whole vectors, elementwise
+    RK_SHARED,       // the cells with a CellRec (Segment::dim of them), one orientation an item
+    RK_STEP,         // D entries outside the cells, elementwise
+    RK_D1,           // D1 entries one by one (XS_D1 is a RowFam's number)
     RK_MS            // maximal-spin rows, one wavefront each (direction side)
 };
 
 // work lists of one problem.  Segment::wave: 0 one thread per item, 1 one
 // wavefront, 2 one workgroup; Segment::start: first entry of the compact vector;
-// Segment::aux: first row of the full vector (explicit rows)
+// Segment::aux: first row of the full vector
 struct RedWork {
-    std::vector<Segment> p, r, n;   // direction, residual and norm passes
+    // start and end of a solve, direction, residual, norms
+    std::vector<Segment> start, dir, res, norm;
+    std::vector<AbRec> ab;
+    std::vector<CellRec> cell;
+    std::vector<uint64_t> bits;             // one a cell, set for those with a CellRec; every
+                                            // irrep starts on a word (Segment::aux of RK_CELLS)
+    std::vector<uint32_t> rank;             // CellRecs before each word's first
 };
 
 // false: the layout has rows the reduced form does not cover (T1, T2,
@@ -29,24 +42,35 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
 
 #if defined(__HIPCC__)
 
+// a tile of a work list: a workgroup's share of a segment, with the segment beside
+// it (one read instead of a search)
+struct RedTile {
+    Segment sg;
+    int64_t first;      // first item of the tile
+};
+
 // one problem of the plan, in device memory.  Offsets place its share of the
 // concatenated vectors; [b0, b0 + nb) are the workgroups that work on it
 struct RedProb {
     RedLayout R;
     const DevLayout *full;              // the full layout: rows of rhs and y
     int64_t oD, oR, oS, oM;
-    const Segment *seg[3];              // direction, residual, norm pass
-    const int64_t *tile0[3];            // tile prefix of each list (nseg + 1 entries)
-    int nseg[3];
+    const RedTile *tile[4];             // RedWork's lists, cut into tiles
+    int ntile[4];
+    const AbRec *ab;
+    const CellRec *cell;
+    const uint64_t *bits;
+    const uint32_t *rank;
     int b0, nb;
 };
 
-// the vectors of a solve (concatenated over the problems)
+// the vectors of a solve (concatenated over the problems); pairs are indexed by the
+// iteration parity
 struct RedBufs {
-    double *g, *u, *w, *v[2], *t;       // nD each
-    double *r, *p[2];                   // nR each
+    double *g, *t, *w, *u[2], *v[2];    // nD + 1 each (the last one zero)
+    double *r, *p[2];                   // nR + 1 each
     double *s;                          // nS
-    double *mu, *nu[2], *om, *ams;      // nM each
+    double *mu[2], *nu[2], *om, *ams;   // nM + 1 each
     double *part;                       // kRedParts per workgroup
     double *scal;                       // kRedScal per problem
 };
@@ -89,6 +113,7 @@ private:
     int *d_blk_ = nullptr;              // problem of each workgroup
     void *d_work_ = nullptr;            // segments and tile prefixes
     int np_ = 0, nblk_ = 0;
+    bool full_ = true;
     int64_t nD_ = 0, nR_ = 0, nS_ = 0, nM_ = 0;
 };
 

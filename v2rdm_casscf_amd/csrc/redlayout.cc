@@ -5,18 +5,17 @@ namespace v2g {
 
 bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWork &w)
 {
-    if (!Lt.xsegs_t2.empty()) return false;
+    if (!Lt.xsegs_t2.empty() || Lt.dimx >= ((int64_t)1 << 30)) return false;
     R.L = dev;
     for (int b = 0; b < XB_COUNT; b++)
         for (int h = 0; h < kMaxIrrep; h++) R.L.xoff[b][h] = -1;
     for (int f = 0; f < RF_COUNT; f++)
         for (int s = 0; s < 6; s++)
             for (int h = 0; h < kMaxIrrep; h++) R.L.rowoff[f][s][h] = -1;
-    for (int f = 0; f < SF_COUNT; f++)
-        for (int h = 0; h < kMaxIrrep; h++) R.soff[f][h] = -1;
     const bool q2 = Lt.q2_plain(), g2 = Lt.g2_plain();
     R.nblk_d = Lt.opt.spin ? (Lt.singlet ? 1 : 4) : 0;
     R.nM = Lt.opt.spin && g2 ? 2 * Lt.gems_ab[0] : 0;
+    R.cells = Lt.opt.spin && Lt.singlet ? 1 : 0;
 
     auto seg = [](std::vector<Segment> &v, int kind, int sub, int h, int dim, int64_t start,
                   int64_t count, int64_t aux, int mode) {
@@ -35,19 +34,21 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
     auto sq = [](int64_t n) { return n * n; };
 
     // D2 / D1 entries
-    int64_t o = 0;
-    std::vector<Segment> ab, aa, d1;
-    for (int h = 0; h < Lt.nirrep; h++) {
-        R.L.xoff[XB_D2AB][h] = o;
-        seg(ab, XS_D2AB, 0, h, Lt.gems_ab[h], o, sq(Lt.gems_ab[h]), 0, 0);
-        o += sq(Lt.gems_ab[h]);
+    int64_t o = 0, k = 0;
+    for (int h = 0; h < kMaxIrrep; h++) {
+        const int64_t ga = h < Lt.nirrep ? Lt.gems_aa[h] : 0;
+        R.ab0[h] = o;
+        R.aa0[h] = k;
+        o += 4 * sq(ga);
+        k += sq(ga);
     }
-    for (int s = 0; s < 2; s++)
-        for (int h = 0; h < Lt.nirrep; h++) {
-            R.L.xoff[s ? XB_D2BB : XB_D2AA][h] = o;
-            seg(aa, XS_D2AA, s, h, Lt.gems_aa[h], o, sq(Lt.gems_aa[h]), 0, 0);
-            o += sq(Lt.gems_aa[h]);
-        }
+    const int64_t ndiag = (int64_t)Lt.amo * Lt.gems_ab[0];
+    R.dA = o;
+    R.dB = o + ndiag;
+    R.nAB = o + 2 * ndiag;
+    R.nAA = k;
+    o = R.nAB + 2 * R.nAA;
+    std::vector<Segment> d1;
     for (int s = 0; s < 2; s++)
         for (int h = 0; h < Lt.nirrep; h++) {
             const int64_t n = Lt.opt.amopi[h];
@@ -56,6 +57,7 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
             o += sq(n);
         }
     R.nD = o;
+    const int64_t nd1 = R.nD1 = (R.nD - R.nAB - 2 * R.nAA) / 2;
 
     // self slots
     o = 0;
@@ -64,23 +66,19 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
         if (f == SF_Q2AB || f == SF_Q2AA || f == SF_Q2BB) on = q2;
         else if (f >= SF_G2AB && f <= SF_G2B) on = g2;
         else if (f >= SF_D0 && f <= SF_D3) on = f - SF_D0 < R.nblk_d;
-        if (!on) continue;
-        for (int h = 0; h < Lt.nirrep; h++) {
-            R.soff[f][h] = o;
-            o += f < kSfAb ? sq(Lt.gems_ab[h])
-                           : f <= SF_Q2BB ? sq(Lt.gems_aa[h]) : sq(Lt.opt.amopi[h]);
-        }
+        R.soff[f] = on ? o : -1;
+        if (on) o += f < kSfAb ? R.nAB : f <= SF_Q2BB ? R.nAA : nd1;
     }
     R.nS = o;
 
-    // explicit rows, in the order of the full layout; the long rows lead the
-    // residual pass (a workgroup for a trace, a wavefront for a contraction)
-    o = 0;
+    // explicit rows: those aligned with cells, then the others in the order of the
+    // full layout; a workgroup for a trace, a wavefront for a contraction
+    o = R.cells ? 3 * R.nAA : 0;
+    const int64_t rest0 = o;
     std::vector<Segment> lng, rest;
     for (const Segment &s : Lt.rowsegs) {
         switch (s.kind) {
-        case RF_TRACE: case RF_S2: case RF_CONTR: case RF_SPIN_D1: case RF_SPIN_D2:
-        case RF_SPIN_ANTI: case RF_MAXSPIN: break;
+        case RF_TRACE: case RF_S2: case RF_CONTR: case RF_SPIN_D1: case RF_MAXSPIN: break;
         default: continue;
         }
         R.L.rowoff[s.kind][s.sub][s.h] = o;
@@ -90,27 +88,88 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
         o += s.count;
     }
     R.nR = o;
+    // contraction rows are looked up by their D1 entry's place: the first irrep's offset
+    // is their base also when it has no orbitals
+    for (int sub = 0; sub < 6; sub++)
+        for (int h = 1; h < Lt.nirrep; h++)
+            if (R.L.rowoff[RF_CONTR][sub][0] < 0 && R.L.rowoff[RF_CONTR][sub][h] >= 0)
+                R.L.rowoff[RF_CONTR][sub][0] =
+                    R.L.rowoff[RF_CONTR][sub][h] - (R.L.xoff[XB_D1A][h] - R.L.xoff[XB_D1A][0]);
 
-    // passes
-    auto cat = [](std::vector<Segment> &a, const std::vector<Segment> &b) { a.insert(a.end(), b.begin(), b.end()); };
-    cat(w.p, d1);
-    if (R.nM)
-        for (int k = 0; k < 2; k++)
-            seg(w.p, RK_MS, k, 0, Lt.gems_ab[0], R.L.rowoff[RF_MAXSPIN][k][0], Lt.gems_ab[0], 0, 1);
-    cat(w.p, ab);
-    cat(w.p, aa);
-    seg(w.p, RK_ROWS, 0, 0, 0, 0, R.nR, 0, 0);
-    seg(w.p, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
-    cat(w.r, lng);
-    cat(w.r, rest);
-    seg(w.r, RK_DVEC, 0, 0, 0, 0, R.nD, 0, 0);
-    seg(w.r, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
-    cat(w.n, ab);
-    cat(w.n, aa);
-    for (Segment s : d1) {
-        s.wave = 0;
-        w.n.push_back(s);
+    // the listed cells (pairs that share an orbital) and the D2ab entries outside cells
+    auto first = [](int pr) { return pr & 0xffff; };
+    auto second = [](int pr) { return pr >> 16; };
+    std::vector<Segment> bulk;
+    RedLayout H = R;   // with the tables of this side
+    H.L.sym = Lt.sym.data();
+    H.L.gab = Lt.gab.data();
+    H.L.gaa = Lt.gaa.data();
+    for (int h = 0; h < Lt.nirrep; h++) {
+        const int *b = Lt.baa.data() + Lt.baa_off[h];
+        const size_t word = w.bits.size();
+        seg(bulk, RK_CELLS, 0, h, Lt.gems_aa[h], 0, sq(Lt.gems_aa[h]), (int64_t)word, 0);
+        w.bits.resize(word + (size_t)((sq(Lt.gems_aa[h]) + 63) / 64), 0);
+        for (int I = 0; I < Lt.gems_aa[h]; I++)
+            for (int K = 0; K < Lt.gems_aa[h]; K++) {
+                const int p = first(b[I]), q = second(b[I]), r = first(b[K]), s = second(b[K]);
+                if (p != r && p != s && q != r && q != s) continue;
+                const int64_t c = (int64_t)I * Lt.gems_aa[h] + K;
+                w.bits[word + c / 64] |= (uint64_t)1 << (c % 64);
+                w.cell.push_back(rows::make_cell_rec(H, p, q, r, s));
+            }
     }
+    const int *b0 = Lt.bab.data() + Lt.bab_off[0];
+    for (int d = 0; d < Lt.amo; d++)
+        for (int n = 0; n < Lt.gems_ab[0]; n++) {
+            const int p = first(b0[n]), q = second(b0[n]);
+            w.ab.push_back(rows::make_ab_rec(H, d, d, p, q));
+            if (p != q) w.ab.push_back(rows::make_ab_rec(H, p, q, d, d));
+        }
+    const int64_t nout = (int64_t)w.ab.size();
+    // listed cells before each word's first
+    w.rank.resize(w.bits.size());
+    for (size_t i = 0, n = 0; i < w.bits.size(); i++) {
+        w.rank[i] = (uint32_t)n;
+        n += (size_t)__builtin_popcountll(w.bits[i]);
+    }
+
+    // passes: the long rows first, so that no workgroup is left with one at the end
+    auto cat = [](std::vector<Segment> &a, const std::vector<Segment> &b) { a.insert(a.end(), b.begin(), b.end()); };
+    std::vector<Segment> ms;
+    if (R.nM)
+        for (int m = 0; m < 2; m++)
+            seg(ms, RK_MS, m, 0, Lt.gems_ab[0], R.L.rowoff[RF_MAXSPIN][m][0], Lt.gems_ab[0],
+                dev.rowoff[RF_MAXSPIN][m][0], 1);
+    cat(w.start, d1);
+    cat(w.start, ms);
+    for (int h = 0; h < Lt.nirrep; h++)
+        seg(w.start, RK_AB, 0, h, Lt.gems_aa[h], R.ab0[h], 4 * sq(Lt.gems_aa[h]), 0, 0);
+    seg(w.start, RK_DIAG, 0, 0, 0, R.dA, 2 * ndiag, 0, 0);
+    for (int h = 0; h < Lt.nirrep; h++)
+        seg(w.start, RK_AA, 0, h, Lt.gems_aa[h], R.aa0[h], sq(Lt.gems_aa[h]), 0, 0);
+    seg(w.start, RK_DVEC, 0, 0, 0, 0, R.nD, 0, 0);
+    seg(w.start, RK_RVEC, 0, 0, 0, 0, R.nR, 0, 0);
+    seg(w.start, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
+    cat(w.dir, d1);
+    cat(w.dir, ms);
+    seg(w.dir, RK_LIST_AB, 0, 0, 0, 0, nout, 0, 0);
+    cat(w.dir, bulk);
+    seg(w.dir, RK_ROWS, 0, 0, 0, rest0, R.nR - rest0, 0, 0);
+    seg(w.dir, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
+    cat(w.res, lng);
+    cat(w.res, rest);
+    seg(w.res, RK_STEP, 0, 0, 0, R.dA, 2 * ndiag, 0, 0);
+    seg(w.res, RK_STEP, 0, 0, 0, R.nAB + 2 * R.nAA, 2 * nd1, 0, 0);
+    cat(w.res, bulk);
+    seg(w.res, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
+    for (Segment s : d1) {
+        s.kind = RK_D1;
+        s.wave = 0;
+        w.norm.push_back(s);
+    }
+    seg(w.norm, RK_LIST_AB, 0, 0, 0, 0, nout, 0, 0);
+    seg(w.norm, RK_SHARED, 0, 0, (int)w.cell.size(), 0, 4 * (int64_t)w.cell.size(), 0, 0);
+    cat(w.norm, bulk);
     return true;
 }
 

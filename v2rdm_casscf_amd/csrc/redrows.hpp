@@ -15,7 +15,14 @@
 //
 // The self parts of s are kept aligned with the D2 entry they read: a G2ab,
 // G2ba or G2 super-block row reads exactly one D2ab (or D2aa) entry (pq|rs), so
-// its slot is that entry's, and all index permutations of the G2 maps vanish.
+// its slot is that entry's.  The entries in turn are stored by "cell": for a pair
+// p > q and a pair r > s the four D2ab entries (pq|rs), (qp|rs), (pq|sr), (qp|sr)
+// lie at the same place of four arrays, beside the cell's D2aa and D2bb entry.
+// D200, the like-spin quadrants and the antisymmetry rows only mix what is in one
+// cell, so on a cell whose pairs share no orbital the whole operator is a few
+// multiply-adds on its own numbers: no index arithmetic and no gather.  Cells that
+// share an orbital, and the entries with p == q or r == s, also meet D1, the
+// traces, contractions, S^2 and the maximal-spin rows; they are listed.
 #pragma once
 #include "rowterms.hpp"
 
@@ -37,40 +44,117 @@ enum SelfFam : int {
 };
 
 struct RedLayout {
-    // compact view: xoff of the D2 / D1 blocks in a vector of nD entries, rowoff
-    // of the explicit rows in a vector of nR entries; other blocks and rows absent
+    // xoff of the D1 blocks in a D vector (the offsets count the entries; D, R and M
+    // vectors end with one more, a zero, for indices that stand for no entry), rowoff of the explicit rows that are not
+    // aligned with cells in an R vector; other blocks and rows absent
     DevLayout L;
-    int64_t soff[SF_COUNT][kMaxIrrep];   // slot ranges in the self vector, -1 absent
+    // positions of the D2ab entries: 4 gems_aa^2 from ab0[h] on (orientation
+    // (p < q) + 2 (r < s), then the cell), the entries (pp|rs) from dA and (pq|rr),
+    // p != q, from dB on.  A D vector is [D2ab: nAB][D2aa: nAA][D2bb: nAA][D1a][D1b]
+    int64_t ab0[kMaxIrrep], aa0[kMaxIrrep], dA, dB, nAB, nAA;
+    int64_t soff[SF_COUNT];              // first slot of a family, -1 absent
     int64_t nD, nR, nS;
-    int nM;          // maximal-spin rows (2 gems_ab[0], or 0); their rowoff is compact too
+    // cell-aligned explicit rows (singlets with spin rows): D2aa - D2bb, then the two
+    // antisymmetry rows; nAA each from 0, or cells = 0
+    int cells;
+    int64_t nD1;     // D1a entries
+    int nM;          // maximal-spin rows (2 gems_ab[0], or 0)
     int nblk_d;      // D200 quadrants: 0 (spin off), 1 (singlet), 4
 };
+
+// a D2ab entry outside the cells (p == q or r == s): where everything lies that its rows read, -1 never occurs (the
+// zero at the end of the vector stands for an absent entry)
+struct AbRec {
+    int32_t pos, p1, p2, p3;   // (pq|rs), (qp|rs), (pq|sr), (qp|sr)
+    int32_t ka;                // its D2aa entry
+    int32_t pr, rp;            // D1a entries (p,r), (r,p) when q == s
+    int32_t qs, sq;            // D1b entries (q,s), (s,q) when p == r
+    int32_t m0, m1;            // maximal-spin rows when s == p, q == r
+    int32_t flags;             // AbFlag
+};
+enum AbFlag : int { AF_NEG = 1, AF_BRA = 2, AF_KET = 4, AF_QS = 8, AF_PR = 16, AF_S2 = 32 };
+
+// a listed cell: its pairs share an orbital k, or both orbitals.  With i and j the others
+// of the two pairs, a shared orbital puts D1a(i,j) into the rows of (ik|jk), D1b(i,j) into
+// those of (ki|kj), and the maximal-spin rows into (ki|jk) and (ik|kj)
+struct CellRec {
+    int32_t pos, k;            // first D2ab entry, place among the cells
+    int32_t ij[2], ji[2];      // D1a entries (i,j), (j,i)
+    int32_t m0[2], m1[2];      // maximal-spin rows of (ki|jk), (ik|kj)
+    int32_t row;               // place within the irrep
+    int32_t flags;             // orientation of (ik|jk) in bits 0-1 and 2-3, CellFlag, irrep << 8
+};
+enum CellFlag : int { CF_TWO = 16 };
 
 namespace rows {
 
 struct AbEntry {
-    int h, IJ, KL, p, q, r, s;
-    int64_t e;       // IJ g + KL
+    int p, q, r, s;
+    int64_t pos;
 };
 
-V2G_HD inline AbEntry ab_entry(const DevLayout &L, int h, int64_t e)
+V2G_HD inline int64_t ab_pos(const RedLayout &R, int p, int q, int r, int s)
 {
-    AbEntry a;
-    a.h = h;
-    a.e = e;
-    split_index(e, L.gems_ab[h], a.IJ, a.KL);
-    const int pij = L.bab[L.bab_off[h] + a.IJ], pkl = L.bab[L.bab_off[h] + a.KL];
-    a.p = P0(pij);
-    a.q = P1(pij);
-    a.r = P0(pkl);
-    a.s = P1(pkl);
+    const DevLayout &L = R.L;
+    if (p == q) return R.dA + (int64_t)p * L.gems_ab[0] + L.gab[r * L.amo + s];
+    if (r == s) return R.dB + (int64_t)r * L.gems_ab[0] + L.gab[p * L.amo + q];
+    const int h = L.sym[p] ^ L.sym[q];
+    const int64_t ga = L.gems_aa[h];
+    return R.ab0[h] + ((p < q) + 2 * (r < s)) * ga * ga + L.gaa[p * L.amo + q] * ga + L.gaa[r * L.amo + s];
+}
+
+// cell of (pq|rs), p != q, r != s: the place of its D2aa entry among the nAA
+V2G_HD inline int64_t aa_pos(const RedLayout &R, int p, int q, int r, int s)
+{
+    const DevLayout &L = R.L;
+    const int h = L.sym[p] ^ L.sym[q];
+    return R.aa0[h] + (int64_t)L.gaa[p * L.amo + q] * L.gems_aa[h] + L.gaa[r * L.amo + s];
+}
+
+V2G_HD inline AbEntry ab_entry(const RedLayout &R, int p, int q, int r, int s)
+{
+    return {p, q, r, s, ab_pos(R, p, q, r, s)};
+}
+
+// the pairs p > q, r > s of cell c of irrep h
+V2G_HD inline AbEntry cell_entry(const RedLayout &R, int h, int64_t c)
+{
+    const DevLayout &L = R.L;
+    int I, K;
+    split_index(c, L.gems_aa[h], I, K);
+    const int b = L.baa[L.baa_off[h] + I], k = L.baa[L.baa_off[h] + K];
+    return {P0(b), P1(b), P0(k), P1(k), R.ab0[h] + c};
+}
+
+V2G_HD inline bool cell_shares(const AbEntry &a)
+{
+    return a.p == a.r || a.p == a.s || a.q == a.r || a.q == a.s;
+}
+
+// entry number i (0 .. 4 gems_aa^2) of irrep h in position order
+V2G_HD inline AbEntry cell_ab(const RedLayout &R, int h, int64_t i)
+{
+    const int64_t cc = (int64_t)R.L.gems_aa[h] * R.L.gems_aa[h];
+    const int o = (int)(i / cc);
+    AbEntry a = cell_entry(R, h, i - o * cc);
+    if (o & 1) { const int t = a.p; a.p = a.q; a.q = t; }
+    if (o & 2) { const int t = a.r; a.r = a.s; a.s = t; }
+    a.pos += o * cc;
     return a;
 }
 
-// slot of (pq|rs) within its irrep's aligned range
-V2G_HD inline int64_t ab_slot(const DevLayout &L, int p, int q, int r, int s)
+// entry number i (0 .. 2 amo gems_ab[0]) of those with p == q or r == s; false: none
+V2G_HD inline bool diag_ab(const RedLayout &R, int64_t i, AbEntry &a)
 {
-    return (int64_t)L.gab[p * L.amo + q] * L.gems_ab[L.sym[p] ^ L.sym[q]] + L.gab[r * L.amo + s];
+    const DevLayout &L = R.L;
+    const int g0 = L.gems_ab[0];
+    const int d = (int)(i / g0), pr = L.bab[L.bab_off[0] + i % g0];
+    if (d < L.amo) {
+        a = {d, d, P0(pr), P1(pr), R.dA + i};
+        return true;
+    }
+    a = {P0(pr), P1(pr), d - L.amo, d - L.amo, R.dB + (i - (int64_t)L.amo * g0)};
+    return a.p != a.q;
 }
 
 V2G_HD inline int64_t d1_col(const DevLayout &L, int w, int p, int q)
@@ -99,23 +183,22 @@ V2G_HD inline void d200_coef(int blk, bool singlet, bool pq, bool rs, double (&c
     }
 }
 
-// the D2 / D1 parts of the Q2 and G2 rows aligned with entry a; X is a vector of nD
-// entries
+// the D2 / D1 parts of the Q2 and G2 rows aligned with entry a; X is a D vector
 template <class X>
 struct SelfAb {
     double x, q2, g1, g2, ga, gb;   // x: the mixed-spin quadrants' part too
     V2G_HD inline SelfAb(const RedLayout &R, const AbEntry &a, const X &v)
     {
         const DevLayout &L = R.L;
-        x = v[L.xoff[XB_D2AB][a.h] + a.e];
+        x = v[a.pos];
         q2 = x;
         g1 = g2 = -x;
         ga = gb = 0.0;
         if (L.g2 && a.p != a.q && a.r != a.s) {
-            const int64_t k = (int64_t)L.gaa[a.p * L.amo + a.q] * L.gems_aa[a.h] + L.gaa[a.r * L.amo + a.s];
+            const int64_t k = R.nAB + aa_pos(R, a.p, a.q, a.r, a.s);
             const double sg = ((a.p < a.q) == (a.r < a.s)) ? -1.0 : 1.0;
-            ga = sg * v[L.xoff[XB_D2AA][a.h] + k];
-            gb = sg * v[L.xoff[XB_D2BB][a.h] + k];
+            ga = sg * v[k];
+            gb = sg * v[k + R.nAA];
         }
         if (a.q == a.s) {
             if (L.q2) q2 -= v[d1_col(L, XB_D1A, a.r, a.p)];
@@ -139,13 +222,10 @@ struct D200Ab {
     double v0, v1, v2, v3;          // x at (pq|rs), (qp|rs), (pq|sr), (qp|sr)
     V2G_HD inline D200Ab(const RedLayout &R, const AbEntry &a, const X &v)
     {
-        const DevLayout &L = R.L;
-        const int64_t b = L.xoff[XB_D2AB][a.h], g = L.gems_ab[a.h];
-        const int64_t qp = L.gab[a.q * L.amo + a.p], sr = L.gab[a.s * L.amo + a.r];
-        v0 = v[b + a.e];
-        v1 = v[b + qp * g + a.KL];
-        v2 = v[b + a.IJ * g + sr];
-        v3 = v[b + qp * g + sr];
+        v0 = v[a.pos];
+        v1 = v[ab_pos(R, a.q, a.p, a.r, a.s)];
+        v2 = v[ab_pos(R, a.p, a.q, a.s, a.r)];
+        v3 = v[ab_pos(R, a.q, a.p, a.s, a.r)];
     }
     V2G_HD inline double row(const RedLayout &R, const AbEntry &a, int blk) const
     {
@@ -155,16 +235,13 @@ struct D200Ab {
     }
 };
 
-// the D2 / D1 part of a Q2aa / Q2bb row (spin sp) at entry e of irrep h
+// the D2 / D1 part of the Q2aa / Q2bb row (spin sp) of the cell a
 template <class X>
-V2G_HD inline double self_row_aa(const RedLayout &R, int sp, int h, int64_t e, const X &x)
+V2G_HD inline double self_row_aa(const RedLayout &R, int sp, const AbEntry &a, const X &x)
 {
     const DevLayout &L = R.L;
-    int IJ, KL;
-    split_index(e, L.gems_aa[h], IJ, KL);
-    const int pij = L.baa[L.baa_off[h] + IJ], pkl = L.baa[L.baa_off[h] + KL];
-    const int i = P0(pij), j = P1(pij), k = P0(pkl), l = P1(pkl), wd = sp ? XB_D1B : XB_D1A;
-    double v = x[L.xoff[sp ? XB_D2BB : XB_D2AA][h] + e];
+    const int i = a.p, j = a.q, k = a.r, l = a.s, wd = sp ? XB_D1B : XB_D1A;
+    double v = x[R.nAB + sp * R.nAA + aa_pos(R, i, j, k, l)];
     if (j == l) v -= x[d1_col(L, wd, k, i)];
     if (j == k) v += x[d1_col(L, wd, l, i)];
     if (i == l) v += x[d1_col(L, wd, k, j)];
@@ -172,8 +249,8 @@ V2G_HD inline double self_row_aa(const RedLayout &R, int sp, int h, int64_t e, c
     return v;
 }
 
-// (P m)(e): the maximal-spin generator on the G2ba row of the aligned entry a
-// (non-zero on irrep 0 only: s == p or q == r imply it)
+// (P m)(e): the maximal-spin generator on the G2ba row aligned with (pq|rs)
+// (s == p or q == r imply that the row lies in irrep 0)
 template <class M>
 V2G_HD inline double ms_part(const RedLayout &R, int p, int q, int r, int s, const M &m)
 {
@@ -186,95 +263,33 @@ V2G_HD inline double ms_part(const RedLayout &R, int p, int q, int r, int s, con
     return v;
 }
 
-// (B2^T B2 x)(e) + (the G2ba rows' share of -B2^T P m, whose sign is +): a D2ab entry
-template <class X, class M>
-V2G_HD inline double gram_ab(const RedLayout &R, const AbEntry &a, const X &x, const M &m)
-{
-    const DevLayout &L = R.L;
-    const double v = x[L.xoff[XB_D2AB][a.h] + a.e];
-    double t = (L.q2 ? v : 0.0) + (L.g2 ? 4.0 * v : 0.0);
-    if (a.q == a.s) {
-        if (L.q2) t -= x[d1_col(L, XB_D1A, a.r, a.p)];
-        if (L.g2) t -= x[d1_col(L, XB_D1A, a.p, a.r)];
-    }
-    if (a.p == a.r) {
-        if (L.q2) t -= x[d1_col(L, XB_D1B, a.s, a.q)];
-        if (L.g2) t -= x[d1_col(L, XB_D1B, a.q, a.s)];
-    }
-    if (L.g2) t += ms_part(R, a.p, a.q, a.r, a.s, m);
-    if (R.nblk_d) {
-        const D200Ab<X> w(R, a, x);
-        // sum over a row's four source entries of (coefficient x row value)
-        const double ip = a.p == a.q ? 0.5 : 1.0, ir = a.r == a.s ? 0.5 : 1.0;
-        t += (ip * ir) * ((w.v0 + w.v1) + (w.v2 + w.v3));
-        if (!L.singlet) {
-            t += ip * ((w.v0 + w.v1) - (w.v2 + w.v3));
-            t += ir * ((w.v0 + w.v2) - (w.v1 + w.v3));
-            t += (w.v0 + w.v3) - (w.v1 + w.v2);
-        }
-    }
-    return t;
-}
-
-// the same for a D2aa / D2bb entry (spin sp)
-template <class X>
-V2G_HD inline double gram_aa(const RedLayout &R, int sp, int h, int64_t e, const X &x)
-{
-    const DevLayout &L = R.L;
-    double t = L.q2 ? self_row_aa(R, sp, h, e, x) : 0.0;
-    if (L.g2) {
-        int IJ, KL;
-        split_index(e, L.gems_aa[h], IJ, KL);
-        const int pij = L.baa[L.baa_off[h] + IJ], pkl = L.baa[L.baa_off[h] + KL];
-        const int wd = sp ? XB_D1B : XB_D1A;
-        t += 4.0 * x[L.xoff[sp ? XB_D2BB : XB_D2AA][h] + e];
-        // rows ((i,j),(k,l)) of the like-spin quadrant, {i,l} = pair 1, {k,j} = pair 2
-        for (int a = 0; a < 2; a++)
-            for (int b = 0; b < 2; b++) {
-                const int i = a ? P1(pij) : P0(pij), l = a ? P0(pij) : P1(pij);
-                const int k = b ? P1(pkl) : P0(pkl), j = b ? P0(pkl) : P1(pkl);
-                if (j != l) continue;
-                const double sg = ((i < l) == (k < j)) ? 1.0 : -1.0;
-                t -= sg * x[d1_col(L, wd, i, k)];
-            }
-    }
-    return t;
-}
-
-// the same for a D1 entry: lane-strided share of one wavefront
+// B2^T (B2 x - P m) on a D1 entry: lane-strided share of one wavefront
 template <class X, class M>
 V2G_HD inline double gram_d1(const RedLayout &R, int sp, int h, int64_t item, int lane, const X &x,
                              const M &m)
 {
     const DevLayout &L = R.L;
-    const int amo = L.amo, n = L.amopi[h];
+    const int n = L.amopi[h];
     const int A = (int)(item / n) + L.poff[h], B = (int)(item % n) + L.poff[h];
     const int wd = sp ? XB_D1B : XB_D1A, wo = sp ? XB_D1A : XB_D1B;
+    // D1(A,B) itself: the D1 + Q1 row, then one Q2ab and two G2 rows for every t and a
+    // like-spin Q2 row for every t that differs from A and B
     const double xd = x[L.xoff[wd][h] + item];
-    double v = lane == 0 ? xd : 0.0;   // D1 + Q1 row
-    for (int t = lane; t < amo; t += 64) {
-        const int ht = L.sym[B] ^ L.sym[t];
-        const int64_t bt = sp ? L.gab[t * amo + B] : L.gab[B * amo + t];
-        const int64_t at = sp ? L.gab[t * amo + A] : L.gab[A * amo + t];
-        const int64_t g = L.gems_ab[ht], bab = L.xoff[XB_D2AB][ht];
+    const int others = L.amo - (A == B ? 1 : 2);
+    double v = lane == 0 ? xd * (1.0 + (L.q2 ? L.amo + others : 0) + (L.g2 ? 2.0 * L.amo : 0.0)) : 0.0;
+    for (int t = lane; t < L.amo; t += 64) {
+        const bool in = t != A && t != B;
+        const double sg = ((A < t) == (B < t)) ? 1.0 : -1.0;
+        const int64_t k = in ? R.nAB + sp * R.nAA : 0;
         if (L.q2) {
-            v -= x[bab + bt * g + at] - xd;
-            if (A == B) v += x[d1_col(L, wo, t, t)];
-            if (t != A && t != B) {
-                const double sg = ((B > t) == (A > t)) ? 1.0 : -1.0;
-                v -= sg * self_row_aa(R, sp, ht,
-                                      (int64_t)L.gaa[B * amo + t] * L.gems_aa[ht] + L.gaa[A * amo + t], x);
-            }
+            v -= x[sp ? ab_pos(R, t, B, t, A) : ab_pos(R, B, t, A, t)];
+            if (in) v -= sg * x[k + aa_pos(R, B, t, A, t)];
+            if (A == B) v += x[d1_col(L, wo, t, t)] + (in ? x[d1_col(L, wd, t, t)] : 0.0);
         }
         if (L.g2) {
-            v += xd - x[bab + at * g + bt];     // G2ab (alpha) / G2ba (beta)
+            v -= x[sp ? ab_pos(R, t, A, t, B) : ab_pos(R, A, t, B, t)];   // G2ab / G2ba
+            if (in) v -= sg * x[k + aa_pos(R, A, t, B, t)];              // like-spin quadrant
             if (sp) v -= ms_part(R, t, A, t, B, m);
-            v += xd;                            // like-spin quadrant
-            if (t != A && t != B) {
-                const double sg = ((A < t) == (B < t)) ? 1.0 : -1.0;
-                v -= sg * x[L.xoff[sp ? XB_D2BB : XB_D2AA][ht] +
-                            (int64_t)L.gaa[A * amo + t] * L.gems_aa[ht] + L.gaa[B * amo + t]];
-            }
         }
     }
     return v;
@@ -285,42 +300,33 @@ template <class S>
 V2G_HD inline double self_at_ab(const RedLayout &R, const AbEntry &a, const S &s)
 {
     const DevLayout &L = R.L;
-    const int64_t g = L.gems_ab[a.h];
     double t = 0.0;
-    if (L.q2) t += s[R.soff[SF_Q2AB][a.h] + a.e];
+    if (L.q2) t += s[R.soff[SF_Q2AB] + a.pos];
     if (L.g2)
-        t += (s[R.soff[SF_G2X][a.h] + a.e] + s[R.soff[SF_G2Y][a.h] + a.e]) -
-             (s[R.soff[SF_G2AB][a.h] + a.e] + s[R.soff[SF_G2BA][a.h] + a.e]);
+        t += (s[R.soff[SF_G2X] + a.pos] + s[R.soff[SF_G2Y] + a.pos]) -
+             (s[R.soff[SF_G2AB] + a.pos] + s[R.soff[SF_G2BA] + a.pos]);
     if (R.nblk_d) {
-        const int64_t qp = L.gab[a.q * L.amo + a.p], sr = L.gab[a.s * L.amo + a.r];
+        const int64_t p1 = ab_pos(R, a.q, a.p, a.r, a.s), p2 = ab_pos(R, a.p, a.q, a.s, a.r),
+                      p3 = ab_pos(R, a.q, a.p, a.s, a.r);
         for (int k = 0; k < R.nblk_d; k++) {
             double c[4];
             d200_coef(k, L.singlet, a.p == a.q, a.r == a.s, c);
-            const int64_t b = R.soff[SF_D0 + k][a.h];
-            t += c[0] * s[b + a.e] + c[1] * s[b + qp * g + a.KL] + c[2] * s[b + a.IJ * g + sr] +
-                 c[3] * s[b + qp * g + sr];
+            const int64_t b = R.soff[SF_D0 + k];
+            t += c[0] * s[b + a.pos] + c[1] * s[b + p1] + c[2] * s[b + p2] + c[3] * s[b + p3];
         }
     }
     return t;
 }
 
 template <class S>
-V2G_HD inline double self_at_aa(const RedLayout &R, int sp, int h, int64_t e, const S &s)
+V2G_HD inline double self_at_aa(const RedLayout &R, int sp, int h, const AbEntry &a, const S &s)
 {
     const DevLayout &L = R.L;
-    double t = L.q2 ? s[R.soff[sp ? SF_Q2BB : SF_Q2AA][h] + e] : 0.0;
+    double t = L.q2 ? s[R.soff[sp ? SF_Q2BB : SF_Q2AA] + aa_pos(R, a.p, a.q, a.r, a.s)] : 0.0;
     if (L.g2) {
-        int IJ, KL;
-        split_index(e, L.gems_aa[h], IJ, KL);
-        const int pij = L.baa[L.baa_off[h] + IJ], pkl = L.baa[L.baa_off[h] + KL];
-        const int64_t b0 = R.soff[sp ? SF_G2B : SF_G2A][h], g = L.gems_ab[h];
-        for (int a = 0; a < 2; a++)
-            for (int b = 0; b < 2; b++) {
-                const int i = a ? P1(pij) : P0(pij), l = a ? P0(pij) : P1(pij);
-                const int k = b ? P1(pkl) : P0(pkl), j = b ? P0(pkl) : P1(pkl);
-                const double sg = ((i < l) == (k < j)) ? 1.0 : -1.0;
-                t -= sg * s[b0 + (int64_t)L.gab[i * L.amo + l] * g + L.gab[k * L.amo + j]];
-            }
+        const int64_t cc = (int64_t)L.gems_aa[h] * L.gems_aa[h];
+        const int64_t b = R.soff[sp ? SF_G2B : SF_G2A] + a.pos;
+        t += (s[b + cc] + s[b + 2 * cc]) - (s[b] + s[b + 3 * cc]);
     }
     return t;
 }
@@ -329,47 +335,24 @@ template <class S>
 V2G_HD inline double self_at_d1(const RedLayout &R, int sp, int h, int64_t item, int lane, const S &s)
 {
     const DevLayout &L = R.L;
-    const int amo = L.amo, n = L.amopi[h];
+    const int n = L.amopi[h];
     const int A = (int)(item / n) + L.poff[h], B = (int)(item % n) + L.poff[h];
-    double v = lane == 0 ? s[R.soff[sp ? SF_Q1B : SF_Q1A][h] + item] : 0.0;
-    for (int t = lane; t < amo; t += 64) {
-        const int ht = L.sym[B] ^ L.sym[t];
-        const int64_t g = L.gems_ab[ht];
-        const int64_t bt = sp ? L.gab[t * amo + B] : L.gab[B * amo + t];
-        const int64_t at = sp ? L.gab[t * amo + A] : L.gab[A * amo + t];
+    double v = lane == 0 ? s[R.soff[sp ? SF_Q1B : SF_Q1A] + (L.xoff[sp ? XB_D1B : XB_D1A][h] -
+                                                             L.xoff[sp ? XB_D1B : XB_D1A][0]) + item]
+                         : 0.0;
+    for (int t = lane; t < L.amo; t += 64) {
         if (L.q2) {
-            v -= s[R.soff[SF_Q2AB][ht] + bt * g + at];
+            v -= s[R.soff[SF_Q2AB] + (sp ? ab_pos(R, t, B, t, A) : ab_pos(R, B, t, A, t))];
             if (t != A && t != B) {
                 const double sg = ((B > t) == (A > t)) ? 1.0 : -1.0;
-                v -= sg * s[R.soff[sp ? SF_Q2BB : SF_Q2AA][ht] +
-                            (int64_t)L.gaa[B * amo + t] * L.gems_aa[ht] + L.gaa[A * amo + t]];
+                v -= sg * s[R.soff[sp ? SF_Q2BB : SF_Q2AA] + aa_pos(R, B, t, A, t)];
             }
         }
         if (L.g2) {
-            v += s[R.soff[sp ? SF_G2BA : SF_G2AB][ht] + at * g + bt];
+            v += s[R.soff[sp ? SF_G2BA : SF_G2AB] + (sp ? ab_pos(R, t, A, t, B) : ab_pos(R, A, t, B, t))];
             // the like-spin quadrant's row ((A,t),(B,t)) reads (At|Bt)
-            v += s[R.soff[sp ? SF_G2B : SF_G2A][ht] + (int64_t)L.gab[A * amo + t] * g + L.gab[B * amo + t]];
+            v += s[R.soff[sp ? SF_G2B : SF_G2A] + ab_pos(R, A, t, B, t)];
         }
-    }
-    return v;
-}
-
-// maximal-spin row `item` of orientation o (0: G2ba entries (kl, ii), 1: (ii, kl)):
-// lane-strided share of sum_i p_self over its G2ba rows, p_self = d s + B2 x - P m
-template <class S, class X, class M>
-V2G_HD inline double ms_row_self(const RedLayout &R, int o, int item, int lane, double d, const S &s,
-                                 const X &x, const M &m)
-{
-    const DevLayout &L = R.L;
-    const int pr = L.bab[L.bab_off[0] + item], k = P0(pr), l = P1(pr);
-    double v = 0.0;
-    for (int i = lane; i < L.amo; i += 64) {
-        // the row's pairs are (q, r) and (s, p)
-        const int q = o ? i : k, r = o ? i : l, ss = o ? k : i, p = o ? l : i;
-        const int hh = L.sym[p] ^ L.sym[q];
-        const int64_t e = ab_slot(L, p, q, r, ss);
-        v += d * s[R.soff[SF_G2BA][hh] + e] - x[L.xoff[XB_D2AB][hh] + e] - ms_part(R, p, q, r, ss, m);
-        if (p == r) v += x[d1_col(L, XB_D1B, q, ss)];
     }
     return v;
 }
@@ -387,7 +370,70 @@ V2G_HD inline double ms_row_gram(const RedLayout &R, int o, int item, int lane, 
     return v;
 }
 
-// the row of the full layout Lo that the slot of family f at an aligned entry stands for
+// maximal-spin row `item` of orientation o (0: G2ba entries (kl, ii), 1: (ii, kl)):
+// lane-strided share of sum_i p_self over its G2ba rows, p_self = d s + B2 x - P m
+template <class S, class X, class M>
+V2G_HD inline double ms_row_self(const RedLayout &R, int o, int item, int lane, double d, const S &s,
+                                 const X &x, const M &m)
+{
+    const DevLayout &L = R.L;
+    const int pr = L.bab[L.bab_off[0] + item], k = P0(pr), l = P1(pr);
+    // the D1b part: its only row with p == r; the P m parts sum to P^T P m
+    double v = lane == 0 ? (o ? x[d1_col(L, XB_D1B, l, k)] : x[d1_col(L, XB_D1B, k, l)]) : 0.0;
+    v -= ms_row_gram(R, o, item, lane, m);
+    for (int i = lane; i < L.amo; i += 64) {
+        // the row's pairs are (q, r) and (s, p)
+        const int64_t e = o ? ab_pos(R, l, i, i, k) : ab_pos(R, i, k, l, i);
+        v += d * s[R.soff[SF_G2BA] + e] - x[e];
+    }
+    return v;
+}
+
+// ---- explicit rows that are not aligned with cells: their value on a D vector --
+// a trace, S^2 or contraction row: lane-strided share of `lanes` threads
+template <class X>
+V2G_HD inline double long_row(const RedLayout &R, const Segment &sg, int64_t item, int lane, int lanes,
+                              const X &x)
+{
+    const DevLayout &L = R.L;
+    const int amo = L.amo;
+    double v = 0.0;
+    if (sg.kind == RF_CONTR) {
+        const int n = sg.dim, sub = sg.sub;
+        const int i = (int)(item / n) + L.poff[sg.h], j = (int)(item % n) + L.poff[sg.h];
+        const bool beta = sub == 1 || sub == 3 || sub == 5;
+        if (lane == 0) {
+            const double c = sub == 0 ? L.nb : sub == 1 ? L.na : sub == 2 ? L.na - 1.0
+                           : sub == 3 ? L.nb - 1.0 : L.na + L.nb - 1.0;
+            v += c * x[d1_col(L, beta ? XB_D1B : XB_D1A, i, j)];
+        }
+        for (int k = lane; k < amo; k += lanes) {
+            if (sub < 2 || sub >= 4) v -= x[beta ? ab_pos(R, k, i, k, j) : ab_pos(R, i, k, j, k)];
+            if (sub >= 2 && i != k && j != k) {
+                const double s2 = ((i < k) == (j < k)) ? 1.0 : -1.0;
+                v -= s2 * x[R.nAB + (beta ? R.nAA : 0) + aa_pos(R, i, k, j, k)];
+            }
+        }
+        return v;
+    }
+    for (int pq = lane; pq < amo * amo; pq += lanes) {
+        const int i = pq / amo, j = pq % amo;
+        if (sg.kind == RF_S2) {
+            v += x[ab_pos(R, i, j, j, i)];
+            continue;
+        }
+        if (sg.sub == 0 || sg.sub == 3) v += (sg.sub ? 2.0 : 1.0) * x[ab_pos(R, i, j, i, j)];
+        if (sg.sub > 0 && i != j) {
+            const int64_t k = R.nAB + aa_pos(R, i, j, i, j);
+            if (sg.sub != 2) v += x[k];
+            if (sg.sub != 1) v += x[k + R.nAA];
+        }
+    }
+    return v;
+}
+
+// ---- rows of the full layout -------------------------------------------------
+// the row of the full layout Lo that family f's slot of an aligned entry stands for
 V2G_HD inline int64_t self_row_ab(const DevLayout &Lo, int f, const AbEntry &a)
 {
     const int amo = Lo.amo;
@@ -395,7 +441,10 @@ V2G_HD inline int64_t self_row_ab(const DevLayout &Lo, int f, const AbEntry &a)
     const int p = a.p, q = a.q, r = a.r, s = a.s;
     auto GAB = [&](int x, int y) -> int64_t { return gab[x * amo + y]; };
     switch (f) {
-    case SF_Q2AB: return Lo.rowoff[RF_Q2AB][0][a.h] + a.e;
+    case SF_Q2AB: {
+        const int h = sym[p] ^ sym[q];
+        return Lo.rowoff[RF_Q2AB][0][h] + GAB(p, q) * Lo.gems_ab[h] + GAB(r, s);
+    }
     case SF_G2AB: {
         const int h = sym[p] ^ sym[s];
         return Lo.rowoff[RF_G2AB][0][h] + GAB(p, s) * Lo.gems_ab[h] + GAB(r, q);
@@ -420,10 +469,10 @@ V2G_HD inline int64_t self_row_ab(const DevLayout &Lo, int f, const AbEntry &a)
         return Lo.rowoff[RF_G2AA][0][h] + (b + GAB(p, s)) * 2 * g + b + GAB(r, q);
     }
     default: {
-        if (Lo.singlet) return Lo.rowoff[RF_SPIN_D200][0][a.h] + a.e;
-        const int k = f - SF_D0;
-        const int64_t g = Lo.gems_ab[a.h];
-        return Lo.rowoff[RF_SPIN_D200_4][0][a.h] + (a.IJ + (k >> 1) * g) * 2 * g + a.KL + (k & 1) * g;
+        const int h = sym[p] ^ sym[q], k = f - SF_D0;
+        const int64_t g = Lo.gems_ab[h];
+        if (Lo.singlet) return Lo.rowoff[RF_SPIN_D200][0][h] + GAB(p, q) * g + GAB(r, s);
+        return Lo.rowoff[RF_SPIN_D200_4][0][h] + (GAB(p, q) + (k >> 1) * g) * 2 * g + GAB(r, s) + (k & 1) * g;
     }
     }
 }
@@ -433,6 +482,284 @@ V2G_HD inline int64_t self_row_d1(const DevLayout &Lo, int sp, int h, int64_t it
 {
     const int n = Lo.amopi[h];
     return Lo.rowoff[RF_D1Q1][sp][h] + (item % n) * n + item / n;
+}
+
+// A^T y on entry a of the D2ab blocks / the cell a of the D2aa, D2bb blocks, from full rows
+template <class Y>
+V2G_HD inline double full_at_ab(const DevLayout &Lo, const AbEntry &a, const Y &y)
+{
+    Segment sg{};
+    sg.h = Lo.sym[a.p] ^ Lo.sym[a.q];
+    sg.dim = Lo.gems_ab[sg.h];
+    return atu_d2ab(Lo, sg, (int64_t)Lo.gab[a.p * Lo.amo + a.q] * sg.dim + Lo.gab[a.r * Lo.amo + a.s], y);
+}
+
+template <class Y>
+V2G_HD inline double full_at_aa(const DevLayout &Lo, int sp, const AbEntry &a, const Y &y)
+{
+    Segment sg{};
+    sg.h = Lo.sym[a.p] ^ Lo.sym[a.q];
+    sg.sub = sp;
+    sg.dim = Lo.gems_aa[sg.h];
+    return atu_d2aa(Lo, sg, (int64_t)Lo.gaa[a.p * Lo.amo + a.q] * sg.dim + Lo.gaa[a.r * Lo.amo + a.s], y);
+}
+
+// ---- listed entries ------------------------------------------------------------
+V2G_HD inline AbRec make_ab_rec(const RedLayout &R, int p, int q, int r, int s)
+{
+    const DevLayout &L = R.L;
+    AbRec a;
+    a.pos = (int32_t)ab_pos(R, p, q, r, s);
+    a.p1 = (int32_t)ab_pos(R, q, p, r, s);
+    a.p2 = (int32_t)ab_pos(R, p, q, s, r);
+    a.p3 = (int32_t)ab_pos(R, q, p, s, r);
+    const bool diag = p == q || r == s;
+    a.ka = (int32_t)(diag ? R.nD : R.nAB + aa_pos(R, p, q, r, s));
+    a.pr = (int32_t)(q == s ? d1_col(L, XB_D1A, p, r) : R.nD);
+    a.rp = (int32_t)(q == s ? d1_col(L, XB_D1A, r, p) : R.nD);
+    a.qs = (int32_t)(p == r ? d1_col(L, XB_D1B, q, s) : R.nD);
+    a.sq = (int32_t)(p == r ? d1_col(L, XB_D1B, s, q) : R.nD);
+    a.m0 = R.nM && s == p ? L.gab[q * L.amo + r] : R.nM;
+    a.m1 = R.nM && q == r ? L.gems_ab[0] + L.gab[s * L.amo + p] : R.nM;
+    a.flags = ((p < q) == (r < s) ? 0 : AF_NEG) | (p == q ? AF_BRA : 0) | (r == s ? AF_KET : 0) |
+              (q == s ? AF_QS : 0) | (p == r ? AF_PR : 0) | (p == s && q == r ? AF_S2 : 0);
+    return a;
+}
+
+// p > q, r > s with a common orbital
+V2G_HD inline CellRec make_cell_rec(const RedLayout &R, int p, int q, int r, int s)
+{
+    const DevLayout &L = R.L;
+    const int h = L.sym[p] ^ L.sym[q];
+    CellRec c;
+    c.pos = (int32_t)ab_pos(R, p, q, r, s);
+    c.k = (int32_t)aa_pos(R, p, q, r, s);
+    c.row = (int32_t)(c.k - R.aa0[h]);
+    c.flags = h << 8;
+    int n = 0;
+    for (int u = 0; u < 2; u++)
+        for (int w = 0; w < 2; w++) {
+            // bra (i,l), ket (j,k) by orientation u + 2 w of the cell; l == k is shared
+            const int i = u ? q : p, l = u ? p : q, j = w ? s : r, k = w ? r : s;
+            if (k != l || n == 2) continue;
+            c.ij[n] = (int32_t)d1_col(L, XB_D1A, i, j);
+            c.ji[n] = (int32_t)d1_col(L, XB_D1A, j, i);
+            c.m0[n] = R.nM ? L.gab[i * L.amo + j] : 0;
+            c.m1[n] = R.nM ? L.gems_ab[0] + L.gab[j * L.amo + i] : 0;
+            c.flags |= (u + 2 * w) << (2 * n);
+            if (n) c.flags |= CF_TWO;
+            n++;
+        }
+    if (n == 1) {
+        c.ij[1] = c.ij[0];
+        c.ji[1] = c.ji[0];
+        c.m0[1] = c.m0[0];
+        c.m1[1] = c.m1[0];
+    }
+    return c;
+}
+
+// what a listed D2ab entry reads of a D vector
+struct AbVals {
+    double x0, x1, x2, x3, aa, bb, arp, apr, bpr, bsq, bqs;
+    template <class X>
+    V2G_HD inline AbVals(const RedLayout &R, const AbRec &a, const X &x)
+    {
+        x0 = x[a.pos];
+        x1 = x[a.p1];
+        x2 = x[a.p2];
+        x3 = x[a.p3];
+        aa = x[a.ka];
+        bb = x[a.flags & (AF_BRA | AF_KET) ? a.ka : a.ka + (int32_t)R.nAA];
+        arp = x[a.rp];
+        apr = x[a.pr];
+        bpr = x[a.flags & AF_QS ? a.pr + (int32_t)R.nD1 : a.pr];
+        bsq = x[a.sq];
+        bqs = x[a.qs];
+    }
+    V2G_HD inline double q2() const { return x0 - arp - bsq; }
+    V2G_HD inline double g1() const { return apr - x0; }
+    V2G_HD inline double g2() const { return bqs - x0; }
+    V2G_HD inline double ga(const AbRec &a) const { return a.flags & AF_NEG ? apr + aa : apr - aa; }
+    V2G_HD inline double gb(const AbRec &a) const { return a.flags & AF_NEG ? bpr + bb : bpr - bb; }
+    V2G_HD inline double d200(const RedLayout &R, const AbRec &a, int blk) const
+    {
+        double c[4];
+        d200_coef(blk, R.L.singlet, (a.flags & AF_BRA) != 0, (a.flags & AF_KET) != 0, c);
+        return c[0] * x0 + c[1] * x1 + c[2] * x2 + c[3] * x3;
+    }
+    // B2^T B2 x (gram_ab without its maximal-spin part)
+    V2G_HD inline double gram(const RedLayout &R, const AbRec &a) const
+    {
+        double t = (R.L.q2 ? x0 - arp - bsq : 0.0) + (R.L.g2 ? 4.0 * x0 - apr - bqs : 0.0);
+        if (R.nblk_d) {
+            const double ip = a.flags & AF_BRA ? 0.5 : 1.0, ir = a.flags & AF_KET ? 0.5 : 1.0;
+            t += (ip * ir) * ((x0 + x1) + (x2 + x3));
+            if (!R.L.singlet) {
+                t += ip * ((x0 + x1) - (x2 + x3));
+                t += ir * ((x0 + x2) - (x1 + x3));
+                t += (x0 + x3) - (x1 + x2);
+            }
+        }
+        return t;
+    }
+};
+
+// the explicit rows' share of A^T on a listed D2ab entry
+template <class Y>
+V2G_HD inline double rec_expl_ab(const RedLayout &R, const AbRec &a, const Y &y)
+{
+    const DevLayout &L = R.L;
+    const bool A = a.flags & AF_QS, B = a.flags & AF_PR;
+    const int64_t ca = L.rowoff[RF_CONTR][L.sz ? 0 : 4][0] + (a.pr - L.xoff[XB_D1A][0]);
+    const int64_t cb = L.rowoff[RF_CONTR][L.sz ? 1 : 5][0] + (a.qs - L.xoff[XB_D1B][0]);
+    const int64_t tr = L.rowoff[RF_TRACE][L.sz ? 0 : 3][0];
+    double v = (L.sz ? 1.0 : 2.0) * y[A && B ? tr : R.nR] - y[A ? ca : R.nR] - y[B ? cb : R.nR];
+    if (L.spin) v += y[a.flags & AF_S2 ? L.rowoff[RF_S2][0][0] : R.nR];
+    if (R.cells && !(a.flags & (AF_BRA | AF_KET))) {
+        const int64_t k = a.ka - R.nAB;
+        const double an = 0.5 * (y[R.nAA + k] + y[2 * R.nAA + k]);
+        v += a.flags & AF_NEG ? an : -an;
+    }
+    return v;
+}
+
+// ---- a cell whose pairs share no orbital --------------------------------------
+// its numbers in a D vector: the four D2ab entries by orientation, D2aa, D2bb
+struct Cell {
+    double ab[4], aa, bb;
+};
+
+template <class X>
+V2G_HD inline Cell load_cell(const RedLayout &R, int64_t pos, int64_t cc, int64_t k, const X &x)
+{
+    Cell c;
+    for (int o = 0; o < 4; o++) c.ab[o] = x[pos + o * cc];
+    c.aa = x[R.nAB + k];
+    c.bb = x[R.nAB + R.nAA + k];
+    return c;
+}
+
+// t = d g + B2^T B2 v + B1^T p on the cell (pr: its three explicit rows' p)
+V2G_HD inline Cell cell_at(bool q2, bool g2, int nd, bool cells, double d, const Cell &g, const Cell &v,
+                           const double (&pr)[3])
+{
+    const double w = (q2 ? 1.0 : 0.0) + (g2 ? 4.0 : 0.0), wd = w + (nd == 4 ? 4.0 : 0.0);
+    const double sum = nd == 1 ? (v.ab[0] + v.ab[1]) + (v.ab[2] + v.ab[3]) : 0.0;
+    const double an = cells ? 0.5 * (pr[1] + pr[2]) : 0.0;
+    Cell t;
+    for (int o = 0; o < 4; o++)
+        t.ab[o] = d * g.ab[o] + wd * v.ab[o] + sum + (o == 1 || o == 2 ? an : -an);
+    t.aa = d * g.aa + w * v.aa + (cells ? pr[0] + pr[1] : 0.0);
+    t.bb = d * g.bb + w * v.bb + (cells ? pr[2] - pr[0] : 0.0);
+    return t;
+}
+
+// the cell's three explicit rows on t
+V2G_HD inline void cell_rows(const Cell &t, double (&a)[3])
+{
+    const double an = 0.5 * ((t.ab[1] + t.ab[2]) - (t.ab[0] + t.ab[3]));
+    a[0] = t.aa - t.bb;
+    a[1] = t.aa + an;
+    a[2] = t.bb + an;
+}
+
+// ---- a listed cell: what a shared orbital adds ---------------------------------
+V2G_HD inline int shared_count(const CellRec &c) { return c.flags & CF_TWO ? 2 : 1; }
+// orientation of (ik|jk); (ki|kj), (ki|jk), (ik|kj) are it xor 3, 1, 2
+V2G_HD inline int shared_or(const CellRec &c, int n) { return c.flags >> (2 * n) & 3; }
+
+// a shared orbital's D1 and maximal-spin numbers
+struct Shared {
+    double aij, aji, bij, bji, m0, m1;
+    template <class X, class M>
+    V2G_HD inline Shared(const RedLayout &R, const CellRec &c, int n, const X &x, const M &m)
+    {
+        aij = x[c.ij[n]];
+        aji = x[c.ji[n]];
+        bij = x[c.ij[n] + (int32_t)R.nD1];
+        bji = x[c.ji[n] + (int32_t)R.nD1];
+        m0 = R.nM ? m[c.m0[n]] : 0.0;
+        m1 = R.nM ? m[c.m1[n]] : 0.0;
+    }
+};
+
+V2G_HD inline void add_or(double (&v)[4], int o, double x)
+{
+    for (int k = 0; k < 4; k++) v[k] += k == o ? x : 0.0;
+}
+
+// adds the terms of the shared orbitals, traces and S^2 to t = cell_at(...)
+template <class X, class M, class Y>
+V2G_HD inline void shared_at(const RedLayout &R, const CellRec &c, const X &x, const M &m, const Y &y, Cell &t)
+{
+    const DevLayout &L = R.L;
+    const int64_t c0 = L.rowoff[RF_CONTR][L.sz ? 0 : 4][0] - L.xoff[XB_D1A][0];
+    const int64_t c1 = L.rowoff[RF_CONTR][L.sz ? 1 : 5][0] - L.xoff[XB_D1A][0];
+    const int64_t c2 = L.rowoff[RF_CONTR][L.sz ? 2 : 4][0] - L.xoff[XB_D1A][0];
+    const int64_t c3 = L.rowoff[RF_CONTR][L.sz ? 3 : 5][0] - L.xoff[XB_D1A][0];
+    const double q2 = L.q2 ? 1.0 : 0.0, g2 = L.g2 ? 1.0 : 0.0;
+    for (int n = 0; n < shared_count(c); n++) {
+        const Shared s(R, c, n, x, m);
+        const int o = shared_or(c, n);
+        add_or(t.ab, o, -(q2 * s.aji + g2 * s.aij + y[c0 + c.ij[n]]));
+        add_or(t.ab, o ^ 3, -(q2 * s.bji + g2 * s.bij + y[c1 + c.ij[n]]));
+        add_or(t.ab, o ^ 1, g2 * s.m0);
+        add_or(t.ab, o ^ 2, g2 * s.m1);
+        // like spins: the pairs' order decides the sign
+        const double sg = o == 0 || o == 3 ? -1.0 : 1.0;
+        t.aa += sg * (q2 * s.aji + g2 * s.aij + y[c2 + c.ij[n]]);
+        t.bb += sg * (q2 * s.bji + g2 * s.bij + y[c3 + c.ij[n]]);
+    }
+    if (c.flags & CF_TWO) {   // the same pair twice: a diagonal entry
+        const double tr = L.sz ? y[L.rowoff[RF_TRACE][0][0]] : 2.0 * y[L.rowoff[RF_TRACE][3][0]];
+        t.ab[0] += tr;
+        t.ab[3] += tr;
+        if (L.spin) {
+            const double s2 = y[L.rowoff[RF_S2][0][0]];
+            t.ab[1] += s2;
+            t.ab[2] += s2;
+        }
+        t.aa += 2.0 * y[L.rowoff[RF_TRACE][L.sz ? 1 : 3][0]];
+        t.bb += 2.0 * y[L.rowoff[RF_TRACE][L.sz ? 2 : 3][0]];
+    }
+}
+
+// the D1 / maximal-spin part that the shared orbitals add to a cell's self rows in
+// orientation o: Q2ab, G2ab (and the alpha quadrant), G2ba, the beta quadrant
+struct SharedAt {
+    double q2 = 0.0, g1 = 0.0, g2 = 0.0, gb = 0.0;
+    template <class X, class M>
+    V2G_HD inline SharedAt(const RedLayout &R, const CellRec &c, int o, const X &x, const M &m)
+    {
+        const int32_t b = (int32_t)R.nD1;
+        for (int n = 0; n < shared_count(c); n++) {
+            const int rel = o ^ shared_or(c, n);
+            if (rel == 0) {          // (ik|jk)
+                q2 -= x[c.ji[n]];
+                g1 += x[c.ij[n]];
+                gb += x[c.ij[n] + b];
+            } else if (rel == 3) {   // (ki|kj)
+                q2 -= x[c.ji[n] + b];
+                g2 += x[c.ij[n] + b];
+            } else if (R.nM) {       // (ki|jk), (ik|kj)
+                g2 -= m[rel == 1 ? c.m0[n] : c.m1[n]];
+            }
+        }
+    }
+};
+
+// what they add to the cell's Q2aa (sp = 0) / Q2bb row
+template <class X>
+V2G_HD inline double shared_q2(const RedLayout &R, const CellRec &c, int sp, const X &x)
+{
+    const int32_t b = sp ? (int32_t)R.nD1 : 0;
+    double v = 0.0;
+    for (int n = 0; n < shared_count(c); n++) {
+        const int o = shared_or(c, n);
+        v += o == 0 || o == 3 ? -x[c.ji[n] + b] : x[c.ji[n] + b];
+    }
+    return v;
 }
 
 }  // namespace rows
