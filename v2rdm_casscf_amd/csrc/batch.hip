@@ -38,6 +38,7 @@
 #include "inputs.hpp"
 #include "kernels.hpp"
 #include "layout.hpp"
+#include "redcg.hpp"
 
 namespace v2g {
 namespace {
@@ -328,7 +329,10 @@ struct v2g_batch {
     DevBuf<v2g::ProbRange> d_pr;
     int64_t dimx = 0, ncon = 0;
     hipStream_t st = nullptr;
-    // CG
+    // CG: the reduced form (redcg.hpp, in cgmem), or the general one for batches with
+    // T1, T2 or spin-adapted problems
+    v2g::RedCG redcg;
+    DevBuf<double> cgmem;
     DevBuf<double> r, p, Ap, t, partial, scal, rowpart, tolv;
     // loop
     DevBuf<double> Ax, Bv, ATy, yhist, xprev, red, redout, coefa, coefb, mus;
@@ -361,6 +365,7 @@ struct v2g_batch {
     std::vector<double> seg_dot(int space, const double *u, const double *v);
     void cg(const double *rhs, double *y, const std::vector<double> &tol, int maxiter,
             std::vector<int> &iters, std::vector<double> &res);
+    template <class F> void capture_chunk(double *y, F enqueue);
     void update_xz(const std::vector<double> &mu, const std::vector<int> &act, const double *y,
                    const double *c, double *x, double *z, bool capped, int cross_order);
 };
@@ -508,13 +513,19 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
         HIPCHK(hipStreamSynchronize(st));
     }
     // buffers
-    r.alloc(ncon);
-    p.alloc(ncon);
-    Ap.alloc(ncon);
-    t.alloc(dimx);
-    partial.alloc((size_t)np * v2g::P_N * v2g::kBRed);
-    scal.alloc((size_t)np * v2g::CG_NSLOTS);
-    rowpart.alloc(std::max<int64_t>(1, plan.row_tiles));
+    std::vector<const v2g::Layout *> lp;
+    for (const auto &l : L) lp.push_back(l.get());
+    if (redcg.build(lp, dls, d_lay.p)) {
+        cgmem.alloc(redcg.doubles());
+    } else {
+        r.alloc(ncon);
+        p.alloc(ncon);
+        Ap.alloc(ncon);
+        t.alloc(dimx);
+        partial.alloc((size_t)np * v2g::P_N * v2g::kBRed);
+        scal.alloc((size_t)np * v2g::CG_NSLOTS);
+        rowpart.alloc(std::max<int64_t>(1, plan.row_tiles));
+    }
     tolv.alloc(np);
     Ax.alloc(ncon);
     Bv.alloc(ncon);
@@ -589,11 +600,58 @@ std::vector<double> v2g_batch::seg_dot(int space, const double *u, const double 
     return out;
 }
 
+// one host thread drives the batch on its own stream: the chunk of CG iterations that
+// enqueue() launches is captured once (it holds kernels only) and replayed
+template <class F>
+void v2g_batch::capture_chunk(double *y, F enqueue)
+{
+    if (cg_exec && cg_exec_y == y) return;
+    if (cg_exec) { (void)hipGraphExecDestroy(cg_exec); cg_exec = nullptr; }
+    hipGraph_t g = nullptr;
+    HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    enqueue();
+    HIPCHK(hipStreamEndCapture(st, &g));
+    const hipError_t e = hipGraphInstantiate(&cg_exec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    HIPCHK(e);
+    cg_exec_y = y;
+}
+
 // CG on every problem whose pact flag is set, tolerance per problem
 void v2g_batch::cg(const double *rhs, double *y, const std::vector<double> &tolh, int maxiter,
                    std::vector<int> &iters, std::vector<double> &res)
 {
     const dim3 gy = grid_of(0);
+    if (redcg.ok()) {
+        HIPCHK(hipMemcpyAsync(tolv.p, tolh.data(), sizeof(double) * np, hipMemcpyHostToDevice, st));
+        const v2g::RedBufs B = redcg.carve(cgmem.p);
+        redcg.start(B, rhs, y, 0.0, tolv.p, pact.p, maxiter, st);
+        std::vector<double> hs((size_t)np * v2g::kRedScal);
+        for (int it = 0;;) {
+            // whole chunks are replayed, a last shorter one is launched
+            const int n = std::max(2, (std::min(v2g::kBChunk, maxiter - it) + 1) / 2 * 2);
+            if (n == v2g::kBChunk) {
+                capture_chunk(y, [&] { redcg.iterate(B, y, v2g::kBChunk, st); });
+                HIPCHK(hipGraphLaunch(cg_exec, st));
+            } else {
+                redcg.iterate(B, y, n, st);
+            }
+            it += n;
+            HIPCHK(hipMemcpyAsync(hs.data(), B.scal, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, st));
+            HIPCHK(hipStreamSynchronize(st));
+            bool all = true;
+            for (int q = 0; q < np && all; q++) all = hs[(size_t)q * v2g::kRedScal + v2g::RS_DONE] != 0.0;
+            if (all || it >= maxiter) break;
+        }
+        redcg.finish(B, y, pact.p, st);
+        iters.assign(np, 0);
+        res.assign(np, 0.0);
+        for (int q = 0; q < np; q++) {
+            iters[q] = (int)hs[(size_t)q * v2g::kRedScal + v2g::RS_ITER];
+            res[q] = hs[(size_t)q * v2g::kRedScal + v2g::RS_NRM];
+        }
+        return;
+    }
     HIPCHK(hipMemcpyAsync(tolv.p, tolh.data(), sizeof(double) * np, hipMemcpyHostToDevice, st));
     v2g::launch_atu(plan, y, t.p, st);
     v2g::launch_au(plan, t.p, Ap.p, st);
@@ -615,19 +673,7 @@ void v2g_batch::cg(const double *rhs, double *y, const std::vector<double> &tolh
                                partial.p, scal.p, par);
         }
     };
-    // one host thread drives the batch on its own stream: the chunk is
-    // captured once (it holds kernels only) and replayed
-    if (!cg_exec || cg_exec_y != y) {
-        if (cg_exec) { (void)hipGraphExecDestroy(cg_exec); cg_exec = nullptr; }
-        hipGraph_t g = nullptr;
-        HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        enqueue_chunk();
-        HIPCHK(hipStreamEndCapture(st, &g));
-        const hipError_t e = hipGraphInstantiate(&cg_exec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        HIPCHK(e);
-        cg_exec_y = y;
-    }
+    capture_chunk(y, enqueue_chunk);
     std::vector<double> hs((size_t)np * v2g::CG_NSLOTS);
     int it = 0;
     for (;;) {
