@@ -80,6 +80,7 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
         p(R.nR + 1), mu(R.nM + 1), nu(R.nM + 1), om(R.nM), ams(R.nM);
     const int64_t ms0 = R.nM ? R.L.rowoff[RF_MAXSPIN][0][0] : 0;
     auto wave = [&](auto fn) { double a = 0.0; for (int l = 0; l < 64; l++) a += fn(l); return a; };
+    auto group = [&](auto fn) { double a = 0.0; for (int l = 0; l < R.lanes; l++) a += fn(l); return a; };
     // every D2 / D1 entry once: ab(entry), aa(spin, cell, irrep, place), d1(segment, item)
     auto each_entry = [&](auto ab, auto aa, auto d1) {
         std::vector<char> seen((size_t)R.nD, 0);
@@ -165,7 +166,7 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
                 if (sg.kind == RF_MAXSPIN) a = msrow(sg.sub, (int)e);
                 else if (sg.kind == RF_SPIN_D1) a = t[R.L.xoff[XB_D1A][sg.h] + e] - t[R.L.xoff[XB_D1B][sg.h] + e];
                 else {
-                    const int lanes = sg.wave == 1 ? 64 : 256;
+                    const int lanes = sg.wave == 3 ? R.lanes : 256;
                     for (int l = 0; l < lanes; l++) a += long_row(R, sg, e, l, lanes, t);
                 }
                 visit(sg.start + e, sg.aux + e, a);
@@ -183,8 +184,8 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
         s.at(sl) = rhs[row] - y[row] - dx + pm;
     });
     explicit_rows([&](int o, int e) {
-        return -wave([&](int l) { return ms_row_self(R, o, e, l, 1.0, ys, zD, none); }) +
-               wave([&](int l) { return ms_row_gram(R, o, e, l, yms); });
+        return -group([&](int l) { return ms_row_self(R, o, e, l, 1.0, ys, zD, none); }) +
+               group([&](int l) { return ms_row_gram(R, o, e, l, yms); });
     }, [&](int64_t i, int64_t row, double a) { r.at(i) = rhs[row] - a; });
     each_entry([&](const AbEntry &a) { g.at(a.pos) = self_at_ab(R, a, s); },
                [&](int sp, const AbEntry &a, int h, int64_t k) { g.at(R.nAB + sp * R.nAA + k) = self_at_aa(R, sp, h, a, s); },
@@ -226,15 +227,15 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
                     const AbRec a = W.ab.at((size_t)i);
                     keep(a.pos, rec_expl_ab(R, a, p) + AbVals(R, a, v).gram(R, a) + (nu[a.m0] + nu[a.m1]));
                 } else if (sg.kind == XS_D1) {
-                    keep(sg.start + i, wave([&](int l) { return atu_d1_wave<false, true>(R.L, sg, i, l, p) +
+                    keep(sg.start + i, group([&](int l) { return atu_d1_wave<false, true>(R.L, sg, i, l, p) +
                                                                 gram_d1(R, sg.sub, sg.h, i, l, v, nu); }));
                 }
             }
         struct Ms { const Vec &p; int64_t o; double operator[](int64_t i) const { return p[o + i]; } } pm{p, ms0};
         for (int k = 0; k < R.nM; k++) {
             const int g0 = R.nM / 2, o = k / g0, e = k % g0;
-            const double self = wave([&](int l) { return ms_row_self(R, o, e, l, d, s, v, nu); });
-            const double gr = wave([&](int l) { return ms_row_gram(R, o, e, l, pm); });
+            const double self = group([&](int l) { return ms_row_self(R, o, e, l, d, s, v, nu); });
+            const double gr = group([&](int l) { return ms_row_gram(R, o, e, l, pm); });
             ams.at(k) = gr - self;
             pap += pm[k] * (gr - 2.0 * self);
         }

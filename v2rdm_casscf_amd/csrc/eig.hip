@@ -85,72 +85,8 @@ __device__ __forceinline__ void rot2x2(double cp, double sp, double cr, double s
     o[3] = fma(sr, u10, cr * u11);
 }
 
-// parallel cyclic Jacobi on the leading m x m part (m even, m <= kP) of the
-// symmetric matrix S (pitch kLd) in LDS, accumulating rotations into Q; rows
-// and columns beyond m are zero in S and the identity in Q, and stay so.
-// Returns the number of rotations applied.
-__device__ int lds_jacobi(double *S, double *Q, int m, double tol, int maxsweeps, int *sh_cnt,
-                          double *sh_c, double *sh_s, int *sh_pa, int *sh_pb)
-{
-    int total = 0;
-    const int h = m / 2;
-    for (int sweep = 0; sweep < maxsweeps; sweep++) {
-        if (threadIdx.x == 0) *sh_cnt = 0;
-        __syncthreads();
-        for (int r = 0; r < m - 1; r++) {
-            if (threadIdx.x < h) {
-                int a, b;
-                circle_pair(m, r, threadIdx.x, a, b);
-                const int p = a < b ? a : b, q = a < b ? b : a;
-                const double apq = S[p * kLd + q];
-                double c = 1.0, s = 0.0;
-                if (fabs(apq) > tol) {
-                    const double app = S[p * kLd + p], aqq = S[q * kLd + q];
-                    jacobi_rotation(app, aqq, apq, c, s);
-                    atomicAdd(sh_cnt, 1);
-                }
-                sh_c[threadIdx.x] = c;
-                sh_s[threadIdx.x] = s;
-                sh_pa[threadIdx.x] = p;
-                sh_pb[threadIdx.x] = q;
-            }
-            __syncthreads();
-            // S <- R^T S R on every 2x2 (row pair, column pair) block
-            for (int w = threadIdx.x; w < h * h; w += kT) {
-                const int P = w / h, R = w % h;
-                const double cp = sh_c[P], sp = sh_s[P], cr = sh_c[R], sr = sh_s[R];
-                if (sp == 0.0 && sr == 0.0) continue;
-                const int p0 = sh_pa[P], p1 = sh_pb[P], r0 = sh_pa[R], r1 = sh_pb[R];
-                const double b00 = S[p0 * kLd + r0], b01 = S[p0 * kLd + r1];
-                const double b10 = S[p1 * kLd + r0], b11 = S[p1 * kLd + r1];
-                double o[4];
-                rot2x2(cp, sp, cr, sr, b00, b01, b10, b11, o);
-                S[p0 * kLd + r0] = o[0];
-                S[p0 * kLd + r1] = o[1];
-                S[p1 * kLd + r0] = o[2];
-                S[p1 * kLd + r1] = o[3];
-            }
-            // Q <- Q R on column pairs (rows beyond m are zero in these columns)
-            for (int w = threadIdx.x; w < m * h; w += kT) {
-                const int row = w / h, R = w % h;
-                const double cr = sh_c[R], sr = sh_s[R];
-                if (sr == 0.0) continue;
-                const int r0 = sh_pa[R], r1 = sh_pb[R];
-                const double v0 = Q[row * kLd + r0], v1 = Q[row * kLd + r1];
-                Q[row * kLd + r0] = fma(cr, v0, -(sr * v1));
-                Q[row * kLd + r1] = fma(sr, v0, cr * v1);
-            }
-            __syncthreads();
-        }
-        const int cnt = *sh_cnt;
-        __syncthreads();
-        total += cnt;
-        if (cnt == 0) break;
-    }
-    return total;
-}
-
-// The pair sub-problems of the large-block path use a leaner variant:
+// Parallel Jacobi in one workgroup, for the pair sub-problems of the large blocks
+// (pair_jacobi) and for whole small blocks (small_jacobi):
 //  * S keeps only its upper triangle (element (i, j) lives at (min, max)); a
 //    step updates the 528 pair blocks (P <= R) instead of all 1024;
 //  * Q lives in registers: wave w, lane l holds column l, rows
@@ -321,55 +257,186 @@ __device__ int pair_jacobi(double *S, double (&q)[PairShape<NT>::kRowsPerWave], 
 }
 
 // ---- small blocks: whole problem in one workgroup --------------------------
-__global__ void __launch_bounds__(kT)
+// Cyclic Jacobi of the leading m x m part of S (m even, m <= kP; upper triangle in
+// LDS), rotations accumulated into q: wave w, lane l holds column l, rows 16 w .. 16 w +
+// 15.  The circle runs over m players, so a small block takes m - 1 steps a sweep.
+// any[2]: whether the step rotated at all (by step parity); a step that did not is
+// over after its first barrier, and a sweep without rotations ends the solve.
+constexpr int kSmallRows = kP * 64 / kT;
+
+__device__ __forceinline__ int wrap(int x, int mm)   // x mod mm, 0 <= x < 3 mm
+{
+    x = x >= 2 * mm ? x - 2 * mm : x;
+    return x >= mm ? x - mm : x;
+}
+
+__device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double tol, int maxsweeps,
+                             const unsigned short *ut, double *sh_c, double *sh_s, int *sh_pa, int *sh_pb,
+                             double *sh_cl, double *sh_sl, int *sh_any)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = m / 2, mm = m - 1, npair = h * (h + 1) / 2;
+    for (int sweep = 0; sweep < maxsweeps; sweep++) {
+        bool rotated_any = false;
+        for (int r = 0; r < mm; r++) {
+            // partner of this lane in step r: m - 1 with r, the others l with 2 r - l mod (m - 1)
+            int pl = lane;
+            if (lane < m)
+                pl = lane == mm ? r : lane == r ? mm : wrap(2 * r - lane + mm, mm);
+            if (wave == 0) {
+                const int p = lane < pl ? lane : pl, qq = lane < pl ? pl : lane;
+                bool rot = false;
+                if (lane == p && lane < qq) {
+                    const double apq = S[p * kLd + qq];
+                    double c = 1.0, sn = 0.0;
+                    if (fabs(apq) > tol) {
+                        jacobi_rotation(S[p * kLd + p], S[qq * kLd + qq], apq, c, sn);
+                        rot = true;
+                    }
+                    int k = 0;
+                    if (lane != r && qq != mm) {
+                        const int d = wrap(lane - r + mm, mm);
+                        k = d <= h - 1 ? d : wrap(r - lane + mm, mm);
+                    }
+                    sh_c[k] = c;
+                    sh_s[k] = sn;
+                    sh_pa[k] = p;
+                    sh_pb[k] = qq;
+                    sh_cl[p] = sh_cl[qq] = c;
+                    sh_sl[p] = -sn;
+                    sh_sl[qq] = sn;
+                }
+                const unsigned long long b = __ballot(rot);
+                if (lane == 0) sh_any[r & 1] = b != 0;
+            }
+            __syncthreads();
+            if (!sh_any[r & 1]) continue;
+            rotated_any = true;
+            constexpr int kPer = (kUT + kT - 1) / kT;
+            double o[kPer][4];
+            int addr[kPer][4];
+            bool act[kPer];
+#pragma unroll
+            for (int u = 0; u < kPer; u++) {
+                const int w = threadIdx.x + u * kT;
+                act[u] = false;
+                if (w < npair) {
+                    const int P = ut[w] & 0xff, R = ut[w] >> 8;
+                    const double cp = sh_c[P], sp = sh_s[P], cr = sh_c[R], sr = sh_s[R];
+                    act[u] = !(sp == 0.0 && sr == 0.0);
+                    if (act[u]) {
+                        const int p0 = sh_pa[P], p1 = sh_pb[P], r0 = sh_pa[R], r1 = sh_pb[R];
+                        auto ad = [](int i, int j) { return i < j ? i * kLd + j : j * kLd + i; };
+                        addr[u][0] = ad(p0, r0);
+                        addr[u][1] = ad(p0, r1);
+                        addr[u][2] = ad(p1, r0);
+                        addr[u][3] = ad(p1, r1);
+                        rot2x2(cp, sp, cr, sr, S[addr[u][0]], S[addr[u][1]], S[addr[u][2]], S[addr[u][3]], o[u]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kPer; u++)
+                if (act[u])
+#pragma unroll
+                    for (int e = 0; e < 4; e++) S[addr[u][e]] = o[u][e];
+            if (wave * kSmallRows < m) {
+                const double c = lane < m ? sh_cl[lane] : 1.0, sn = lane < m ? sh_sl[lane] : 0.0;
+                double t[kSmallRows];
+#pragma unroll
+                for (int i = 0; i < kSmallRows; i++) t[i] = __shfl(q[i], pl, 64);
+#pragma unroll
+                for (int i = 0; i < kSmallRows; i++) q[i] = fma(c, q[i], sn * t[i]);
+            }
+            __syncthreads();
+        }
+        if (!rotated_any) break;
+        __syncthreads();   // the last step's flag is read before the next sweep's first is written
+    }
+}
+
+// One block (n <= 64) a workgroup.  LDS holds S alone (33 KB; Q lives in registers, M is
+// formed again at the end), so four workgroups share a CU where
+// S, Q and M in LDS let in one: a bond scan has a thousand such blocks at once.
+__global__ void __launch_bounds__(kT, 4)
 k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         const double *__restrict__ c, double *__restrict__ x, double *__restrict__ z, double mu0,
         EigBatch eb)
 {
     __shared__ double S[kP * kLd];
-    __shared__ double Q[kP * kLd];
-    __shared__ double Mv[kP * kLd];
-    __shared__ double sh_c[kP / 2], sh_s[kP / 2], lam[kP], red[kT / 64];
-    __shared__ int sh_pa[kP / 2], sh_pb[kP / 2], sh_cnt;
+    __shared__ double sh_c[kP / 2], sh_s[kP / 2], sh_cl[kP], sh_sl[kP], lam[kP], red[kT / 64];
+    __shared__ int sh_pa[kP / 2], sh_pb[kP / 2], sh_any[2];
+    __shared__ unsigned short ut[kUT];
     const EigBlock B = blocks[blockIdx.x];
     if (eb.active && !eb.active[B.prob]) return;
     const double mu = eb.mus ? eb.mus[B.prob] : mu0;
-    const int n = B.n;
+    const int n = B.n, m = (n + 1) & ~1, h = m / 2;
     const int64_t o = B.xoff;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    // this thread's 16 elements: the layout of the MFMA result (row 16 b + 4 r + lk, column
+    // 16 wave + li)
+    const int col = 16 * wave + li;
+    auto element = [&](int e) -> double {
+        const int row = 16 * (e >> 2) + 4 * (e & 3) + lk;
+        if (row >= n || col >= n) return 0.0;
+        const int64_t ipq = o + (int64_t)row * n + col, iqp = o + (int64_t)col * n + row;
+        return 0.5 * ((aty[ipq] - c[ipq] + mu * x[ipq]) + (aty[iqp] - c[iqp] + mu * x[iqp]));
+    };
     double fro = 0.0;
-    for (int w = threadIdx.x; w < kP * kP; w += kT) {
-        const int p = w / kP, q = w % kP;
-        double v = 0.0;
-        if (p < n && q < n) {
-            const int64_t ipq = o + (int64_t)p * n + q, iqp = o + (int64_t)q * n + p;
-            v = 0.5 * ((aty[ipq] - c[ipq] + mu * x[ipq]) + (aty[iqp] - c[iqp] + mu * x[iqp]));
-        }
-        S[p * kLd + q] = v;
-        Mv[p * kLd + q] = v;
-        Q[p * kLd + q] = (p == q) ? 1.0 : 0.0;
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const double v = element(e);
+        S[(16 * (e >> 2) + 4 * (e & 3) + lk) * kLd + col] = v;
         fro += v * v;
     }
+    for (int P = 0, w0 = 0; P < h; w0 += h - P, P++)
+        for (int k = threadIdx.x; k < h - P; k += kT) ut[w0 + k] = (unsigned short)(P | ((P + k) << 8));
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) fro += __shfl_xor(fro, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = fro;
+    if (lane == 0) red[wave] = fro;
     __syncthreads();
     double tot = 0.0;
     for (int i = 0; i < kT / 64; i++) tot += red[i];
     const double tol = 1e-15 * sqrt(tot) + 1e-300;
-    // the circle runs over n rounded up to even indices, not all kP
-    const int m = (n + 1) & ~1;
-    lds_jacobi(S, Q, m, tol, 60, &sh_cnt, sh_c, sh_s, sh_pa, sh_pb);
+    double q[kSmallRows];
+#pragma unroll
+    for (int i = 0; i < kSmallRows; i++) q[i] = (wave * kSmallRows + i == lane) ? 1.0 : 0.0;
+    if (n > 1)
+        small_jacobi(S, q, m, tol, 60, ut, sh_c, sh_s, sh_pa, sh_pb, sh_cl, sh_sl, sh_any);
+    __syncthreads();
     if (threadIdx.x < kP) {
         const double l = S[threadIdx.x * kLd + threadIdx.x];
-        lam[threadIdx.x] = l > 0.0 ? l / mu : 0.0;
+        lam[threadIdx.x] = threadIdx.x < m && l > 0.0 ? l / mu : 0.0;
     }
+    __syncthreads();   // the diagonal has been read: S takes Q
+#pragma unroll
+    for (int i = 0; i < kSmallRows; i++) S[(wave * kSmallRows + i) * kLd + lane] = q[i];
+    // M once more, before x is overwritten: 16 registers held through the solve would spill
+    double Mv[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) Mv[e] = element(e);
     __syncthreads();
-    for (int w = threadIdx.x; w < n * n; w += kT) {
-        const int p = w / n, q = w % n;
-        double s = 0.0;
-        for (int j = 0; j < m; j++) s += Q[p * kLd + j] * lam[j] * Q[q * kLd + j];
-        x[o + w] = s;
-        z[o + w] = mu * s - Mv[p * kLd + q];
+    // x = Q diag(lam) Q^T, a 64 x 16 strip a wave
+    v4d acc[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) acc[b] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < m; k0 += 4) {
+        const int k = k0 + lk;
+        const double l = lam[k], bv = S[col * kLd + k];
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+            if (16 * b < n)
+                acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * b + li) * kLd + k] * l, bv, acc[b], 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        const int row = 16 * (e >> 2) + 4 * (e & 3) + lk;
+        if (row < n && col < n) {
+            const int64_t i = o + (int64_t)row * n + col;
+            const double xv = acc[e >> 2][e & 3];
+            x[i] = xv;
+            z[i] = mu * xv - Mv[e];
+        }
     }
 }
 

@@ -53,6 +53,13 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// sum over an aligned group of g lanes (16, 32 or 64)
+__device__ __forceinline__ double group_sum(double v, int g)
+{
+    for (int o = g >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
 // sums of N values over the workgroup, in a fixed order; valid in every thread
 template <int N>
 __device__ __forceinline__ void block_sums(double (&v)[N], double *sh)
@@ -113,6 +120,10 @@ __device__ __forceinline__ void for_tiles(const Place &pl, int k, F fn)
         } else if (sg.wave == 1) {
             const int64_t i = tl.first + (threadIdx.x >> 6);
             if (i < sg.count) fn(sg, i, (int)(threadIdx.x & 63));
+        } else if (sg.wave == 3) {
+            const int g = pl.pr->R.lanes;
+            const int64_t i = tl.first + threadIdx.x / g;
+            if (i < sg.count) fn(sg, i, (int)(threadIdx.x % g));
         } else {
             fn(sg, tl.first, (int)threadIdx.x);
         }
@@ -436,7 +447,7 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
         } else if (sg.kind == RK_MS) {
             // sum_i of A^T y over the row's G2ba entries: P^T P y_ms - P^T y_self
             const int pr = R.L.bab[R.L.bab_off[0] + i], k = P0(pr), l = P1(pr);
-            double v = ms_row_gram(R, sg.sub, (int)i, lane, ms);
+            double v = lane < R.lanes ? ms_row_gram(R, sg.sub, (int)i, lane, ms) : 0.0;
             for (int j = lane; j < R.L.amo; j += 64) {
                 const AbEntry a{sg.sub ? l : j, sg.sub ? j : k, sg.sub ? j : l, sg.sub ? k : j, 0};
                 v -= y[self_row_ab(Lo, SF_G2BA, a)];
@@ -449,7 +460,7 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
         if (sg.kind == RF_SPIN_D1) {
             row(sg.start + i, sg.aux + i, t[R.L.xoff[XB_D1A][sg.h] + i] - t[R.L.xoff[XB_D1B][sg.h] + i]);
         } else if (sg.kind == RF_CONTR) {
-            const double v = wave_sum(long_row(R, sg, i, lane, 64, t));
+            const double v = group_sum(long_row(R, sg, i, lane, R.lanes, t), R.lanes);
             if (lane == 0) row(sg.start + i, sg.aux + i, v);
         } else if (sg.wave == 2) {
             double v[1] = {long_row(R, sg, i, lane, kNT, t)};
@@ -539,8 +550,8 @@ k_red_dir(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
             keep(a.pos, t);
         } else if (sg.kind == XS_D1) {
             const int64_t k = sg.start + i;
-            const double t = wave_sum(atu_d1_wave<false, true>(R.L, sg, i, lane, p) +
-                                      gram_d1(R, sg.sub, sg.h, i, lane, v, nu)) + d * V.g[k];
+            const double t = group_sum(atu_d1_wave<false, true>(R.L, sg, i, lane, p) +
+                                           gram_d1(R, sg.sub, sg.h, i, lane, v, nu), R.lanes) + d * V.g[k];
             if (lane == 0) keep(k, t);
         } else if (sg.kind == RK_ROWS) {
             V.p1[sg.start + i] = p[sg.start + i];
@@ -551,8 +562,8 @@ k_red_dir(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
             // of ||A^T p||^2 beyond ||p_self||^2
             const int64_t m0 = R.L.rowoff[RF_MAXSPIN][0][0];
             const Axpy ps{V.r + m0, V.p0 + m0, ev.beta};
-            const double self = wave_sum(ms_row_self(R, sg.sub, (int)i, lane, d, Ptr{V.s}, v, nu));
-            const double gr = wave_sum(ms_row_gram(R, sg.sub, (int)i, lane, ps));
+            const double self = group_sum(ms_row_self(R, sg.sub, (int)i, lane, d, Ptr{V.s}, v, nu), R.lanes);
+            const double gr = group_sum(ms_row_gram(R, sg.sub, (int)i, lane, ps), R.lanes);
             if (lane == 0) {
                 const int64_t k = sg.sub * (R.nM / 2) + i;
                 V.ams[k] = gr - self;
@@ -641,7 +652,7 @@ k_red_res(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
         } else if (sg.kind == RF_SPIN_D1) {
             row(sg.start + i, sg.aux + i, t[R.L.xoff[XB_D1A][sg.h] + i] - t[R.L.xoff[XB_D1B][sg.h] + i]);
         } else if (sg.kind == RF_CONTR) {
-            const double at = wave_sum(long_row(R, sg, i, lane, 64, t));
+            const double at = group_sum(long_row(R, sg, i, lane, R.lanes, t), R.lanes);
             if (lane == 0) row(sg.start + i, sg.aux + i, at);
         } else if (sg.wave == 2) {
             double at[1] = {long_row(R, sg, i, lane, kNT, t)};
@@ -851,7 +862,7 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
             const auto &v = k == 0 ? work[q].start : k == 1 ? work[q].dir : k == 2 ? work[q].res : work[q].norm;
             to[4 * q + k] = tl.size();
             for (const Segment &s : v) {
-                const int64_t per = s.wave == 0 ? kNT : s.wave == 1 ? kWaves : 1;
+                const int64_t per = s.wave == 0 ? kNT : s.wave == 1 ? kWaves : s.wave == 3 ? kNT / prob[q].R.lanes : 1;
                 for (int64_t i = 0; i < s.count; i += per) tl.push_back({s, i});
             }
             prob[q].ntile[k] = (int)(tl.size() - to[4 * q + k]);

@@ -24,7 +24,7 @@ enum RedKind : int {
 };
 
 // work lists of one problem.  Segment::wave: 0 one thread per item, 1 one
-// wavefront, 2 one workgroup; Segment::start: first entry of the compact vector;
+// wavefront, 2 one workgroup, 3 RedLayout::lanes threads; Segment::start: first entry of the compact vector;
 // Segment::aux: first row of the full vector
 struct RedWork {
     // start and end of a solve, direction, residual, norms

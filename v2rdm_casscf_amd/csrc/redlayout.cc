@@ -15,6 +15,7 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
     const bool q2 = Lt.q2_plain(), g2 = Lt.g2_plain();
     R.nblk_d = Lt.opt.spin ? (Lt.singlet ? 1 : 4) : 0;
     R.nM = Lt.opt.spin && g2 ? 2 * Lt.gems_ab[0] : 0;
+    R.lanes = Lt.amo <= 16 ? 16 : Lt.amo <= 32 ? 32 : 64;
     R.cells = Lt.opt.spin && Lt.singlet ? 1 : 0;
 
     auto seg = [](std::vector<Segment> &v, int kind, int sub, int h, int dim, int64_t start,
@@ -150,13 +151,19 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
     seg(w.start, RK_DVEC, 0, 0, 0, 0, R.nD, 0, 0);
     seg(w.start, RK_RVEC, 0, 0, 0, 0, R.nR, 0, 0);
     seg(w.start, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
-    cat(w.dir, d1);
-    cat(w.dir, ms);
+    // rows summed over the orbitals take a full wavefront only where the orbitals fill it
+    auto grouped = [](std::vector<Segment> v) {
+        for (Segment &x : v)
+            if (x.wave == 1) x.wave = 3;
+        return v;
+    };
+    cat(w.dir, grouped(d1));
+    cat(w.dir, grouped(ms));
     seg(w.dir, RK_LIST_AB, 0, 0, 0, 0, nout, 0, 0);
     cat(w.dir, bulk);
     seg(w.dir, RK_ROWS, 0, 0, 0, rest0, R.nR - rest0, 0, 0);
     seg(w.dir, RK_MVEC, 0, 0, 0, 0, R.nM, 0, 0);
-    cat(w.res, lng);
+    cat(w.res, grouped(lng));
     cat(w.res, rest);
     seg(w.res, RK_STEP, 0, 0, 0, R.dA, 2 * ndiag, 0, 0);
     seg(w.res, RK_STEP, 0, 0, 0, R.nAB + 2 * R.nAA, 2 * nd1, 0, 0);

@@ -59,6 +59,7 @@ struct RedLayout {
     int cells;
     int64_t nD1;     // D1a entries
     int nM;          // maximal-spin rows (2 gems_ab[0], or 0)
+    int lanes;       // threads that share a row summed over the orbitals: 16, 32 or 64
     int nblk_d;      // D200 quadrants: 0 (spin off), 1 (singlet), 4
 };
 
@@ -263,7 +264,7 @@ V2G_HD inline double ms_part(const RedLayout &R, int p, int q, int r, int s, con
     return v;
 }
 
-// B2^T (B2 x - P m) on a D1 entry: lane-strided share of one wavefront
+// B2^T (B2 x - P m) on a D1 entry: lane-strided share of R.lanes threads
 template <class X, class M>
 V2G_HD inline double gram_d1(const RedLayout &R, int sp, int h, int64_t item, int lane, const X &x,
                              const M &m)
@@ -277,7 +278,7 @@ V2G_HD inline double gram_d1(const RedLayout &R, int sp, int h, int64_t item, in
     const double xd = x[L.xoff[wd][h] + item];
     const int others = L.amo - (A == B ? 1 : 2);
     double v = lane == 0 ? xd * (1.0 + (L.q2 ? L.amo + others : 0) + (L.g2 ? 2.0 * L.amo : 0.0)) : 0.0;
-    for (int t = lane; t < L.amo; t += 64) {
+    for (int t = lane; t < L.amo; t += R.lanes) {
         const bool in = t != A && t != B;
         const double sg = ((A < t) == (B < t)) ? 1.0 : -1.0;
         const int64_t k = in ? R.nAB + sp * R.nAA : 0;
@@ -366,7 +367,7 @@ V2G_HD inline double ms_row_gram(const RedLayout &R, int o, int item, int lane, 
     const int pr = L.bab[L.bab_off[0] + item];
     double v = lane == 0 ? L.amo * m[o * g0 + item] : 0.0;
     if (P0(pr) == P1(pr))
-        for (int i = lane; i < L.amo; i += 64) v += m[(1 - o) * g0 + L.gab[i * L.amo + i]];
+        for (int i = lane; i < L.amo; i += R.lanes) v += m[(1 - o) * g0 + L.gab[i * L.amo + i]];
     return v;
 }
 
@@ -381,7 +382,7 @@ V2G_HD inline double ms_row_self(const RedLayout &R, int o, int item, int lane, 
     // the D1b part: its only row with p == r; the P m parts sum to P^T P m
     double v = lane == 0 ? (o ? x[d1_col(L, XB_D1B, l, k)] : x[d1_col(L, XB_D1B, k, l)]) : 0.0;
     v -= ms_row_gram(R, o, item, lane, m);
-    for (int i = lane; i < L.amo; i += 64) {
+    for (int i = lane; i < L.amo; i += R.lanes) {
         // the row's pairs are (q, r) and (s, p)
         const int64_t e = o ? ab_pos(R, l, i, i, k) : ab_pos(R, i, k, l, i);
         v += d * s[R.soff[SF_G2BA] + e] - x[e];
