@@ -109,6 +109,7 @@ struct v2g_solver {
     double last_cg_nrm0 = 0.0;     // ||r|| at the start of the last CG solve
     // eigen split
     std::vector<v2g::EigBlock> small, large;
+    int ntiny = 0;   // leading small blocks of n <= kTinyN
     DevBuf<v2g::EigBlock> d_small, d_large;
     DevBuf<double> Mw, Aw, Tw, Vw, Qbuf, tol, frop;
     DevBuf<int> active, counter;
@@ -344,6 +345,7 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
     // kLaneMinN on, the rounds are latency-bound (two lanes, 1024-thread pairs)
     pair_wide = max_N >= kLaneMinN;
     configure_lanes(max_N >= kLaneMinN ? kMaxLanes : 1);
+    ntiny = v2g::eig_order_small(small);
     d_small.upload(small);
     if (!large.empty()) {
         Mw.alloc(woff);
@@ -728,7 +730,7 @@ void v2g_solver::update_xz(double mu, const double *y, const double *c, double *
                            int warm_sweep_cap, int inner_sweep_cap, int cross_order)
 {
     v2g::launch_atu(plan, y, ATy.p, st);
-    v2g::eig_small(d_small.p, (int)small.size(), ATy.p, c, x, zv, mu, st);
+    v2g::eig_small(d_small.p, (int)small.size(), ntiny, ATy.p, c, x, zv, mu, st);
     last_sweeps = 0;
     if (large.empty()) return;
     const int cold = warm ? 0 : 1;

@@ -339,6 +339,7 @@ struct v2g_batch {
     DevBuf<int> pact, pfirst, pone;
     // eigen split
     std::vector<v2g::EigBlock> small, large;
+    int ntiny = 0;   // leading small blocks of n <= kTinyN
     DevBuf<v2g::EigBlock> d_small, d_large;
     DevBuf<double> Mw, Aw, Tw, Vw, Qbuf, tol, frop;
     DevBuf<int> active, counter;
@@ -563,6 +564,7 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
         max_tiles = std::max(max_tiles, (int64_t)npair * (npair + 1) / 2 + (int64_t)npair * npair);
     }
     pair_wide = max_N >= 512;
+    ntiny = v2g::eig_order_small(small);
     d_small.upload(small);
     d_large.upload(large);
     if (!large.empty()) {
@@ -705,7 +707,7 @@ void v2g_batch::update_xz(const std::vector<double> &mu, const std::vector<int> 
     eb.mus = mus.p;
     eb.active = pact.p;
     v2g::launch_atu(plan, y, ATy.p, st);
-    v2g::eig_small(d_small.p, (int)small.size(), ATy.p, c, x, z, 1.0, st, eb);
+    v2g::eig_small(d_small.p, (int)small.size(), ntiny, ATy.p, c, x, z, 1.0, st, eb);
     if (large.empty()) return;
     const int nl = (int)large.size();
     const int cold = warm ? 0 : 1;

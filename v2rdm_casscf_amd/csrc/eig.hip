@@ -19,6 +19,8 @@
 // Blocks with n <= 64 are solved completely by one workgroup (no warm start).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "eig.hpp"
 
 namespace v2g {
@@ -257,12 +259,14 @@ __device__ int pair_jacobi(double *S, double (&q)[PairShape<NT>::kRowsPerWave], 
 }
 
 // ---- small blocks: whole problem in one workgroup --------------------------
-// Cyclic Jacobi of the leading m x m part of S (m even, m <= kP; upper triangle in
-// LDS), rotations accumulated into q: wave w, lane l holds column l, rows 16 w .. 16 w +
-// 15.  The circle runs over m players, so a small block takes m - 1 steps a sweep.
+// Cyclic Jacobi of the leading m x m part of S (m even, m <= MAXN; upper triangle in
+// LDS), rotations accumulated into q: thread t holds column t % MAXN, rows 16 (t / MAXN)
+// .. + 15.  The circle runs over m players, so a small block takes m - 1 steps a sweep.
 // any[2]: whether the step rotated at all (by step parity); a step that did not is
 // over after its first barrier, and a sweep without rotations ends the solve.
-constexpr int kSmallRows = kP * 64 / kT;
+// MAXN = 64 takes 256 threads; MAXN = 32 a single wavefront, whose steps have nothing to
+// wait for but their own LDS accesses.
+constexpr int kSmallRows = 16;
 
 __device__ __forceinline__ int wrap(int x, int mm)   // x mod mm, 0 <= x < 3 mm
 {
@@ -270,11 +274,13 @@ __device__ __forceinline__ int wrap(int x, int mm)   // x mod mm, 0 <= x < 3 mm
     return x >= mm ? x - mm : x;
 }
 
+template <int NT, int MAXN>
 __device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double tol, int maxsweeps,
                              const unsigned short *ut, double *sh_c, double *sh_s, int *sh_pa, int *sh_pb,
                              double *sh_cl, double *sh_sl, int *sh_any)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int kLd = MAXN + 1;
+    const int lane = threadIdx.x % MAXN, group = threadIdx.x / MAXN;
     const int h = m / 2, mm = m - 1, npair = h * (h + 1) / 2;
     for (int sweep = 0; sweep < maxsweeps; sweep++) {
         bool rotated_any = false;
@@ -283,10 +289,10 @@ __device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double t
             int pl = lane;
             if (lane < m)
                 pl = lane == mm ? r : lane == r ? mm : wrap(2 * r - lane + mm, mm);
-            if (wave == 0) {
+            if (threadIdx.x < 64) {
                 const int p = lane < pl ? lane : pl, qq = lane < pl ? pl : lane;
                 bool rot = false;
-                if (lane == p && lane < qq) {
+                if (group == 0 && lane == p && lane < qq) {
                     const double apq = S[p * kLd + qq];
                     double c = 1.0, sn = 0.0;
                     if (fabs(apq) > tol) {
@@ -307,18 +313,18 @@ __device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double t
                     sh_sl[qq] = sn;
                 }
                 const unsigned long long b = __ballot(rot);
-                if (lane == 0) sh_any[r & 1] = b != 0;
+                if (threadIdx.x == 0) sh_any[r & 1] = b != 0;
             }
             __syncthreads();
             if (!sh_any[r & 1]) continue;
             rotated_any = true;
-            constexpr int kPer = (kUT + kT - 1) / kT;
+            constexpr int kPairs = (MAXN / 2) * (MAXN / 2 + 1) / 2, kPer = (kPairs + NT - 1) / NT;
             double o[kPer][4];
             int addr[kPer][4];
             bool act[kPer];
 #pragma unroll
             for (int u = 0; u < kPer; u++) {
-                const int w = threadIdx.x + u * kT;
+                const int w = threadIdx.x + u * NT;
                 act[u] = false;
                 if (w < npair) {
                     const int P = ut[w] & 0xff, R = ut[w] >> 8;
@@ -340,11 +346,11 @@ __device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double t
                 if (act[u])
 #pragma unroll
                     for (int e = 0; e < 4; e++) S[addr[u][e]] = o[u][e];
-            if (wave * kSmallRows < m) {
+            if (group * kSmallRows < m) {   // rows from m on stay zero in these columns
                 const double c = lane < m ? sh_cl[lane] : 1.0, sn = lane < m ? sh_sl[lane] : 0.0;
                 double t[kSmallRows];
 #pragma unroll
-                for (int i = 0; i < kSmallRows; i++) t[i] = __shfl(q[i], pl, 64);
+                for (int i = 0; i < kSmallRows; i++) t[i] = __shfl(q[i], pl, MAXN);
 #pragma unroll
                 for (int i = 0; i < kSmallRows; i++) q[i] = fma(c, q[i], sn * t[i]);
             }
@@ -358,26 +364,30 @@ __device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double t
 // One block (n <= 64) a workgroup.  LDS holds S alone (33 KB; Q lives in registers, M is
 // formed again at the end), so four workgroups share a CU where
 // S, Q and M in LDS let in one: a bond scan has a thousand such blocks at once.
-__global__ void __launch_bounds__(kT, 4)
+template <int NT, int MAXN>
+__global__ void __launch_bounds__(NT, NT == 64 ? 3 : 4)
 k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         const double *__restrict__ c, double *__restrict__ x, double *__restrict__ z, double mu0,
         EigBatch eb)
 {
-    __shared__ double S[kP * kLd];
-    __shared__ double sh_c[kP / 2], sh_s[kP / 2], sh_cl[kP], sh_sl[kP], lam[kP], red[kT / 64];
-    __shared__ int sh_pa[kP / 2], sh_pb[kP / 2], sh_any[2];
-    __shared__ unsigned short ut[kUT];
+    constexpr int kLd = MAXN + 1, kWav = NT / 64, kStrips = MAXN / 16 / kWav, kRowB = MAXN / 16;
+    __shared__ double S[MAXN * kLd];
+    __shared__ double sh_c[MAXN / 2], sh_s[MAXN / 2], sh_cl[MAXN], sh_sl[MAXN], lam[MAXN], red[kWav];
+    __shared__ int sh_pa[MAXN / 2], sh_pb[MAXN / 2], sh_any[2];
+    __shared__ unsigned short ut[(MAXN / 2) * (MAXN / 2 + 1) / 2];
     const EigBlock B = blocks[blockIdx.x];
     if (eb.active && !eb.active[B.prob]) return;
     const double mu = eb.mus ? eb.mus[B.prob] : mu0;
     const int n = B.n, m = (n + 1) & ~1, h = m / 2;
     const int64_t o = B.xoff;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
-    // this thread's 16 elements: the layout of the MFMA result (row 16 b + 4 r + lk, column
-    // 16 wave + li)
-    const int col = 16 * wave + li;
+    // this thread's 16 elements: the layout of the MFMA results of the wave's column
+    // strips (row 16 b + 4 r + lk, column 16 strip + li)
+    static_assert(kStrips * kRowB * 4 == 16, "16 elements a thread");
+    auto row_of = [&](int e) { return 16 * (e / 4 % kRowB) + 4 * (e & 3) + lk; };
+    auto col_of = [&](int e) { return 16 * (wave * kStrips + e / (4 * kRowB)) + li; };
     auto element = [&](int e) -> double {
-        const int row = 16 * (e >> 2) + 4 * (e & 3) + lk;
+        const int row = row_of(e), col = col_of(e);
         if (row >= n || col >= n) return 0.0;
         const int64_t ipq = o + (int64_t)row * n + col, iqp = o + (int64_t)col * n + row;
         return 0.5 * ((aty[ipq] - c[ipq] + mu * x[ipq]) + (aty[iqp] - c[iqp] + mu * x[iqp]));
@@ -386,56 +396,61 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
 #pragma unroll
     for (int e = 0; e < 16; e++) {
         const double v = element(e);
-        S[(16 * (e >> 2) + 4 * (e & 3) + lk) * kLd + col] = v;
+        S[row_of(e) * kLd + col_of(e)] = v;
         fro += v * v;
     }
     for (int P = 0, w0 = 0; P < h; w0 += h - P, P++)
-        for (int k = threadIdx.x; k < h - P; k += kT) ut[w0 + k] = (unsigned short)(P | ((P + k) << 8));
+        for (int k = threadIdx.x; k < h - P; k += NT) ut[w0 + k] = (unsigned short)(P | ((P + k) << 8));
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) fro += __shfl_xor(fro, off, 64);
     if (lane == 0) red[wave] = fro;
     __syncthreads();
     double tot = 0.0;
-    for (int i = 0; i < kT / 64; i++) tot += red[i];
+    for (int i = 0; i < kWav; i++) tot += red[i];
     const double tol = 1e-15 * sqrt(tot) + 1e-300;
+    const int qc = threadIdx.x % MAXN, qr = threadIdx.x / MAXN * kSmallRows;
     double q[kSmallRows];
 #pragma unroll
-    for (int i = 0; i < kSmallRows; i++) q[i] = (wave * kSmallRows + i == lane) ? 1.0 : 0.0;
+    for (int i = 0; i < kSmallRows; i++) q[i] = (qr + i == qc) ? 1.0 : 0.0;
     if (n > 1)
-        small_jacobi(S, q, m, tol, 60, ut, sh_c, sh_s, sh_pa, sh_pb, sh_cl, sh_sl, sh_any);
+        small_jacobi<NT, MAXN>(S, q, m, tol, 60, ut, sh_c, sh_s, sh_pa, sh_pb, sh_cl, sh_sl, sh_any);
     __syncthreads();
-    if (threadIdx.x < kP) {
+    if (threadIdx.x < MAXN) {
         const double l = S[threadIdx.x * kLd + threadIdx.x];
         lam[threadIdx.x] = threadIdx.x < m && l > 0.0 ? l / mu : 0.0;
     }
     __syncthreads();   // the diagonal has been read: S takes Q
 #pragma unroll
-    for (int i = 0; i < kSmallRows; i++) S[(wave * kSmallRows + i) * kLd + lane] = q[i];
+    for (int i = 0; i < kSmallRows; i++) S[(qr + i) * kLd + qc] = q[i];
     // M once more, before x is overwritten: 16 registers held through the solve would spill
     double Mv[16];
 #pragma unroll
     for (int e = 0; e < 16; e++) Mv[e] = element(e);
     __syncthreads();
-    // x = Q diag(lam) Q^T, a 64 x 16 strip a wave
-    v4d acc[4];
+    // x = Q diag(lam) Q^T, one or two 16-column strips a wave
 #pragma unroll
-    for (int b = 0; b < 4; b++) acc[b] = v4d{0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < m; k0 += 4) {
-        const int k = k0 + lk;
-        const double l = lam[k], bv = S[col * kLd + k];
+    for (int st = 0; st < kStrips; st++) {
+        v4d acc[kRowB];
 #pragma unroll
-        for (int b = 0; b < 4; b++)
-            if (16 * b < n)
-                acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * b + li) * kLd + k] * l, bv, acc[b], 0, 0, 0);
-    }
+        for (int b = 0; b < kRowB; b++) acc[b] = v4d{0.0, 0.0, 0.0, 0.0};
+        const int col = 16 * (wave * kStrips + st) + li;
+        for (int k0 = 0; k0 < m; k0 += 4) {
+            const int k = k0 + lk;
+            const double l = lam[k], bv = S[col * kLd + k];
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const int row = 16 * (e >> 2) + 4 * (e & 3) + lk;
-        if (row < n && col < n) {
-            const int64_t i = o + (int64_t)row * n + col;
-            const double xv = acc[e >> 2][e & 3];
-            x[i] = xv;
-            z[i] = mu * xv - Mv[e];
+            for (int b = 0; b < kRowB; b++)
+                if (16 * b < n)
+                    acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[(16 * b + li) * kLd + k] * l, bv, acc[b], 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4 * kRowB; e++) {
+            const int row = 16 * (e >> 2) + 4 * (e & 3) + lk;
+            if (row < n && col < n) {
+                const int64_t i = o + (int64_t)row * n + col;
+                const double xv = acc[e >> 2][e & 3];
+                x[i] = xv;
+                z[i] = mu * xv - Mv[st * 4 * kRowB + e];
+            }
         }
     }
 }
@@ -853,11 +868,26 @@ k_z(const EigBlock *__restrict__ blocks, const double *__restrict__ x,
 
 }  // namespace
 
-void eig_small(const EigBlock *blocks, int nblocks, const double *aty, const double *c, double *x,
+int eig_order_small(std::vector<EigBlock> &small)
+{
+    std::stable_sort(small.begin(), small.end(), [](const EigBlock &a, const EigBlock &b) {
+        const bool ta = a.n <= kTinyN, tb = b.n <= kTinyN;
+        return ta != tb ? ta : a.n > b.n;
+    });
+    int n = 0;
+    for (const auto &b : small) n += b.n <= kTinyN;
+    return n;
+}
+
+void eig_small(const EigBlock *blocks, int nblocks, int ntiny, const double *aty, const double *c, double *x,
                double *z, double mu, hipStream_t st, EigBatch eb)
 {
-    if (nblocks > 0)
-        hipLaunchKernelGGL(k_small, dim3(nblocks), dim3(kT), 0, st, blocks, aty, c, x, z, mu, eb);
+    // blocks[0 .. ntiny) have n <= 32: a wavefront each; the others 256 threads
+    if (ntiny > 0)
+        hipLaunchKernelGGL((k_small<64, 32>), dim3(ntiny), dim3(64), 0, st, blocks, aty, c, x, z, mu, eb);
+    if (nblocks > ntiny)
+        hipLaunchKernelGGL((k_small<256, 64>), dim3(nblocks - ntiny), dim3(256), 0, st, blocks + ntiny, aty,
+                           c, x, z, mu, eb);
 }
 
 void eig_build_m(const EigBlock *blocks, int nblocks, int max_N, const double *aty, const double *c,

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace v2g {
 
@@ -43,7 +44,12 @@ struct GemmDesc {
     int sym;        // 1: C is symmetric (M == N); only upper tiles are computed
 };
 
-void eig_small(const EigBlock *blocks, int nblocks, const double *aty, const double *c, double *x,
+// blocks of n <= 64, those with n <= kTinyN first (ntiny of them)
+constexpr int kTinyN = 32;
+// puts the small blocks into that order, the largest first within each part (the longest
+// solves start first); returns ntiny
+int eig_order_small(std::vector<EigBlock> &small);
+void eig_small(const EigBlock *blocks, int nblocks, int ntiny, const double *aty, const double *c, double *x,
                double *z, double mu, hipStream_t st, EigBatch eb = {});
 // max_N: the largest padded dimension among the blocks
 void eig_build_m(const EigBlock *blocks, int nblocks, int max_N, const double *aty, const double *c,
