@@ -46,27 +46,33 @@ __device__ __forceinline__ void circle_pair(int m, int r, int k, int &a, int &b)
 // Jacobi rotation (c, s) that annihilates apq.  t = tan(theta), the smaller
 // root: the textbook t = sgn(th) / (|th| + sqrt(th^2 + 1)), th = d / e with
 // d = aqq - app, e = 2 apq, multiplied through by |e|, gives
-// t = sgn(d) e / (|d| + sqrt(d^2 + e^2)): one division instead of three.
-// c = 1 / sqrt(1 + t^2) (1 <= 1 + t^2 <= 2) from the hardware reciprocal square
-// root and two Newton steps; s = t c.
+// t = sgn(d) e / (|d| + sqrt(d^2 + e^2)); c = 1 / sqrt(1 + t^2), s = t c.
+// Both roots and the quotient come from the hardware estimates (better than 2^-20) and
+// one third-order step each, which leaves the rounding of its own last operation: a
+// step of the pair problems waits for this chain, and the library's root and
+// division are about twice as long.
+__device__ __forceinline__ double rsqrt_refined(double x)   // 1 / sqrt(x), x normal and finite
+{
+    const double y = __builtin_amdgcn_rsq(x), e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double &c,
                                                 double &s)
 {
     const double d = aqq - app, e = 2.0 * apq;
-    const double r = sqrt(fma(d, d, e * e));
+    const double h = fma(d, d, e * e);
     double t;
-    if (r > 0.0) {
-        t = (d >= 0.0 ? e : -e) / (fabs(d) + r);
-    } else {   // d^2 + e^2 underflows: the textbook form
+    if (h > 1e-280 && h < 1e280) {
+        const double den = fabs(d) + h * rsqrt_refined(h);
+        const double y = __builtin_amdgcn_rcp(den), f = fma(-den, y, 1.0);
+        t = (d >= 0.0 ? e : -e) * fma(y, fma(f, f, f), y);
+    } else {   // d^2 + e^2 leaves the range: the textbook form
         const double th = d / e;
         t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
     }
-    const double x = fma(t, t, 1.0), hx = 0.5 * x;
-    double y = __builtin_amdgcn_rsq(x);
-    y = fma(y, fma(-hx * y, y, 0.5), y);
-    y = fma(y, fma(-hx * y, y, 0.5), y);
-    c = y;
-    s = t * y;
+    c = rsqrt_refined(fma(t, t, 1.0));
+    s = t * c;
 }
 
 // R_P^T B R_R for one 2 x 2 block B = [b00 b01; b10 b11] with R = [c s; -s c]
@@ -88,297 +94,264 @@ __device__ __forceinline__ void rot2x2(double cp, double sp, double cr, double s
 }
 
 // Parallel Jacobi in one workgroup, for the pair sub-problems of the large blocks
-// (pair_jacobi) and for whole small blocks (small_jacobi):
-//  * S keeps only its upper triangle (element (i, j) lives at (min, max)); a
-//    step updates the 528 pair blocks (P <= R) instead of all 1024;
-//  * Q lives in registers: wave w, lane l holds column l, rows
-//    kRowsPerWave w .. kRowsPerWave (w + 1) - 1.
-//    A column rotation needs the partner column only, which sits in the
-//    partner lane of the same wave, so Q moves through lane shuffles and never
-//    touches LDS.  That leaves one 64 x 65 FP64 array of LDS per workgroup.
-// In step r of the circle method, lane l is paired with 63 <-> r and
-// l <-> (2r - l) mod 63 otherwise; circle_slot(r, l) is the pair's slot (the
-// k of circle_pair(kP, r, k)).
-// x mod 63 for 0 <= x < 189 without a division
-__device__ __forceinline__ int mod63(int x)
-{
-    x = x >= 2 * (kP - 1) ? x - 2 * (kP - 1) : x;
-    return x >= kP - 1 ? x - (kP - 1) : x;
-}
-
-__device__ __forceinline__ int circle_partner(int r, int l)
-{
-    if (l == kP - 1) return r;
-    if (l == r) return kP - 1;
-    return mod63(2 * r - l + (kP - 1));
-}
-
-__device__ __forceinline__ int circle_slot(int r, int l)
-{
-    if (l == kP - 1 || l == r) return 0;
-    const int d = mod63(l - r + (kP - 1));
-    return d <= kP / 2 - 1 ? d : mod63(r - l + (kP - 1));
-}
-
-constexpr int kUT = (kP / 2) * (kP / 2 + 1) / 2;   // 528 pair blocks with P <= R
-// Workgroup size NT of the pair problems.  Large problems have a few hundred
-// pair problems per round, so a step's latency sets the time: NT = 1024 (16
-// waves, one S block and 4 rows of Q per thread) shortens it.  Many small
-// problems at once (bond scans) are throughput-bound: NT = 256 does the same
-// work in fewer instructions.
-template <int NT> struct PairShape {
-    static constexpr int kRowsPerWave = kP * 64 / NT;   // rows of Q a wave holds
-    static constexpr int kUTper = (kUT + NT - 1) / NT;  // S blocks per thread
+// (k_pair_eig) and for whole small blocks (k_small).  m = 2 h indices, h slots; step r
+// rotates one pair of indices a slot:
+//  * cyclic order (the circle method): slot 0 holds (r, m - 1), slot k (r + k, r - k)
+//    modulo m - 1; m - 1 steps visit every pair once;
+//  * cross order (CROSS, m = 64): slot k holds (k, 32 + (k + r) mod 32); 32 steps rotate
+//    every pair with one index in each half once and no pair inside a half.  A split's
+//    sweep uses it after its first round: that round's cyclic order has already rotated
+//    the pairs inside every column block (each block takes part in every round), so the
+//    sweep still visits every pair, in 31 fewer dependent steps per later round.
+// A step is a chain: the pair's elements -> rotation -> update of S = R^T S R and Q <- Q R
+// -> the next step's elements.  What bounds a pair problem is that chain's latency (a few
+// hundred workgroups of one CU each), so the next step's rotations are formed beside
+// this step's update instead of after it: a lane of wave 0 owns the 2 x 2 block of S that
+// holds its next pair (blocks {k - 1, k + 1} of the cyclic order, {k, k + 1} of the cross
+// order), updates it first, and goes on to the rotation, the pair's new diagonal and the
+// publication of (c, s) while the other threads update the other blocks.  One barrier a
+// step.  2 500-wide blocks, 40 pair problems a launch: 58 -> @@ us a launch (1 400 -> @@ ns
+// a step); every index is computed, not looked up, so the reads of S need not wait.
+//  * S keeps its upper triangle (element (i, j) lives at (min, max)), 66 (MAXN + 2) doubles
+//    a row: the accesses of a step walk diagonals and anti-diagonals, whose strides (67, 65)
+//    are odd;
+//  * Q lives in registers.  Cyclic order: a lane holds one column, rows of its wave; the
+//    partner column is fetched by lane shuffles.  Cross order: a lane holds one row, its
+//    wave the columns of a few slots, rotated in place; then the second half's columns
+//    move on by one slot (a register move; one column a wave goes through LDS).
+// NT = 1024: S in the first eight waves, Q in the other eight: where a launch has a few
+// hundred pair problems.  NT = 256 does the same work in fewer instructions, for many small
+// problems at once (bond scans).
+template <int NT, int MAXN, bool CROSS> struct JacobiShape {
+    static constexpr int kH = MAXN / 2, kLd = MAXN + 2;
+    static constexpr int kST = NT == 1024 ? NT / 2 : NT;               // threads of S: the first
+    static constexpr int kU = (kH * (kH - 3) / 2 + kH + kST - 1) / kST;   // blocks of S a thread
+    static constexpr int kQ0 = NT == 1024 ? NT / 2 : 0, kQT = NT - kQ0;   // threads of Q
+    static constexpr int kQ = MAXN * MAXN / kQT;                       // entries of Q a thread
+    static constexpr int kXw = CROSS ? kQT / 64 : 0;
+    static_assert(!CROSS || MAXN == 64, "the cross order is for 64 indices");
+    struct Lds {
+        double2 rot[2][kH];       // (c, s) of the slots, by step parity
+        int any[2];               // whether the step rotates at all
+        double xch[CROSS ? 2 * kXw * 64 : 1];
+    };
 };
 
-// Per step, wave 0 publishes each slot's rotation (sh_c, sh_s) and index pair
-// (sh_pa < sh_pb) for the S update, and each lane's own signed rotation
-// (sh_cl, sh_sl) for the Q update, so no other wave recomputes circle positions.
-// Cross-pair order (bip != 0): step r pairs lane l < 32 (column block a)
-// with lane 32 + ((l + r) mod 32) (column block b), so 32 steps rotate every
-// pair with one index in each block once and no pair inside a block.  A
-// tracking sweep uses it after its first round: that round's cyclic order has
-// already rotated the pairs inside every column block (each block takes part
-// in every round), so the sweep still visits every pair, in 32 + 31 fewer
-// dependent steps per later round.
-__device__ __forceinline__ int cross_partner(int r, int l)
+// the slot at place c of the cycle 0, 1, 3, 5, .., 4, 2 in which the cyclic order's next
+// pairs join neighbours
+__device__ __forceinline__ int cycle_slot(int c, int h)
 {
-    return l < kP / 2 ? kP / 2 + ((l + r) & (kP / 2 - 1)) : ((l - kP / 2 - r) & (kP / 2 - 1));
+    const int odd = h / 2;
+    return c == 0 ? 0 : c <= odd ? 2 * c - 1 : 2 * (h - c);
 }
 
-template <int NT>
-__device__ int pair_jacobi(double *S, double (&q)[PairShape<NT>::kRowsPerWave], double tol,
-                           int maxsweeps, const unsigned short *ut, int *sh_cnt, double *sh_c,
-                           double *sh_s, int *sh_pa, int *sh_pb, double *sh_cl, double *sh_sl,
-                           int bip)
+// Returns whether anything was rotated.  q: see JacobiShape::kQ; on return (CROSS) lane =
+// row, q[s] column s0 + s, q[kQ / 2 + s] column 32 + s0 + s, s0 = kQ / 2 times the wave of Q;
+// else thread t of Q holds column t % MAXN, rows kQ (t / MAXN) ..
+template <int NT, int MAXN, bool CROSS>
+__device__ __forceinline__ bool jacobi(double *S, double (&q)[JacobiShape<NT, MAXN, CROSS>::kQ], int m, double tol,
+                                       int maxsweeps, typename JacobiShape<NT, MAXN, CROSS>::Lds &sh)
 {
-    constexpr int kRowsPerWave = PairShape<NT>::kRowsPerWave, kUTper = PairShape<NT>::kUTper;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // this thread's upper-triangle pair blocks (fixed for the whole solve)
-    int myP[kUTper], myR[kUTper];
+    using Sh = JacobiShape<NT, MAXN, CROSS>;
+    constexpr int kLd = Sh::kLd, kH = Sh::kH, kU = Sh::kU, kQ = Sh::kQ;
+    const int tid = threadIdx.x, h = m / 2, mm = m - 1, nsteps = CROSS ? h : mm;
+    const bool lead = tid < h;      // a lane of wave 0 that forms the rotations of slot tid
+    const bool ofS = tid < Sh::kST, ofQ = tid >= Sh::kQ0;
+    // the two indices of a slot at step 0, and one step on
+    auto first = [&](int k) { return CROSS ? k : k == 0 ? mm : k; };
+    auto second = [&](int k) { return CROSS ? kH + k : k == 0 ? 0 : mm - k; };
+    auto next1 = [&](int x) { return CROSS ? x : x == mm ? mm : x + 1 == mm ? 0 : x + 1; };
+    auto next2 = [&](int x) { return CROSS ? kH + ((x + 1) & (kH - 1)) : x + 1 == mm ? 0 : x + 1; };
+    auto at = [](int i, int j) { return i < j ? i * kLd + j : j * kLd + i; };
+    // this thread's blocks (P < R): slots and their current indices
+    int P[kU], R[kU], p1[kU], p2[kU], r1[kU], r2[kU];
+    bool have[kU];
 #pragma unroll
-    for (int u = 0; u < kUTper; u++) {
-        const int w = threadIdx.x + u * NT;
-        myP[u] = w < kUT ? (ut[w] & 0xff) : -1;
-        myR[u] = w < kUT ? (ut[w] >> 8) : -1;
+    for (int u = 0; u < kU; u++) {
+        const int id = u * Sh::kST + tid - kH;
+        int a, b;
+        if (id < 0) {
+            a = CROSS ? tid : max(tid - 1, 0);
+            b = CROSS ? (tid + 1) & (kH - 1) : min(tid + 1, h - 1);
+            have[u] = lead && h > 1;
+        } else {
+            const int delta = 2 + id / h, c = id % h, c2 = c + delta < h ? c + delta : c + delta - h;
+            have[u] = ofS && (2 * delta < h || (2 * delta == h && c < delta));
+            a = CROSS ? c : cycle_slot(c, h);
+            b = CROSS ? c2 : cycle_slot(c2, h);
+        }
+        P[u] = have[u] ? min(a, b) : 0;
+        R[u] = have[u] ? max(a, b) : 0;
+        p1[u] = first(P[u]);
+        p2[u] = second(P[u]);
+        r1[u] = first(R[u]);
+        r2[u] = second(R[u]);
     }
-    int total = 0;
+    // wave 0: the pair of slot tid
+    int l1 = first(lead ? tid : 0), l2 = second(lead ? tid : 0);
+    auto publish = [&](int buf, double app, double aqq, double apq) {
+        bool rot = false;
+        if (lead) {
+            double c = 1.0, s = 0.0;
+            const int p = min(l1, l2), r = max(l1, l2);
+            if (fabs(apq) > tol) {
+                jacobi_rotation(app, aqq, apq, c, s);
+                rot = true;
+                double o[4];
+                rot2x2(c, s, c, s, app, apq, apq, aqq, o);
+                S[p * kLd + p] = o[0];
+                S[p * kLd + r] = o[2];
+                S[r * kLd + r] = o[3];
+            }
+            sh.rot[buf][tid] = make_double2(c, s);
+        }
+        const unsigned long long b = __ballot(rot);
+        if (tid == 0) sh.any[buf] = b != 0;
+    };
+    if (tid < 64) {
+        const int p = min(l1, l2), r = max(l1, l2);
+        publish(0, S[p * kLd + p], S[r * kLd + r], S[p * kLd + r]);
+        if (NT > 64) __builtin_amdgcn_s_setprio(3);
+    }
+    // Q: cyclic order: this lane's column and its distance from the step number
+    const int qlane = tid % MAXN, qwave = (tid - Sh::kQ0) / 64;
+    int dist = qlane, partner_r = 0;    // (qlane - r) mod mm; r
+    bool first_step = true, total = false;
+    int buf = 0;
+    __syncthreads();
     for (int sweep = 0; sweep < maxsweeps; sweep++) {
-        if (threadIdx.x == 0) *sh_cnt = 0;
-        __syncthreads();
-        const int nsteps = bip ? kP / 2 : kP - 1;
+        bool swept = false;
         for (int r = 0; r < nsteps; r++) {
-            const int pl = bip ? cross_partner(r, lane) : circle_partner(r, lane);
-            if (wave == 0) {
-                const int p = lane < pl ? lane : pl, qq = lane < pl ? pl : lane;
-                bool rotated = false;
-                if (lane == p) {
-                    const double apq = S[p * kLd + qq];
-                    double c = 1.0, sn = 0.0;
-                    if (fabs(apq) > tol) {
-                        const double app = S[p * kLd + p], aqq = S[qq * kLd + qq];
-                        jacobi_rotation(app, aqq, apq, c, sn);
-                        rotated = true;
-                    }
-                    const int k = bip ? p : circle_slot(r, lane);
-                    sh_c[k] = c;
-                    sh_s[k] = sn;
-                    sh_pa[k] = p;
-                    sh_pb[k] = qq;
-                    // column p becomes c q_p - s q_qq, column qq c q_qq + s q_p
-                    sh_cl[p] = c;
-                    sh_sl[p] = -sn;
-                    sh_cl[qq] = c;
-                    sh_sl[qq] = sn;
+            const bool any = sh.any[buf] != 0, last = sweep + 1 == maxsweeps && r + 1 == nsteps;
+            swept |= any;
+            if (ofS && !last) {
+                int n1 = 0, n2 = 0;
+                double app = 0.0, aqq = 0.0, apq = 0.0;
+                if (tid < 64) {
+                    n1 = next1(l1);
+                    n2 = next2(l2);
+                    l1 = n1;
+                    l2 = n2;
+                    app = S[n1 * kLd + n1];
+                    aqq = S[n2 * kLd + n2];
+                    if (n1 > n2) { const double t = app; app = aqq; aqq = t; }
+                    apq = S[at(n1, n2)];
                 }
-                const unsigned long long b = __ballot(rotated);
-                if (lane == 0 && b) *sh_cnt += __popcll(b);
-            }
-            __syncthreads();
-            // S <- R^T S R on the upper-triangle pair blocks.  A thread owns up
-            // to kUTper blocks; all their LDS reads are issued before any
-            // write (the blocks are disjoint), so their latencies overlap.
-            {
-                int addr[kUTper][4];
-                double bv[kUTper][4], cf[kUTper][4];
-                bool act[kUTper];
+                if (any) {
+                    int ad[kU][4];
+                    double bv[kU][4];
+                    double2 cp[kU], cr[kU];
 #pragma unroll
-                for (int u = 0; u < kUTper; u++) {
-                    act[u] = false;
-                    if (myP[u] >= 0) {
-                        const int P = myP[u], R = myR[u];
-                        cf[u][0] = sh_c[P];
-                        cf[u][1] = sh_s[P];
-                        cf[u][2] = sh_c[R];
-                        cf[u][3] = sh_s[R];
-                        act[u] = !(cf[u][1] == 0.0 && cf[u][3] == 0.0);
-                        const int p0 = sh_pa[P], p1 = sh_pb[P], r0 = sh_pa[R], r1 = sh_pb[R];
-                        auto ad = [](int i, int j) { return i < j ? i * kLd + j : j * kLd + i; };
-                        addr[u][0] = ad(p0, r0);
-                        addr[u][1] = ad(p0, r1);
-                        addr[u][2] = ad(p1, r0);
-                        addr[u][3] = ad(p1, r1);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < kUTper; u++)
-                    if (act[u]) {
-#pragma unroll
-                        for (int e = 0; e < 4; e++) bv[u][e] = S[addr[u][e]];
+                    for (int u = 0; u < kU; u++) {
+                        cp[u] = sh.rot[buf][P[u]];
+                        cr[u] = sh.rot[buf][R[u]];
+                        const int pl = min(p1[u], p2[u]), ph = max(p1[u], p2[u]);
+                        const int rl = min(r1[u], r2[u]), rh = max(r1[u], r2[u]);
+                        ad[u][0] = at(pl, rl);
+                        ad[u][1] = at(pl, rh);
+                        ad[u][2] = at(ph, rl);
+                        ad[u][3] = at(ph, rh);
                     }
 #pragma unroll
-                for (int u = 0; u < kUTper; u++)
-                    if (act[u]) {
-                        const double cp = cf[u][0], sp = cf[u][1], cr = cf[u][2], sr = cf[u][3];
-                        const double b00 = bv[u][0], b01 = bv[u][1], b10 = bv[u][2], b11 = bv[u][3];
+                    for (int u = 0; u < kU; u++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) bv[u][e] = S[ad[u][e]];
+#pragma unroll
+                    for (int u = 0; u < kU; u++) {
+                        if (!have[u] || (cp[u].y == 0.0 && cr[u].y == 0.0)) continue;
                         double o[4];
-                        rot2x2(cp, sp, cr, sr, b00, b01, b10, b11, o);
+                        rot2x2(cp[u].x, cp[u].y, cr[u].x, cr[u].y, bv[u][0], bv[u][1], bv[u][2], bv[u][3], o);
 #pragma unroll
-                        for (int e = 0; e < 4; e++) S[addr[u][e]] = o[e];
+                        for (int e = 0; e < 4; e++) S[ad[u][e]] = o[e];
+                        if (u == 0 && lead) {
+                            const int w = at(n1, n2);
+                            apq = w == ad[u][0] ? o[0] : w == ad[u][1] ? o[1] : w == ad[u][2] ? o[2] : o[3];
+                        }
                     }
-            }
-            // Q <- Q R in registers; every lane takes part in the shuffles
-            {
-                const double c = sh_cl[lane], sn = sh_sl[lane];
-                // all shuffles first, then the arithmetic: one wait for the
-                // whole batch instead of one per row
-                double o[kRowsPerWave];
+                }
+                if (tid < 64) publish(buf ^ 1, app, aqq, apq);
 #pragma unroll
-                for (int i = 0; i < kRowsPerWave; i++) o[i] = __shfl(q[i], pl, 64);
-#pragma unroll
-                for (int i = 0; i < kRowsPerWave; i++) q[i] = fma(c, q[i], sn * o[i]);
+                for (int u = 0; u < kU; u++) {
+                    p1[u] = next1(p1[u]);
+                    p2[u] = next2(p2[u]);
+                    r1[u] = next1(r1[u]);
+                    r2[u] = next2(r2[u]);
+                }
             }
+            if (ofQ) {
+                if constexpr (CROSS) {
+                    constexpr int kS = kQ / 2, kW = Sh::kXw;
+                    if (!first_step) q[kQ - 1] = sh.xch[((buf ^ 1) * kW + (qwave + 1) % kW) * 64 + (tid & 63)];
+                    if (any) {
+#pragma unroll
+                        for (int s = 0; s < kS; s++) {
+                            const double2 cs = sh.rot[buf][qwave * kS + s];
+                            const double a = q[s], b = q[kS + s];
+                            q[s] = fma(cs.x, a, -cs.y * b);
+                            q[kS + s] = fma(cs.x, b, cs.y * a);
+                        }
+                    }
+                    sh.xch[(buf * kW + qwave) * 64 + (tid & 63)] = q[kS];
+#pragma unroll
+                    for (int s = 0; s + 1 < kS; s++) q[kS + s] = q[kS + s + 1];
+                    first_step = false;
+                } else {
+                    if (any && (tid - Sh::kQ0) / MAXN * kQ < m) {   // rows from m on stay zero
+                        const bool in = qlane < m;
+                        int pl = qlane, slot = 0;
+                        if (in) {
+                            pl = qlane == mm ? partner_r : dist == 0 ? mm : partner_r - dist + (partner_r < dist ? mm : 0);
+                            slot = qlane == mm ? 0 : dist < h ? dist : mm - dist;
+                        }
+                        const double2 cs = sh.rot[buf][slot];
+                        const double c = in ? cs.x : 1.0, sn = in ? (qlane < pl ? -cs.y : cs.y) : 0.0;
+                        // all shuffles first, then the arithmetic: one wait for the batch
+                        double o[kQ];
+#pragma unroll
+                        for (int i = 0; i < kQ; i++) o[i] = __shfl(q[i], pl, MAXN);
+#pragma unroll
+                        for (int i = 0; i < kQ; i++) q[i] = fma(c, q[i], sn * o[i]);
+                    }
+                    dist = dist == 0 ? mm - 1 : dist - 1;
+                    partner_r = partner_r + 1 == mm ? 0 : partner_r + 1;
+                }
+            }
+            buf ^= 1;
             __syncthreads();
         }
-        const int cnt = *sh_cnt;
-        __syncthreads();
-        total += cnt;
-        if (cnt == 0) break;
+        total |= swept;
+        if (!swept) break;
     }
+    if constexpr (CROSS) {
+        if (ofQ && !first_step)
+            q[kQ - 1] = sh.xch[((buf ^ 1) * Sh::kXw + (qwave + 1) % Sh::kXw) * 64 + (tid & 63)];
+    }
+    if (NT > 64 && tid < 64) __builtin_amdgcn_s_setprio(0);
     return total;
 }
 
-// ---- small blocks: whole problem in one workgroup --------------------------
-// Cyclic Jacobi of the leading m x m part of S (m even, m <= MAXN; upper triangle in
-// LDS), rotations accumulated into q: thread t holds column t % MAXN, rows 16 (t / MAXN)
-// .. + 15.  The circle runs over m players, so a small block takes m - 1 steps a sweep.
-// any[2]: whether the step rotated at all (by step parity); a step that did not is
-// over after its first barrier, and a sweep without rotations ends the solve.
-// MAXN = 64 takes 256 threads; MAXN = 32 a single wavefront, whose steps have nothing to
-// wait for but their own LDS accesses.
-constexpr int kSmallRows = 16;
-
-__device__ __forceinline__ int wrap(int x, int mm)   // x mod mm, 0 <= x < 3 mm
-{
-    x = x >= 2 * mm ? x - 2 * mm : x;
-    return x >= mm ? x - mm : x;
-}
-
-template <int NT, int MAXN>
-__device__ void small_jacobi(double *S, double (&q)[kSmallRows], int m, double tol, int maxsweeps,
-                             const unsigned short *ut, double *sh_c, double *sh_s, int *sh_pa, int *sh_pb,
-                             double *sh_cl, double *sh_sl, int *sh_any)
-{
-    constexpr int kLd = MAXN + 1;
-    const int lane = threadIdx.x % MAXN, group = threadIdx.x / MAXN;
-    const int h = m / 2, mm = m - 1, npair = h * (h + 1) / 2;
-    for (int sweep = 0; sweep < maxsweeps; sweep++) {
-        bool rotated_any = false;
-        for (int r = 0; r < mm; r++) {
-            // partner of this lane in step r: m - 1 with r, the others l with 2 r - l mod (m - 1)
-            int pl = lane;
-            if (lane < m)
-                pl = lane == mm ? r : lane == r ? mm : wrap(2 * r - lane + mm, mm);
-            if (threadIdx.x < 64) {
-                const int p = lane < pl ? lane : pl, qq = lane < pl ? pl : lane;
-                bool rot = false;
-                if (group == 0 && lane == p && lane < qq) {
-                    const double apq = S[p * kLd + qq];
-                    double c = 1.0, sn = 0.0;
-                    if (fabs(apq) > tol) {
-                        jacobi_rotation(S[p * kLd + p], S[qq * kLd + qq], apq, c, sn);
-                        rot = true;
-                    }
-                    int k = 0;
-                    if (lane != r && qq != mm) {
-                        const int d = wrap(lane - r + mm, mm);
-                        k = d <= h - 1 ? d : wrap(r - lane + mm, mm);
-                    }
-                    sh_c[k] = c;
-                    sh_s[k] = sn;
-                    sh_pa[k] = p;
-                    sh_pb[k] = qq;
-                    sh_cl[p] = sh_cl[qq] = c;
-                    sh_sl[p] = -sn;
-                    sh_sl[qq] = sn;
-                }
-                const unsigned long long b = __ballot(rot);
-                if (threadIdx.x == 0) sh_any[r & 1] = b != 0;
-            }
-            __syncthreads();
-            if (!sh_any[r & 1]) continue;
-            rotated_any = true;
-            constexpr int kPairs = (MAXN / 2) * (MAXN / 2 + 1) / 2, kPer = (kPairs + NT - 1) / NT;
-            double o[kPer][4];
-            int addr[kPer][4];
-            bool act[kPer];
-#pragma unroll
-            for (int u = 0; u < kPer; u++) {
-                const int w = threadIdx.x + u * NT;
-                act[u] = false;
-                if (w < npair) {
-                    const int P = ut[w] & 0xff, R = ut[w] >> 8;
-                    const double cp = sh_c[P], sp = sh_s[P], cr = sh_c[R], sr = sh_s[R];
-                    act[u] = !(sp == 0.0 && sr == 0.0);
-                    if (act[u]) {
-                        const int p0 = sh_pa[P], p1 = sh_pb[P], r0 = sh_pa[R], r1 = sh_pb[R];
-                        auto ad = [](int i, int j) { return i < j ? i * kLd + j : j * kLd + i; };
-                        addr[u][0] = ad(p0, r0);
-                        addr[u][1] = ad(p0, r1);
-                        addr[u][2] = ad(p1, r0);
-                        addr[u][3] = ad(p1, r1);
-                        rot2x2(cp, sp, cr, sr, S[addr[u][0]], S[addr[u][1]], S[addr[u][2]], S[addr[u][3]], o[u]);
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kPer; u++)
-                if (act[u])
-#pragma unroll
-                    for (int e = 0; e < 4; e++) S[addr[u][e]] = o[u][e];
-            if (group * kSmallRows < m) {   // rows from m on stay zero in these columns
-                const double c = lane < m ? sh_cl[lane] : 1.0, sn = lane < m ? sh_sl[lane] : 0.0;
-                double t[kSmallRows];
-#pragma unroll
-                for (int i = 0; i < kSmallRows; i++) t[i] = __shfl(q[i], pl, MAXN);
-#pragma unroll
-                for (int i = 0; i < kSmallRows; i++) q[i] = fma(c, q[i], sn * t[i]);
-            }
-            __syncthreads();
-        }
-        if (!rotated_any) break;
-        __syncthreads();   // the last step's flag is read before the next sweep's first is written
-    }
-}
-
-// One block (n <= 64) a workgroup.  LDS holds S alone (33 KB; Q lives in registers, M is
+// One block (n <= 64) a workgroup.  LDS holds S alone (34 KB; Q lives in registers, M is
 // formed again at the end), so four workgroups share a CU where
 // S, Q and M in LDS let in one: a bond scan has a thousand such blocks at once.
+// MAXN = 64 takes 256 threads; MAXN = 32 a single wavefront, whose steps have nothing to
+// wait for but their own LDS accesses.
 template <int NT, int MAXN>
 __global__ void __launch_bounds__(NT, NT == 64 ? 3 : 4)
 k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         const double *__restrict__ c, double *__restrict__ x, double *__restrict__ z, double mu0,
         EigBatch eb)
 {
-    constexpr int kLd = MAXN + 1, kWav = NT / 64, kStrips = MAXN / 16 / kWav, kRowB = MAXN / 16;
+    using Shape = JacobiShape<NT, MAXN, false>;
+    constexpr int kLd = Shape::kLd, kWav = NT / 64, kStrips = MAXN / 16 / kWav, kRowB = MAXN / 16;
+    constexpr int kSmallRows = Shape::kQ;
+    static_assert(kSmallRows == 16, "16 rows of Q a thread");
     __shared__ double S[MAXN * kLd];
-    __shared__ double sh_c[MAXN / 2], sh_s[MAXN / 2], sh_cl[MAXN], sh_sl[MAXN], lam[MAXN], red[kWav];
-    __shared__ int sh_pa[MAXN / 2], sh_pb[MAXN / 2], sh_any[2];
-    __shared__ unsigned short ut[(MAXN / 2) * (MAXN / 2 + 1) / 2];
+    __shared__ double lam[MAXN], red[kWav];
+    __shared__ typename Shape::Lds sh;
     const EigBlock B = blocks[blockIdx.x];
     if (eb.active && !eb.active[B.prob]) return;
     const double mu = eb.mus ? eb.mus[B.prob] : mu0;
-    const int n = B.n, m = (n + 1) & ~1, h = m / 2;
+    const int n = B.n, m = (n + 1) & ~1;
     const int64_t o = B.xoff;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
     // this thread's 16 elements: the layout of the MFMA results of the wave's column
@@ -399,8 +372,6 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         S[row_of(e) * kLd + col_of(e)] = v;
         fro += v * v;
     }
-    for (int P = 0, w0 = 0; P < h; w0 += h - P, P++)
-        for (int k = threadIdx.x; k < h - P; k += NT) ut[w0 + k] = (unsigned short)(P | ((P + k) << 8));
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) fro += __shfl_xor(fro, off, 64);
     if (lane == 0) red[wave] = fro;
@@ -412,8 +383,7 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
     double q[kSmallRows];
 #pragma unroll
     for (int i = 0; i < kSmallRows; i++) q[i] = (qr + i == qc) ? 1.0 : 0.0;
-    if (n > 1)
-        small_jacobi<NT, MAXN>(S, q, m, tol, 60, ut, sh_c, sh_s, sh_pa, sh_pb, sh_cl, sh_sl, sh_any);
+    if (n > 1) jacobi<NT, MAXN, false>(S, q, m, tol, 60, sh);
     __syncthreads();
     if (threadIdx.x < MAXN) {
         const double l = S[threadIdx.x * kLd + threadIdx.x];
@@ -577,17 +547,17 @@ __device__ __forceinline__ void ordered_pair(int m, int r, int k, int &a, int &b
     if (a > b) { const int t = a; a = b; b = t; }
 }
 
-template <int NT>
-__global__ void __launch_bounds__(NT)
+template <int NT, bool CROSS>
+__global__ void __launch_bounds__(NT, NT == 256 ? 4 : 1)
 k_pair_eig(const EigBlock *__restrict__ blocks, int round, const double *__restrict__ Aw,
            double *__restrict__ Qbuf, int *__restrict__ active, const double *__restrict__ tol,
-           int *__restrict__ counter, int inner_sweeps, int bip, EigBatch eb)
+           int *__restrict__ counter, int inner_sweeps, EigBatch eb)
 {
+    using Shape = JacobiShape<NT, kP, CROSS>;
+    constexpr int kLd = Shape::kLd, kQ = Shape::kQ;
     __shared__ double S[kP * kLd];
-    __shared__ double sh_c[kP / 2], sh_s[kP / 2];
-    __shared__ int sh_pa[kP / 2], sh_pb[kP / 2], sh_cnt;
-    __shared__ double sh_cl[kP], sh_sl[kP];
-    __shared__ unsigned short ut[kUT];
+    __shared__ typename Shape::Lds sh;
+    __shared__ int sh_big;
     const EigBlock B = blocks[blockIdx.y];
     const int nbk = B.N / 32;
     const int k = blockIdx.x;
@@ -600,20 +570,14 @@ k_pair_eig(const EigBlock *__restrict__ blocks, int round, const double *__restr
     ordered_pair(nbk, round, k, a, b);
     const double *A = Aw + B.woff;
     const double tl = tol[blockIdx.y];
-    if (threadIdx.x == 0) sh_cnt = 0;
-    for (int w = threadIdx.x; w < kUT; w += NT) {
-        int P = 0, rem = w;
-        while (rem >= kP / 2 - P) { rem -= kP / 2 - P; P++; }
-        ut[w] = (unsigned short)(P | ((P + rem) << 8));
-    }
-    __syncthreads();
+    if (threadIdx.x == 0) sh_big = 0;
     int big = 0;
+    // thread (i0, j) loads rows i0, i0 + NT / kP, ... of column j, all
+    // loads in flight at once
+    // the upper triangle of the pair matrix is all that is used: its
+    // (b, a) sub-block is stale in A and is not loaded
+    const int j = threadIdx.x & (kP - 1), i0 = threadIdx.x / kP;
     {
-        // thread (i0, j) loads rows i0, i0 + NT / kP, ... of column j, all
-        // loads in flight at once
-        // the upper triangle of the pair matrix is all pair_jacobi reads: its
-        // (b, a) sub-block is stale in A and is not loaded
-        const int j = threadIdx.x & (kP - 1), i0 = threadIdx.x / kP;
         const int64_t colj = pair_index(a, b, j);
         double v[kP * kP / NT];
 #pragma unroll
@@ -628,27 +592,46 @@ k_pair_eig(const EigBlock *__restrict__ blocks, int round, const double *__restr
             big |= (i < j && fabs(v[u]) > tl);
         }
     }
-    if (big) atomicOr(&sh_cnt, 1);
     __syncthreads();
-    const int any_big = sh_cnt;  // uniform across the workgroup
-    __syncthreads();             // every thread has read sh_cnt before it is reused
-    if (any_big == 0) {          // already diagonal to tolerance: identity rotation
+    if (big) sh_big = 1;
+    __syncthreads();
+    if (!sh_big) {   // uniform; already diagonal to tolerance: identity rotation
         if (threadIdx.x == 0) active[B.poff + k] = 0;
         return;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int kRowsPerWave = PairShape<NT>::kRowsPerWave;
-    double q[kRowsPerWave];
+    const int lane = threadIdx.x & 63, qw = ((int)threadIdx.x - Shape::kQ0) >> 6;
+    double q[kQ];
 #pragma unroll
-    for (int i = 0; i < kRowsPerWave; i++) q[i] = (wave * kRowsPerWave + i == lane) ? 1.0 : 0.0;
-    const int rot = pair_jacobi<NT>(S, q, tl, inner_sweeps, ut, &sh_cnt, sh_c, sh_s, sh_pa, sh_pb,
-                                    sh_cl, sh_sl, bip);
-    double *Qo = Qbuf + B.qoff + (int64_t)k * kP * kP;
-#pragma unroll
-    for (int i = 0; i < kRowsPerWave; i++) Qo[(wave * kRowsPerWave + i) * kP + lane] = q[i];
+    for (int i = 0; i < kQ; i++) {
+        // cross order: lane = row, entry i a column; cyclic: lane = column, entry i a row
+        const int other = CROSS ? (i < kQ / 2 ? qw * (kQ / 2) + i : 32 + qw * (kQ / 2) + i - kQ / 2) : qw * kQ + i;
+        q[i] = other == lane ? 1.0 : 0.0;
+    }
+    const bool rot = jacobi<NT, kP, CROSS>(S, q, kP, tl, inner_sweeps, sh);
     if (threadIdx.x == 0) {
-        active[B.poff + k] = rot > 0;
-        if (rot > 0) atomicAdd(counter, 1);
+        active[B.poff + k] = rot;
+        if (rot) atomicAdd(counter, 1);
+    }
+    if (!rot) return;
+    double *Qo = Qbuf + B.qoff + (int64_t)k * kP * kP;
+    if (!CROSS) {
+        if (qw >= 0)
+#pragma unroll
+            for (int i = 0; i < kQ; i++) Qo[(qw * kQ + i) * kP + lane] = q[i];
+        return;
+    }
+    // through S, which nothing needs any more, into rows of 512 bytes
+    if (qw >= 0)
+#pragma unroll
+        for (int i = 0; i < kQ / 2; i++) {
+            S[lane * kLd + qw * (kQ / 2) + i] = q[i];
+            S[lane * kLd + 32 + qw * (kQ / 2) + i] = q[kQ / 2 + i];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kP * kP / NT; u++) {
+        const int i = i0 + u * (NT / kP);
+        Qo[i * kP + j] = S[i * kLd + j];
     }
 }
 
@@ -911,12 +894,10 @@ void eig_pairs(const EigBlock *blocks, int nblocks, int maxpairs, int round, con
                double *Qbuf, int *active, const double *tol, int *counter, int inner_sweeps,
                int wide, int bip, hipStream_t st, EigBatch eb)
 {
-    if (wide)
-        hipLaunchKernelGGL(k_pair_eig<1024>, dim3(maxpairs, nblocks), dim3(1024), 0, st, blocks, round,
-                           Aw, Qbuf, active, tol, counter, inner_sweeps, bip, eb);
-    else
-        hipLaunchKernelGGL(k_pair_eig<256>, dim3(maxpairs, nblocks), dim3(256), 0, st, blocks, round,
-                           Aw, Qbuf, active, tol, counter, inner_sweeps, bip, eb);
+    auto *k = wide ? (bip ? k_pair_eig<1024, true> : k_pair_eig<1024, false>)
+                   : (bip ? k_pair_eig<256, true> : k_pair_eig<256, false>);
+    hipLaunchKernelGGL(k, dim3(maxpairs, nblocks), dim3(wide ? 1024 : 256), 0, st, blocks, round, Aw, Qbuf,
+                       active, tol, counter, inner_sweeps, eb);
 }
 
 void eig_apply(const EigBlock *blocks, int nblocks, int64_t maxtiles, int round, double *Aw,
