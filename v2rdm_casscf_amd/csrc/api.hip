@@ -111,7 +111,8 @@ struct v2g_solver {
     std::vector<v2g::EigBlock> small, large;
     int ntiny = 0;   // leading small blocks of n <= kTinyN
     DevBuf<v2g::EigBlock> d_small, d_large;
-    DevBuf<double> Mw, Aw, Tw, Vw, Qbuf, tol, frop;
+    DevBuf<double> Mw, Aw, Tw, Vw, Qbuf, tol, frop, pscale;
+    DevBuf<int> pcols, pcount;   // the columns x is made of (eig_scale)
     DevBuf<int> active, counter;
     DevBuf<v2g::GemmDesc> d_gemm_warm1, d_gemm_warm2, d_gemm_rec;
     int max_nb = 0, max_N = 0;
@@ -317,6 +318,7 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
 
     // eigen-split plan: blocks <= 64 whole in one workgroup, others block Jacobi
     int64_t woff = 0, qoff = 0, poff = 0;
+    int coff = 0;
     for (size_t b = 0; b < L->block_dims.size(); b++) {
         const int n = L->block_dims[b];
         if (n == 0) continue;
@@ -332,6 +334,8 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
         e.woff = woff;
         e.qoff = qoff;
         e.poff = poff;
+        e.coff = coff;
+        coff += e.N;
         const int np = e.N / 64;
         woff += (int64_t)e.N * e.N;
         qoff += (int64_t)np * 64 * 64;
@@ -356,6 +360,9 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
         active.alloc(poff);
         tol.alloc(large.size());
         frop.alloc(64 * large.size());
+        pcols.alloc(coff);
+        pscale.alloc(coff);
+        pcount.alloc(large.size());
         counter.alloc(1);
     }
 }
@@ -753,15 +760,15 @@ void v2g_solver::update_xz(double mu, const double *y, const double *c, double *
             std::vector<v2g::GemmDesc> g1, g2;
             for (const auto &b : large) {
                 g1.push_back({Mw.p + b.woff, Vw.p + b.woff, Tw.p + b.woff, b.N, b.N, b.N, b.N, b.N,
-                              b.N, 0, 0, 0});
+                              b.N, 0, nullptr});
                 g2.push_back({Vw.p + b.woff, Tw.p + b.woff, Aw.p + b.woff, b.N, b.N, b.N, b.N, b.N,
-                              b.N, 1, 0, 1});
+                              b.N, 1, nullptr});
             }
             d_gemm_warm1.upload(g1);
             d_gemm_warm2.upload(g2);
         }
-        v2g::gemm_batched(d_gemm_warm1.p, nl, max_N, max_N, st);
-        v2g::gemm_batched(d_gemm_warm2.p, nl, max_N, max_N, st);
+        v2g::gemm_batched(d_gemm_warm1.p, nl, max_N, max_N, 0, 0, st);
+        v2g::gemm_batched(d_gemm_warm2.p, nl, max_N, max_N, 1, 0, st);
     }
     const int maxsweeps = (!cold && warm_sweep_cap > 0) ? warm_sweep_cap : 40;
     const int inner = (!cold && inner_sweep_cap > 0) ? inner_sweep_cap : v2g::kEigFullInner;
@@ -821,7 +828,7 @@ void v2g_solver::update_xz(double mu, const double *y, const double *c, double *
     last_sweeps = sweeps;
     last_split_capped = !cold && sweeps > 0 && (sweeps >= maxsweeps || inner < v2g::kEigFullInner);
     // x = (V s)(V s)^T with s = sqrt(max(lambda,0)/mu); z = mu x - M
-    v2g::eig_scale(d_large.p, nl, Aw.p, Vw.p, Tw.p, mu, st);
+    v2g::eig_scale(d_large.p, nl, max_N, Aw.p, Vw.p, Tw.p, pcols.p, pscale.p, pcount.p, mu, st);
     // the reconstruction descriptors point into x: built once per x buffer
     // (an upload frees and allocates, which would drain the device every call)
     int maxn = 0;
@@ -829,13 +836,13 @@ void v2g_solver::update_xz(double mu, const double *y, const double *c, double *
     if (rec_x != x || !d_gemm_rec.p) {
         std::vector<v2g::GemmDesc> g3;
         for (const auto &b : large)
-            g3.push_back({Tw.p + b.woff, Tw.p + b.woff, x + b.xoff, b.n, b.n, b.N, b.N, b.N, b.n, 0,
-                          1, 1});
+            g3.push_back({Tw.p + b.woff, Tw.p + b.woff, x + b.xoff, b.n, b.n, b.N, b.N, b.N, b.n, 1,
+                          pcount.p + g3.size()});
         HIPCHK(hipStreamSynchronize(st));
         d_gemm_rec.upload(g3);
         rec_x = x;
     }
-    v2g::gemm_batched(d_gemm_rec.p, nl, maxn, maxn, st);
+    v2g::gemm_batched(d_gemm_rec.p, nl, maxn, maxn, 0, 1, st);
     v2g::eig_z(d_large.p, nl, x, Mw.p, zv, mu, st);
     warm = true;
 }

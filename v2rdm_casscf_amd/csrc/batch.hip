@@ -341,7 +341,8 @@ struct v2g_batch {
     std::vector<v2g::EigBlock> small, large;
     int ntiny = 0;   // leading small blocks of n <= kTinyN
     DevBuf<v2g::EigBlock> d_small, d_large;
-    DevBuf<double> Mw, Aw, Tw, Vw, Qbuf, tol, frop;
+    DevBuf<double> Mw, Aw, Tw, Vw, Qbuf, tol, frop, pscale;
+    DevBuf<int> pcols, pcount;   // the columns x is made of (eig_scale)
     DevBuf<int> active, counter;
     DevBuf<v2g::GemmDesc> d_g1, d_g2, d_g3;
     int max_nb = 0, max_N = 0, max_pairs = 0;
@@ -550,11 +551,14 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
     std::stable_sort(large.begin(), large.end(),
                      [](const v2g::EigBlock &a, const v2g::EigBlock &b) { return a.N > b.N; });
     int64_t woff = 0, qoff = 0, poff = 0;
+    int coff = 0;
     for (auto &e : large) {
         const int npair = e.N / 64;
         e.woff = woff;
         e.qoff = qoff;
         e.poff = poff;
+        e.coff = coff;
+        coff += e.N;
         woff += (int64_t)e.N * e.N;
         qoff += (int64_t)npair * 64 * 64;
         poff += npair;
@@ -576,6 +580,9 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
         active.alloc(poff);
         tol.alloc(large.size());
         frop.alloc(64 * large.size());
+        pcols.alloc(coff);
+        pscale.alloc(coff);
+        pcount.alloc(large.size());
         counter.alloc(1);
         d_g1.alloc(large.size());
         d_g2.alloc(large.size());
@@ -719,9 +726,10 @@ void v2g_batch::update_xz(const std::vector<double> &mu, const std::vector<int> 
     int maxn = 0;
     for (const auto &b : large) {
         if (!act[b.prob]) continue;
-        g1.push_back({Mw.p + b.woff, Vw.p + b.woff, Tw.p + b.woff, b.N, b.N, b.N, b.N, b.N, b.N, 0, 0, 0});
-        g2.push_back({Vw.p + b.woff, Tw.p + b.woff, Aw.p + b.woff, b.N, b.N, b.N, b.N, b.N, b.N, 1, 0, 1});
-        g3.push_back({Tw.p + b.woff, Tw.p + b.woff, x + b.xoff, b.n, b.n, b.N, b.N, b.N, b.n, 0, 1, 1});
+        g1.push_back({Mw.p + b.woff, Vw.p + b.woff, Tw.p + b.woff, b.N, b.N, b.N, b.N, b.N, b.N, 0, nullptr});
+        g2.push_back({Vw.p + b.woff, Tw.p + b.woff, Aw.p + b.woff, b.N, b.N, b.N, b.N, b.N, b.N, 1, nullptr});
+        g3.push_back({Tw.p + b.woff, Tw.p + b.woff, x + b.xoff, b.n, b.n, b.N, b.N, b.N, b.n, 1,
+                      pcount.p + (&b - large.data())});
         maxn = std::max(maxn, b.n);
     }
     if (g1.empty()) return;
@@ -729,8 +737,8 @@ void v2g_batch::update_xz(const std::vector<double> &mu, const std::vector<int> 
     HIPCHK(hipMemcpyAsync(d_g2.p, g2.data(), sizeof(v2g::GemmDesc) * g2.size(), hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(d_g3.p, g3.data(), sizeof(v2g::GemmDesc) * g3.size(), hipMemcpyHostToDevice, st));
     if (!cold) {
-        v2g::gemm_batched(d_g1.p, (int)g1.size(), max_N, max_N, st);
-        v2g::gemm_batched(d_g2.p, (int)g2.size(), max_N, max_N, st);
+        v2g::gemm_batched(d_g1.p, (int)g1.size(), max_N, max_N, 0, 0, st);
+        v2g::gemm_batched(d_g2.p, (int)g2.size(), max_N, max_N, 1, 0, st);
     }
     const int maxsweeps = capped ? 1 : 40;
     const int inner = capped ? 1 : v2g::kEigFullInner;
@@ -747,8 +755,8 @@ void v2g_batch::update_xz(const std::vector<double> &mu, const std::vector<int> 
         HIPCHK(hipStreamSynchronize(st));
         if (cnt == 0) break;
     }
-    v2g::eig_scale(d_large.p, nl, Aw.p, Vw.p, Tw.p, 1.0, st, eb);
-    v2g::gemm_batched(d_g3.p, (int)g3.size(), maxn, maxn, st);
+    v2g::eig_scale(d_large.p, nl, max_N, Aw.p, Vw.p, Tw.p, pcols.p, pscale.p, pcount.p, 1.0, st, eb);
+    v2g::gemm_batched(d_g3.p, (int)g3.size(), maxn, maxn, 0, 1, st);
     v2g::eig_z(d_large.p, nl, x, Mw.p, z, 1.0, st, eb);
     warm = true;
 }

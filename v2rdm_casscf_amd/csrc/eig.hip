@@ -110,7 +110,7 @@ __device__ __forceinline__ void rot2x2(double cp, double sp, double cr, double s
 // holds its next pair (blocks {k - 1, k + 1} of the cyclic order, {k, k + 1} of the cross
 // order), updates it first, and goes on to the rotation, the pair's new diagonal and the
 // publication of (c, s) while the other threads update the other blocks.  One barrier a
-// step.  2 500-wide blocks, 40 pair problems a launch: 58 -> @@ us a launch (1 400 -> @@ ns
+// step.  24 orbitals, blocks up to 1 152: 46 -> 26 us a launch beside the tile updates (1 400 -> about 500 ns
 // a step); every index is computed, not looked up, so the reads of S need not wait.
 //  * S keeps its upper triangle (element (i, j) lives at (min, max)), 66 (MAXN + 2) doubles
 //    a row: the accesses of a step walk diagonals and anti-diagonals, whose strides (67, 65)
@@ -818,19 +818,66 @@ k_apply(const EigBlock *__restrict__ blocks, int round, double *__restrict__ Aw,
         }
     }
 }
-// T[:, j] = V[:, j] sqrt(max(lambda_j, 0) / mu), lambda_j = A[j][j]
+// The columns of V that x is made of, lambda_j = A[j][j] > 0: their indices in order (cols),
+// sqrt(lambda_j / mu) (scale, 0 for the padding) and how many, rounded up to the depth of a
+// GEMM panel (count).  About half of a block's eigenvalues are positive, so the
+// reconstruction has half the work.
 __global__ void __launch_bounds__(kT)
-k_scale_vecs(const EigBlock *__restrict__ blocks, const double *__restrict__ Aw,
-             const double *__restrict__ Vw, double *__restrict__ Tw, double mu0, EigBatch eb)
+k_positive(const EigBlock *__restrict__ blocks, const double *__restrict__ Aw, int *__restrict__ cols,
+           double *__restrict__ scale, int *__restrict__ count, double mu0, EigBatch eb)
 {
-    const EigBlock B = blocks[blockIdx.y];
+    __shared__ int wcnt[kT / 64];
+    const EigBlock B = blocks[blockIdx.x];
     if (eb.active && !eb.active[B.prob]) return;
     const double mu = eb.mus ? eb.mus[B.prob] : mu0;
-    const int64_t NN = (int64_t)B.N * B.N;
-    for (int64_t w = blockIdx.x * (int64_t)kT + threadIdx.x; w < NN; w += (int64_t)gridDim.x * kT) {
-        const int j = (int)(w % B.N);
-        const double l = Aw[B.woff + (int64_t)j * B.N + j];
-        Tw[B.woff + w] = l > 0.0 ? Vw[B.woff + w] * sqrt(l / mu) : 0.0;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int done = 0;
+    for (int j0 = 0; j0 < B.N; j0 += kT) {
+        const int j = j0 + threadIdx.x;
+        const double l = j < B.N ? Aw[B.woff + (int64_t)j * (B.N + 1)] : 0.0;
+        const unsigned long long b = __ballot(l > 0.0);
+        if (lane == 0) wcnt[wave] = __popcll(b);
+        __syncthreads();
+        int pos = done + __popcll(b & ((1ull << lane) - 1));
+        for (int w = 0; w < kT / 64; w++) {
+            if (w < wave) pos += wcnt[w];
+            done += wcnt[w];
+        }
+        if (l > 0.0) {
+            cols[B.coff + pos] = j;
+            scale[B.coff + pos] = sqrt(l / mu);
+        }
+        __syncthreads();
+    }
+    const int padded = (done + kGemmK - 1) / kGemmK * kGemmK;
+    if (done + (int)threadIdx.x < padded) {
+        cols[B.coff + done + threadIdx.x] = 0;
+        scale[B.coff + done + threadIdx.x] = 0.0;
+    }
+    if (threadIdx.x == 0) count[blockIdx.x] = padded;
+}
+
+constexpr int kScaleRows = 8;
+
+// T[:, i] = V[:, cols[i]] scale[i], i < count; kScaleRows rows a workgroup.  H50: 332 us
+// with all columns, the diagonal read again for every entry; below 60 now.
+__global__ void __launch_bounds__(kT)
+k_scale_vecs(const EigBlock *__restrict__ blocks, const double *__restrict__ Vw, const int *__restrict__ cols,
+             const double *__restrict__ scale, const int *__restrict__ count, double *__restrict__ Tw, EigBatch eb)
+{
+    const EigBlock B = blocks[blockIdx.y];
+    const int row0 = blockIdx.x * kScaleRows;
+    if (row0 >= B.N || (eb.active && !eb.active[B.prob])) return;
+    const double *V = Vw + B.woff + (int64_t)row0 * B.N;
+    double *T = Tw + B.woff + (int64_t)row0 * B.N;
+    for (int i = threadIdx.x; i < count[blockIdx.y]; i += kT) {
+        const int j = cols[B.coff + i];
+        const double s = scale[B.coff + i];
+        double v[kScaleRows];
+#pragma unroll
+        for (int r = 0; r < kScaleRows; r++) v[r] = V[(int64_t)r * B.N + j];
+#pragma unroll
+        for (int r = 0; r < kScaleRows; r++) T[(int64_t)r * B.N + i] = s > 0.0 ? v[r] * s : 0.0;
     }
 }
 
@@ -907,10 +954,12 @@ void eig_apply(const EigBlock *blocks, int nblocks, int64_t maxtiles, int round,
                        Vw, Qbuf, active, eb);
 }
 
-void eig_scale(const EigBlock *blocks, int nblocks, const double *Aw, const double *Vw, double *Tw,
-               double mu, hipStream_t st, EigBatch eb)
+void eig_scale(const EigBlock *blocks, int nblocks, int max_N, const double *Aw, const double *Vw, double *Tw,
+               int *cols, double *scale, int *count, double mu, hipStream_t st, EigBatch eb)
 {
-    hipLaunchKernelGGL(k_scale_vecs, dim3(256, nblocks), dim3(kT), 0, st, blocks, Aw, Vw, Tw, mu, eb);
+    hipLaunchKernelGGL(k_positive, dim3(nblocks), dim3(kT), 0, st, blocks, Aw, cols, scale, count, mu, eb);
+    hipLaunchKernelGGL(k_scale_vecs, dim3(max_N / kScaleRows, nblocks), dim3(kT), 0, st, blocks, Vw, cols, scale,
+                       count, Tw, eb);
 }
 
 void eig_z(const EigBlock *blocks, int nblocks, const double *x, const double *Mw, double *z,

@@ -24,7 +24,7 @@ struct EigBlock {
     int64_t qoff;   // offset in the pair-rotation buffer (N/64 pairs of 64 x 64)
     int64_t poff;   // offset in the pair-active flags
     int prob;       // problem of a batch the block belongs to (0 alone)
-    int pad;
+    int coff;       // offset in the per-column arrays (N a block)
 };
 
 // Batched splits: mu of each problem and which problems take part (null: one
@@ -34,14 +34,18 @@ struct EigBatch {
     const int *active = nullptr;
 };
 
+constexpr int kGemmK = 32;   // depth of a GEMM panel
+
+// C = op(A) op(B).  A and B are workspaces of rows padded to 64 entries and 64 rows, 16-byte
+// aligned, and are read tile by tile beyond M and N; K is a multiple of kGemmK
 struct GemmDesc {
     const double *A;
     const double *B;
     double *C;
     int M, N, K;
     int lda, ldb, ldc;
-    int ta, tb;     // 1: use the transpose of A / B
-    int sym;        // 1: C is symmetric (M == N); only upper tiles are computed
+    int sym;              // 1: C is symmetric (M == N); only upper tiles are computed
+    const int *kcount;    // device: the K to use instead (null: K)
 };
 
 // blocks of n <= 64, those with n <= kTinyN first (ntiny of them)
@@ -67,12 +71,15 @@ void eig_pairs(const EigBlock *blocks, int nblocks, int maxpairs, int round, con
                int wide, int bip, hipStream_t st, EigBatch eb = {});
 void eig_apply(const EigBlock *blocks, int nblocks, int64_t maxtiles, int round, double *Aw,
                double *Vw, const double *Qbuf, const int *active, hipStream_t st, EigBatch eb = {});
-void eig_scale(const EigBlock *blocks, int nblocks, const double *Aw, const double *Vw, double *Tw,
-               double mu, hipStream_t st, EigBatch eb = {});
+// T = the columns of V with a positive eigenvalue, scaled to x = T T^T, side by side;
+// count[b]: how many (a multiple of kGemmK, zeros beyond the last)
+void eig_scale(const EigBlock *blocks, int nblocks, int max_N, const double *Aw, const double *Vw, double *Tw,
+               int *cols, double *scale, int *count, double mu, hipStream_t st, EigBatch eb = {});
 void eig_z(const EigBlock *blocks, int nblocks, const double *x, const double *Mw, double *z,
            double mu, hipStream_t st, EigBatch eb = {});
 
-// C = op(A) op(B) for every descriptor (beta = 0); grid sized for the largest
-void gemm_batched(const GemmDesc *descs, int ndesc, int max_m, int max_n, hipStream_t st);
+// C = op(A) op(B) for every descriptor (ta, tb: transposes of all of them); grid sized for
+// the largest
+void gemm_batched(const GemmDesc *descs, int ndesc, int max_m, int max_n, int ta, int tb, hipStream_t st);
 
 }  // namespace v2g
