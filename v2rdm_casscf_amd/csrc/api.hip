@@ -24,6 +24,7 @@
 #include "layout.hpp"
 #include "mlp.hpp"
 #include "redcg.hpp"
+#include "t2maps.hpp"
 #include "spatial.hpp"
 
 #include <random>
@@ -91,6 +92,7 @@ struct v2g_solver {
     // CG: the reduced form of the plain solve (redcg.hpp) and the general form
     // (preconditioned, flexible, layouts with second-pass rows) work in one slab
     v2g::RedCG redcg;
+    v2g::T2Maps t2maps;
     DevBuf<double> cgmem;
     DevBuf<double> t, partial, scal, jacobi, user_minv, rowpart;
     bool have_jacobi = false, have_user = false;
@@ -206,11 +208,15 @@ struct v2g_solver {
         const int64_t n = (L->ncon + 31) / 32 * 32;
         return {cgmem.p, cgmem.p + n, cgmem.p + 2 * n, t.p, partial.p, scal.p, rowpart.p};
     }
-    // fused iterations: rowpart holds x_tiles squares of A^T p, then three
-    // arrays of row_tiles residual partials (the unfused p.Ap partials use the
-    // first row_tiles)
+    // fused iterations: rowpart holds x_parts() squares of A^T p, then three
+    // arrays of row_parts() residual partials (the unfused p.Ap partials use the
+    // first row_parts())
     bool fused_cg() const { return V2G_CG_FUSE && plan.t2_tiles == 0 && plan.x_tiles > 0; }
-    int64_t rowpart_len() const { return std::max<int64_t>(1, plan.x_tiles + 3 * plan.row_tiles); }
+    int64_t rowpart_len() const
+    {
+        return std::max<int64_t>(1, plan.x_parts() + 3 * plan.row_parts());
+    }
+    int64_t all_x_tiles = 0;   // of every primal segment, those of t2maps too
     // general = true: the final residual stays in own_cg_bufs().r
     int cg(const double *rhs, double *y, double tol, int maxiter, int precond, int flexible,
            double *res, bool general = false);
@@ -257,6 +263,7 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
     // G2 row segments get a slice of the precomputed column table (aux)
     std::vector<v2g::Segment> rsegs = L->rowsegs;
     int64_t g2rows = 0;
+    for (int hh = 0; hh < L->nirrep; hh++) plan.tiled = plan.tiled || L->gems_ab[hh] >= v2g::rows::kTileDim;
     for (auto &s : rsegs) {
         const bool g2 = s.kind == v2g::RF_G2AB || s.kind == v2g::RF_G2AA;
         s.aux = g2 && !s.wave ? g2rows : -1;
@@ -267,18 +274,33 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
     plan.rowsegs = d_rowsegs.p;
     plan.row_tile_start = d_rowtiles.p;
     plan.nrowsegs = (int)L->rowsegs.size();
-    plan.x_tiles = tiles(L->xsegs, ts);
-    d_xsegs.upload(L->xsegs);
+    // T2 rows: t2maps takes them and, in A^T, the D2 and D1 entries
+    std::vector<v2g::Segment> xs = L->xsegs, x2 = L->xsegs_t2;
+    all_x_tiles = tiles(xs, ts);
+    if (L->opt.t2) {
+        auto drop = [](std::vector<v2g::Segment> &v, std::initializer_list<int> kinds) {
+            v.erase(std::remove_if(v.begin(), v.end(), [&](const v2g::Segment &s) {
+                return std::find(kinds.begin(), kinds.end(), s.kind) != kinds.end(); }), v.end());
+        };
+        drop(xs, {v2g::XS_D2AB, v2g::XS_D2AA, v2g::XS_D1});
+        drop(x2, {v2g::RF_T2AAB, v2g::RF_T2BIG});
+        t2maps.build(*L, d_lay.p);
+        plan.t2maps = &t2maps;
+        for (const auto &s : L->rowsegs)
+            if (s.kind == v2g::RF_T2AAB || s.kind == v2g::RF_T2BIG) plan.row_tiles_t2 += v2g::tiles_for(s);
+    }
+    plan.x_tiles = tiles(xs, ts);
+    d_xsegs.upload(xs);
     d_xtiles.upload(ts);
     plan.xsegs = d_xsegs.p;
     plan.x_tile_start = d_xtiles.p;
-    plan.nxsegs = (int)L->xsegs.size();
-    plan.t2_tiles = tiles(L->xsegs_t2, ts);
-    d_t2segs.upload(L->xsegs_t2);
+    plan.nxsegs = (int)xs.size();
+    plan.t2_tiles = tiles(x2, ts);
+    d_t2segs.upload(x2);
     d_t2tiles.upload(ts);
     plan.t2segs = d_t2segs.p;
     plan.t2_tile_start = d_t2tiles.p;
-    plan.nt2segs = (int)L->xsegs_t2.size();
+    plan.nt2segs = (int)x2.size();
     // the D1a / D1b blocks must form one range of x that no other block
     // enters, and every column must fit 30 bits, for the packed G2 table
     int64_t d1lo = INT64_MAX, d1hi = -1;
@@ -682,47 +704,50 @@ int v2g_solver::cg_with(const CgBufs &B, bool graphs, const double *rhs, double 
     v2g::cg_init(n, rhs, B.Ap, B.r, B.p, minv, nullptr, B.partial, B.scal, tolv, maxiter, st);
     // one chunk of kCgChunk (even) iterations; every kernel argument is fixed,
     // the iteration number and the done flags live in scal
-    auto enqueue_chunk = [&]() {
+    auto enqueue = [&](int iterations) {
         const bool fused = fused_cg();
-        for (int c = 0; c < kCgChunk; c++) {
+        for (int c = 0; c < iterations; c++) {
             const int par = c & 1;
             const double *done = B.scal + v2g::CG_DONE0 + par;
             if (fused) {
                 // t = A^T p with the tile squares -> alpha; r -= alpha A t in
                 // the A.x launch (A p is never stored) with the r.z, r.r
                 // partials; then y, the test and p as below
-                double *stepp = B.rowpart + plan.x_tiles;
+                double *stepp = B.rowpart + plan.x_parts();
                 v2g::launch_atu(plan, B.p, B.t, st, done, B.rowpart);
-                v2g::cg_alpha_from_tiles(plan.x_tiles, B.rowpart, B.scal, par, st);
+                v2g::cg_alpha_from_tiles(plan.x_parts(), B.rowpart, B.scal, par, st);
                 v2g::CgFuse fz;
                 fz.r = B.r;
                 fz.minv = minv;
                 fz.scal = B.scal;
                 fz.part = stepp;
-                fz.ntiles = plan.row_tiles;
+                fz.ntiles = plan.row_parts();
                 v2g::launch_au(plan, B.t, nullptr, st, done, nullptr, nullptr, fz);
-                v2g::cg_step_from_tiles(plan.row_tiles, stepp, B.partial, B.scal, par, st);
+                v2g::cg_step_from_tiles(plan.row_parts(), stepp, B.partial, B.scal, par, st);
             } else {
                 v2g::launch_atu(plan, B.p, B.t, st, done);
                 v2g::launch_au(plan, B.t, B.Ap, st, done, B.p, B.rowpart);   // Ap and p.Ap
-                v2g::cg_dot_from_rows(plan.row_tiles, B.rowpart, B.partial, B.scal, par, st);
+                v2g::cg_dot_from_rows(plan.row_parts(), B.rowpart, B.partial, B.scal, par, st);
                 v2g::cg_step(n, B.r, B.Ap, minv, B.partial, B.scal, par, st);
             }
             v2g::cg_finish_iter(n, y, B.r, B.p, minv, B.partial, B.scal, par, flexible, st);
         }
     };
     hipGraphExec_t exec = nullptr;
-    if (graphs && n <= kGraphMaxRows) exec = cg_graph(y, minv, flexible ? 1 : 0, enqueue_chunk);
+    if (graphs && n <= kGraphMaxRows && maxiter >= kCgChunk)
+        exec = cg_graph(y, minv, flexible ? 1 : 0, [&] { enqueue(kCgChunk); });
     double hs[v2g::CG_NSLOTS];
     int it = 0;
     for (;;) {
-        if (exec) HIPCHK(hipGraphLaunch(exec, st));
-        else enqueue_chunk();
-        it += kCgChunk;
+        // none beyond maxiter, to an even number
+        const int k = std::max(2, (std::min(kCgChunk, maxiter - it) + 1) / 2 * 2);
+        if (exec && k == kCgChunk) HIPCHK(hipGraphLaunch(exec, st));
+        else enqueue(k);
+        it += k;
         HIPCHK(hipMemcpyAsync(hs, B.scal, sizeof(hs), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         if (hs[v2g::CG_DONE0 + (it & 1)] != 0.0) break;
-        if (it > maxiter + 2 * kCgChunk) break;  // defensive: cannot happen
+        if (it - 2 * kCgChunk > maxiter) break;  // defensive: cannot happen
     }
     if (res) *res = hs[v2g::CG_NRM];
     last_cg_nrm0 = hs[v2g::CG_NRM0];
@@ -977,8 +1002,11 @@ int v2g_cg_solve_noalloc(v2g_handle h, const double *rhs, double *y, double tol,
     // boundary
     auto up = [](int64_t n) { return (n + 31) / 32 * 32; };
     const int64_t ncon = h->L->ncon, dimx = h->L->dimx;
+    // (a plan with more partial sums than tiles keeps them in the handle's own array, so
+    // what fits does not depend on how the rows are dealt out)
+    const int64_t tiles = std::max<int64_t>(1, h->all_x_tiles + 3 * h->plan.row_tiles);
     const int64_t need = 3 * up(ncon) + up(dimx) + up(v2g::kPartialArrays * v2g::kRedBlocks) +
-                         up(v2g::CG_NSLOTS) + up(h->rowpart_len());
+                         up(v2g::CG_NSLOTS) + up(tiles);
     if (need > (int64_t)kScratchDoubles)
         throw std::invalid_argument("problem too large for the allocation-free CG: needs " +
                                     std::to_string(need) + " doubles of scratch, at most " +
@@ -998,7 +1026,7 @@ int v2g_cg_solve_noalloc(v2g_handle h, const double *rhs, double *y, double tol,
     B.t = B.Ap + up(ncon);
     B.partial = B.t + up(dimx);
     B.scal = B.partial + up(v2g::kPartialArrays * v2g::kRedBlocks);
-    B.rowpart = B.scal + up(v2g::CG_NSLOTS);
+    B.rowpart = h->rowpart_len() <= tiles ? B.scal + up(v2g::CG_NSLOTS) : h->rowpart.p;
     const double *minv = precond == 2 ? h->user_minv.p : nullptr;
     const int it = h->cg_with(B, false, rhs, y, tol, maxiter, minv, flexible, resnorm);
     if (iters) *iters = it;

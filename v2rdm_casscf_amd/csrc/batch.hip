@@ -392,6 +392,8 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
             return (const int *)tables.back()->p;
         };
         // block and row offsets of this problem, shifted to its place in the batch
+        for (int hh = 0; hh < L[q]->nirrep; hh++)
+            plan.tiled = plan.tiled || L[q]->gems_ab[hh] >= v2g::rows::kTileDim;
         const v2g::DevLayout dl = v2g::make_dev_layout(
             Lq, {up(Lq.sym), up(Lq.gab), up(Lq.gaa), up(Lq.bab), up(Lq.baa), up(Lq.baab),
                  up(Lq.baba), up(Lq.baaa), up(Lq.b00)},

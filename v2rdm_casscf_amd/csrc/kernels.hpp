@@ -11,6 +11,8 @@
 
 namespace v2g {
 
+class T2Maps;
+
 struct MapPlan {
     const DevLayout *dlay = nullptr;
     const Segment *rowsegs = nullptr;
@@ -31,6 +33,13 @@ struct MapPlan {
     // dlay holds one layout per problem (Segment::prob picks it); the done flag
     // of problem p is done[p * done_stride] (0: one flag for the whole plan)
     int done_stride = 0;
+    bool tiled = false;   // some G2 block is visited by tiles (rowterms.hpp, kTileDim)
+    // the T2 rows and the D2 / D1 entries of A^T they enter (null: with the other rows, and
+    // xsegs / t2segs hold them); the last row_tiles_t2 tiles of rowsegs are these rows'
+    const T2Maps *t2maps = nullptr;
+    int64_t row_tiles_t2 = 0;
+    int64_t row_parts() const;   // partial sums of launch_au
+    int64_t x_parts() const;     // of launch_atu
 };
 
 int64_t tiles_for(const Segment &s);
@@ -42,7 +51,7 @@ void build_g2_index(const MapPlan &p, const std::vector<Segment> &rowsegs, int64
 // The residual update of a CG iteration fused into A.x (r is set): A.x is not
 // stored; r -= alpha (A.x) with alpha = scal[CG_ALPHA], and part[k ntiles +
 // tile] (k = 0, 1, 2) receives the tile's sums of r.z, r.r and r_old.z of the
-// new residual, z = minv r (minv null: z = r); ntiles = the plan's row_tiles
+// new residual, z = minv r (minv null: z = r); ntiles = the plan's row_parts()
 struct CgFuse {
     double *r = nullptr;
     const double *minv = nullptr;
@@ -51,12 +60,12 @@ struct CgFuse {
     int64_t ntiles = 0;
 };
 
-// dotv / rowpart (optional): rowpart[tile] = sum over the tile's rows of dotv . Ax
+// dotv / rowpart (optional): row_parts() partial sums of dotv . Ax
 void launch_au(const MapPlan &p, const double *x, double *Ax, hipStream_t st,
                const double *done = nullptr, const double *dotv = nullptr,
                double *rowpart = nullptr, CgFuse fz = {});
-// sqpart (optional, layouts without second-pass rows only): sqpart[tile] =
-// the tile's sum of squares of A^T.y (x_tiles entries)
+// sqpart (optional, plans without second-pass rows only): x_parts() partial sums of the
+// squares of A^T.y
 void launch_atu(const MapPlan &p, const double *y, double *ATy, hipStream_t st,
                 const double *done = nullptr, double *sqpart = nullptr);
 void launch_row_norm2(const MapPlan &p, double *d, hipStream_t st);

@@ -30,6 +30,7 @@
 #include "devlayout.hpp"
 #include "kernels.hpp"
 #include "rowterms.hpp"
+#include "t2maps.hpp"
 
 namespace v2g {
 
@@ -160,6 +161,7 @@ k_g2_index(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs, i
 
 // fz.r (optional): the CG residual update fused in, r -= alpha (A.x) with the
 // tile sums of the new residual's dot products instead of A.x itself
+template <bool TILED>
 __global__ void __launch_bounds__(kBlock, V2G_AU_WAVES_PER_EU)
 k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
      const int64_t *__restrict__ tile_start, int nseg, const double *__restrict__ x,
@@ -213,7 +215,7 @@ k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
             row[u] = -1;
             if (pos < sg.count) {
                 ci[u] = g2idx[sg.aux + pos];
-                row[u] = row_of(L, sg, pos);
+                row[u] = row_of<TILED>(L, sg, pos);
             }
         }
 #pragma unroll
@@ -240,7 +242,7 @@ k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
         for (int u = 0; u < kPerThread; u++) {
             const int64_t pos = t * kElemTile + u * kBlock + threadIdx.x;
             Gather f{x, 0.0};
-            row[u] = pos < sg.count ? row_of(L, sg, pos) : -1;
+            row[u] = pos < sg.count ? row_of<TILED>(L, sg, pos) : -1;
             if (row[u] >= 0) elem_terms(L, sg, row[u], f);
             v[u] = f.acc;
         }
@@ -394,10 +396,12 @@ k_atu_t2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
 void launch_au(const MapPlan &p, const double *x, double *Ax, hipStream_t st, const double *done,
                const double *dotv, double *rowpart, CgFuse fz)
 {
-    if (p.row_tiles > 0)
-        hipLaunchKernelGGL(k_au, dim3((unsigned)p.row_tiles), dim3(kBlock), 0, st, p.dlay,
+    const int64_t tiles = p.row_tiles - p.row_tiles_t2;
+    if (tiles > 0)
+        hipLaunchKernelGGL(p.tiled ? k_au<true> : k_au<false>, dim3((unsigned)tiles), dim3(kBlock), 0, st, p.dlay,
                            p.rowsegs, p.row_tile_start, p.nrowsegs, x, Ax, done, dotv, rowpart,
                            p.g2idx, p.done_stride, fz);
+    if (p.t2maps) p.t2maps->au(x, Ax, done, dotv, rowpart ? rowpart + tiles : nullptr, fz, tiles, st);
 }
 
 void build_g2_index(const MapPlan &p, const std::vector<Segment> &rowsegs, int64_t d1lo,
@@ -430,10 +434,14 @@ void launch_atu(const MapPlan &p, const double *y, double *ATy, hipStream_t st, 
         hipLaunchKernelGGL(k_atu, dim3((unsigned)chunk_grid(p.x_tiles)), dim3(kBlock), 0, st, p.dlay,
                            p.xsegs, p.x_tile_start, p.nxsegs, y, ATy, done, p.x_tiles, p.done_stride,
                            sqpart);
+    if (p.t2maps) p.t2maps->atu(y, ATy, done, sqpart ? sqpart + p.x_tiles : nullptr, st);
     if (p.t2_tiles > 0)
         hipLaunchKernelGGL(k_atu_t2, dim3((unsigned)p.t2_tiles), dim3(kBlock), 0, st, p.dlay,
                            p.t2segs, p.t2_tile_start, p.nt2segs, y, ATy, done, p.done_stride);
 }
+
+int64_t MapPlan::row_parts() const { return row_tiles - row_tiles_t2 + (t2maps ? t2maps->au_blocks() : 0); }
+int64_t MapPlan::x_parts() const { return x_tiles + (t2maps ? t2maps->atu_blocks() : 0); }
 
 int64_t tiles_for(const Segment &s)
 {
