@@ -119,14 +119,15 @@ __device__ __forceinline__ void rot2x2(double cp, double sp, double cr, double s
 //    partner column is fetched by lane shuffles.  Cross order: a lane holds one row, its
 //    wave the columns of a few slots, rotated in place; then the second half's columns
 //    move on by one slot (a register move; one column a wave goes through LDS).
-// NT = 1024: S in the first eight waves, Q in the other eight: where a launch has a few
-// hundred pair problems.  NT = 256 does the same work in fewer instructions, for many small
-// problems at once (bond scans).
+// From NT = 8 MAXN on, S lies with the first half of the waves and Q with the other: where a
+// launch has a few hundred problems.  256 threads for 64 indices do the same work in fewer
+// instructions, for many small problems at once (bond scans).
 template <int NT, int MAXN, bool CROSS> struct JacobiShape {
     static constexpr int kH = MAXN / 2, kLd = MAXN + 2;
-    static constexpr int kST = NT == 1024 ? NT / 2 : NT;               // threads of S: the first
+    static constexpr bool kSplit = NT >= 8 * MAXN;
+    static constexpr int kST = kSplit ? NT / 2 : NT;                   // threads of S: the first
     static constexpr int kU = (kH * (kH - 3) / 2 + kH + kST - 1) / kST;   // blocks of S a thread
-    static constexpr int kQ0 = NT == 1024 ? NT / 2 : 0, kQT = NT - kQ0;   // threads of Q
+    static constexpr int kQ0 = kSplit ? NT / 2 : 0, kQT = NT - kQ0;       // threads of Q
     static constexpr int kQ = MAXN * MAXN / kQT;                       // entries of Q a thread
     static constexpr int kXw = CROSS ? kQT / 64 : 0;
     static_assert(!CROSS || MAXN == 64, "the cross order is for 64 indices");
@@ -211,7 +212,7 @@ __device__ __forceinline__ bool jacobi(double *S, double (&q)[JacobiShape<NT, MA
     if (tid < 64) {
         const int p = min(l1, l2), r = max(l1, l2);
         publish(0, S[p * kLd + p], S[r * kLd + r], S[p * kLd + r]);
-        if (NT > 64) __builtin_amdgcn_s_setprio(3);
+        __builtin_amdgcn_s_setprio(3);
     }
     // Q: cyclic order: this lane's column and its distance from the step number
     const int qlane = tid % MAXN, qwave = (tid - Sh::kQ0) / 64;
@@ -326,25 +327,23 @@ __device__ __forceinline__ bool jacobi(double *S, double (&q)[JacobiShape<NT, MA
         if (ofQ && !first_step)
             q[kQ - 1] = sh.xch[((buf ^ 1) * Sh::kXw + (qwave + 1) % Sh::kXw) * 64 + (tid & 63)];
     }
-    if (NT > 64 && tid < 64) __builtin_amdgcn_s_setprio(0);
+    if (tid < 64) __builtin_amdgcn_s_setprio(0);
     return total;
 }
 
 // One block (n <= 64) a workgroup.  LDS holds S alone (34 KB; Q lives in registers, M is
 // formed again at the end), so four workgroups share a CU where
 // S, Q and M in LDS let in one: a bond scan has a thousand such blocks at once.
-// MAXN = 64 takes 256 threads; MAXN = 32 a single wavefront, whose steps have nothing to
-// wait for but their own LDS accesses.
 template <int NT, int MAXN>
-__global__ void __launch_bounds__(NT, NT == 64 ? 3 : 4)
+__global__ void __launch_bounds__(NT, 4)   // waves a SIMD
 k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         const double *__restrict__ c, double *__restrict__ x, double *__restrict__ z, double mu0,
         EigBatch eb)
 {
     using Shape = JacobiShape<NT, MAXN, false>;
-    constexpr int kLd = Shape::kLd, kWav = NT / 64, kStrips = MAXN / 16 / kWav, kRowB = MAXN / 16;
-    constexpr int kSmallRows = Shape::kQ;
-    static_assert(kSmallRows == 16, "16 rows of Q a thread");
+    // 16-column strips of the matrix go to the first waves, kEl elements a thread
+    constexpr int kLd = Shape::kLd, kWav = NT / 64, kRowB = MAXN / 16, kSw = kWav < kRowB ? kWav : kRowB;
+    constexpr int kStrips = kRowB / kSw, kEl = 4 * kRowB * kStrips, kSmallRows = Shape::kQ;
     __shared__ double S[MAXN * kLd];
     __shared__ double lam[MAXN], red[kWav];
     __shared__ typename Shape::Lds sh;
@@ -354,9 +353,8 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
     const int n = B.n, m = (n + 1) & ~1;
     const int64_t o = B.xoff;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
-    // this thread's 16 elements: the layout of the MFMA results of the wave's column
+    // this thread's elements: the layout of the MFMA results of the wave's column
     // strips (row 16 b + 4 r + lk, column 16 strip + li)
-    static_assert(kStrips * kRowB * 4 == 16, "16 elements a thread");
     auto row_of = [&](int e) { return 16 * (e / 4 % kRowB) + 4 * (e & 3) + lk; };
     auto col_of = [&](int e) { return 16 * (wave * kStrips + e / (4 * kRowB)) + li; };
     auto element = [&](int e) -> double {
@@ -366,12 +364,13 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         return 0.5 * ((aty[ipq] - c[ipq] + mu * x[ipq]) + (aty[iqp] - c[iqp] + mu * x[iqp]));
     };
     double fro = 0.0;
+    if (wave < kSw)
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const double v = element(e);
-        S[row_of(e) * kLd + col_of(e)] = v;
-        fro += v * v;
-    }
+        for (int e = 0; e < kEl; e++) {
+            const double v = element(e);
+            S[row_of(e) * kLd + col_of(e)] = v;
+            fro += v * v;
+        }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) fro += __shfl_xor(fro, off, 64);
     if (lane == 0) red[wave] = fro;
@@ -379,7 +378,8 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
     double tot = 0.0;
     for (int i = 0; i < kWav; i++) tot += red[i];
     const double tol = 1e-15 * sqrt(tot) + 1e-300;
-    const int qc = threadIdx.x % MAXN, qr = threadIdx.x / MAXN * kSmallRows;
+    const bool ofQ = (int)threadIdx.x >= Shape::kQ0;
+    const int qc = threadIdx.x % MAXN, qr = ((int)threadIdx.x - Shape::kQ0) / MAXN * kSmallRows;
     double q[kSmallRows];
 #pragma unroll
     for (int i = 0; i < kSmallRows; i++) q[i] = (qr + i == qc) ? 1.0 : 0.0;
@@ -390,13 +390,16 @@ k_small(const EigBlock *__restrict__ blocks, const double *__restrict__ aty,
         lam[threadIdx.x] = threadIdx.x < m && l > 0.0 ? l / mu : 0.0;
     }
     __syncthreads();   // the diagonal has been read: S takes Q
+    if (ofQ)
 #pragma unroll
-    for (int i = 0; i < kSmallRows; i++) S[(qr + i) * kLd + qc] = q[i];
-    // M once more, before x is overwritten: 16 registers held through the solve would spill
-    double Mv[16];
+        for (int i = 0; i < kSmallRows; i++) S[(qr + i) * kLd + qc] = q[i];
+    // M once more, before x is overwritten: the registers held through the solve would spill
+    double Mv[kEl];
+    if (wave < kSw)
 #pragma unroll
-    for (int e = 0; e < 16; e++) Mv[e] = element(e);
+        for (int e = 0; e < kEl; e++) Mv[e] = element(e);
     __syncthreads();
+    if (wave >= kSw) return;
     // x = Q diag(lam) Q^T, one or two 16-column strips a wave
 #pragma unroll
     for (int st = 0; st < kStrips; st++) {
@@ -898,6 +901,15 @@ k_z(const EigBlock *__restrict__ blocks, const double *__restrict__ x,
 
 }  // namespace
 
+namespace {
+// Blocks of 33 to 64 that the chip holds at once with 1024 threads each, two a CU: up to
+// there a launch waits for one block's latency (about 400 blocks of 64 chains: 715 against
+// 786 us), beyond for the throughput, which 256 threads have (about 800: 1295 against 1055
+// us).  Blocks up to 32 take 256 threads at any count (128 chains: 201 against 328 us with a
+// wavefront each).
+constexpr int kFewMid = 512;
+}
+
 int eig_order_small(std::vector<EigBlock> &small)
 {
     std::stable_sort(small.begin(), small.end(), [](const EigBlock &a, const EigBlock &b) {
@@ -912,12 +924,12 @@ int eig_order_small(std::vector<EigBlock> &small)
 void eig_small(const EigBlock *blocks, int nblocks, int ntiny, const double *aty, const double *c, double *x,
                double *z, double mu, hipStream_t st, EigBatch eb)
 {
-    // blocks[0 .. ntiny) have n <= 32: a wavefront each; the others 256 threads
+    const int nmid = nblocks - ntiny;
     if (ntiny > 0)
-        hipLaunchKernelGGL((k_small<64, 32>), dim3(ntiny), dim3(64), 0, st, blocks, aty, c, x, z, mu, eb);
-    if (nblocks > ntiny)
-        hipLaunchKernelGGL((k_small<256, 64>), dim3(nblocks - ntiny), dim3(256), 0, st, blocks + ntiny, aty,
-                           c, x, z, mu, eb);
+        hipLaunchKernelGGL((k_small<256, 32>), dim3(ntiny), dim3(256), 0, st, blocks, aty, c, x, z, mu, eb);
+    if (nmid > 0)
+        hipLaunchKernelGGL((nmid <= kFewMid ? k_small<1024, 64> : k_small<256, 64>), dim3(nmid),
+                           dim3(nmid <= kFewMid ? 1024 : 256), 0, st, blocks + ntiny, aty, c, x, z, mu, eb);
 }
 
 void eig_build_m(const EigBlock *blocks, int nblocks, int max_N, const double *aty, const double *c,
