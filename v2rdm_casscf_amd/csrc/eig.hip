@@ -47,16 +47,10 @@ __device__ __forceinline__ void circle_pair(int m, int r, int k, int &a, int &b)
 // root: the textbook t = sgn(th) / (|th| + sqrt(th^2 + 1)), th = d / e with
 // d = aqq - app, e = 2 apq, multiplied through by |e|, gives
 // t = sgn(d) e / (|d| + sqrt(d^2 + e^2)); c = 1 / sqrt(1 + t^2), s = t c.
-// Both roots and the quotient come from the hardware estimates (better than 2^-20) and
-// one third-order step each, which leaves the rounding of its own last operation: a
-// step of the pair problems waits for this chain, and the library's root and
-// division are about twice as long.
-__device__ __forceinline__ double rsqrt_refined(double x)   // 1 / sqrt(x), x normal and finite
-{
-    const double y = __builtin_amdgcn_rsq(x), e = fma(-(x * y), y, 1.0);
-    return fma(y * e, fma(0.375, e, 0.5), y);
-}
-
+// A step of the pair problems waits for this chain.  The root and the quotient are the
+// hardware estimates (better than 2^-20), one third-order step and one correction by the
+// residual each, which rounds as the library's do but without their scaling for the ends
+// of the range (those take the library's); c is the estimate and two Newton steps.
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double &c,
                                                 double &s)
 {
@@ -64,15 +58,31 @@ __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double a
     const double h = fma(d, d, e * e);
     double t;
     if (h > 1e-280 && h < 1e280) {
-        const double den = fabs(d) + h * rsqrt_refined(h);
-        const double y = __builtin_amdgcn_rcp(den), f = fma(-den, y, 1.0);
-        t = (d >= 0.0 ? e : -e) * fma(y, fma(f, f, f), y);
-    } else {   // d^2 + e^2 leaves the range: the textbook form
-        const double th = d / e;
-        t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
+        double y = __builtin_amdgcn_rsq(h);
+        const double f = fma(-(h * y), y, 1.0);
+        y = fma(y * f, fma(0.375, f, 0.5), y);
+        const double r0 = h * y, r = fma(fma(-r0, r0, h), 0.5 * y, r0);
+        const double den = fabs(d) + r, num = d >= 0.0 ? e : -e;
+        double w = __builtin_amdgcn_rcp(den);
+        const double g = fma(-den, w, 1.0);
+        w = fma(w, fma(g, g, g), w);
+        const double q = num * w;
+        t = fma(fma(-den, q, num), w, q);
+    } else {
+        const double r = sqrt(h);
+        if (r > 0.0 && r <= 1.79e308) {
+            t = (d >= 0.0 ? e : -e) / (fabs(d) + r);
+        } else {   // d^2 + e^2 under- or overflows: the textbook form
+            const double th = d / e;
+            t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(fma(th, th, 1.0)));
+        }
     }
-    c = rsqrt_refined(fma(t, t, 1.0));
-    s = t * c;
+    const double x = fma(t, t, 1.0), hx = 0.5 * x;
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(y, fma(-hx * y, y, 0.5), y);
+    y = fma(y, fma(-hx * y, y, 0.5), y);
+    c = y;
+    s = t * y;
 }
 
 // R_P^T B R_R for one 2 x 2 block B = [b00 b01; b10 b11] with R = [c s; -s c]
