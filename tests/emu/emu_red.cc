@@ -72,6 +72,7 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
     RedLayout R;
     RedWork W;
     if (!make_red_layout(L, Lo, R, W)) return -1;
+    R.rowtab = W.rowtab.data();
     if (ncon != L.ncon) return -3;
     g_viol = 0;
     const View rhs{rhs_, ncon}, y{y_, ncon};
@@ -118,7 +119,7 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
         };
         each_entry([&](const AbEntry &a) {
             const SelfAb<std::decay_t<decltype(x)>> o(R, a, x);
-            auto one = [&](int f, double dx, double pm) { visit(R.soff[f] + a.pos, self_row_ab(Lo, f, a), dx, pm); };
+            auto one = [&](int f, double dx, double pm) { visit(R.soff[f] + a.pos, self_row_ab(R, f, a), dx, pm); };
             if (R.L.q2) one(SF_Q2AB, o.q2, 0.0);
             if (R.L.g2) {
                 one(SF_G2AB, o.g1, 0.0);
@@ -173,7 +174,7 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
             }
         for (char c : seen) if (c != 1) g_viol++;
     };
-    each_entry([&](const AbEntry &a) { t.at(a.pos) = full_at_ab(Lo, a, y); },
+    each_entry([&](const AbEntry &a) { t.at(a.pos) = full_at_ab(R, Lo, a, y); },
                [&](int sp, const AbEntry &a, int, int64_t k) { t.at(R.nAB + sp * R.nAA + k) = full_at_aa(Lo, sp, a, y); },
                [&](const Segment &sg, int64_t i) { t.at(sg.start + i) = wave([&](int l) { return atu_d1_wave(Lo, sg, i, l, y); }); });
     // s = rhs - y - B2 t + P y_ms on the self rows, r on the explicit ones
@@ -209,7 +210,7 @@ int emu_red_cg(int nirrep, const int *amopi, int na, int nb, int mult, int q2, i
                     const int64_t k = R.aa0[sg.h] + i, word = sg.aux + i / 64;
                     const uint64_t m = (uint64_t)1 << (i % 64);
                     const bool shares = W.bits.at((size_t)word) & m;
-                    if (shares != cell_shares(a)) g_viol++;
+                    if (shares != (a.p == a.r || a.p == a.s || a.q == a.r || a.q == a.s)) g_viol++;
                     double pr[3] = {0.0, 0.0, 0.0};
                     for (int j = 0; R.cells && j < 3; j++) pr[j] = p[j * R.nAA + k];
                     Cell tc = cell_at(R.L.q2, R.L.g2, R.nblk_d, R.cells, d, load_cell(R, a.pos, sg.count, k, g),

@@ -107,12 +107,14 @@ __device__ __forceinline__ Place place(const RedProb *prob, const int *blk)
 template <class F>
 __device__ __forceinline__ void for_tiles(const Place &pl, int k, F fn)
 {
-    // the lists lead with latency-bound items and end with the cells' streams: every
-    // other workgroup goes through its tiles backwards, so that a CU has both at a time
+    // an iteration's lists lead with latency-bound items and end with the cells' streams:
+    // every other workgroup goes through its tiles backwards, so that a CU has both at a
+    // time.  The start list's tiles share lines of rhs and y with their neighbours: all go
+    // forwards (H50, the four passes 1.17 -> 1.11 ms)
     const int nt = pl.pr->ntile[k], mine = pl.lb < nt ? (nt - 1 - pl.lb) / pl.nb + 1 : 0;
     const RedTile *tiles = pl.pr->tile[k];
     for (int m = 0; m < mine; m++) {
-        const RedTile &tl = tiles[pl.lb + (pl.lb & 1 ? mine - 1 - m : m) * pl.nb];
+        const RedTile &tl = tiles[pl.lb + (pl.lb & 1 && k > 0 ? mine - 1 - m : m) * pl.nb];
         const Segment &sg = tl.sg;
         if (sg.wave == 0) {
             const int64_t i = tl.first + threadIdx.x;
@@ -293,6 +295,11 @@ __device__ __forceinline__ Eval evaluate(const RedBufs &B, const Place &pl, cons
 }
 
 // ---- start of a solve -------------------------------------------------------
+// These passes and the last one, k_red_y, meet the full rows of rhs and y, where the rows of
+// neighbouring entries lie apart: lines that several wavefronts touch bound them (H50: 258, 345,
+// 150 and 357 us; 349, 394, 179 and 445 with the rows' places from the geminal tables).  The
+// entries by blocks of 8 x 8 orbitals, or an entry's rows all loaded before the first
+// store, change nothing.
 
 // t = (A^T y)_D from the full rows; u, v, w, p, mu, nu, om = 0 and the scalars
 __global__ void __launch_bounds__(kNT, 4)
@@ -314,7 +321,7 @@ k_red_aty(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
     for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
         if (is_ab(sg)) {
             AbEntry a;
-            if (start_entry(R, sg, i, a)) V.t[a.pos] = full_at_ab(Lo, a, y);
+            if (start_entry(R, sg, i, a)) V.t[a.pos] = full_at_ab(R, Lo, a, y);
         } else if (sg.kind == RK_AA) {
             const AbEntry a = cell_entry(R, sg.h, i);
             for (int sp = 0; sp < 2; sp++) V.t[R.nAB + sp * R.nAA + sg.start + i] = full_at_aa(Lo, sp, a, y);
@@ -361,7 +368,7 @@ __device__ __forceinline__ void self_slots(const RedLayout &R, const DevLayout &
     if (is_ab(sg)) {
         AbEntry a;
         if (!start_entry(R, sg, i, a)) return;
-        auto one = [&](int f, double o) { fn(R.soff[f] + a.pos, self_row_ab(Lo, f, a), o); };
+        auto one = [&](int f, double o) { fn(R.soff[f] + a.pos, self_row_ab(R, f, a), o); };
         const SelfAb<X> o(R, a, x);
         if (R.L.q2) one(SF_Q2AB, o.q2);
         if (R.L.g2) {
@@ -450,7 +457,7 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
             double v = lane < R.lanes ? ms_row_gram(R, sg.sub, (int)i, lane, ms) : 0.0;
             for (int j = lane; j < R.L.amo; j += 64) {
                 const AbEntry a{sg.sub ? l : j, sg.sub ? j : k, sg.sub ? j : l, sg.sub ? k : j, 0};
-                v -= y[self_row_ab(Lo, SF_G2BA, a)];
+                v -= y[self_row_ab(R, SF_G2BA, a)];
             }
             v = wave_sum(v);
             if (lane == 0) row(sg.start + i, sg.aux + i, v);
@@ -855,7 +862,8 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     std::vector<CellRec> cell;
     std::vector<uint64_t> bits;
     std::vector<uint32_t> rank;
-    std::vector<size_t> to(4 * np_), ao(np_), co(np_), bo(np_);
+    std::vector<int32_t> rowtab;
+    std::vector<size_t> to(4 * np_), ao(np_), co(np_), bo(np_), ro(np_);
     for (int q = 0; q < np_; q++) {
         tiles[q] = 1;
         for (int k = 0; k < 4; k++) {
@@ -872,6 +880,8 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
         ao[q] = ab.size();
         co[q] = cell.size();
         bo[q] = bits.size();
+        ro[q] = rowtab.size();
+        rowtab.insert(rowtab.end(), work[q].rowtab.begin(), work[q].rowtab.end());
         bits.insert(bits.end(), work[q].bits.begin(), work[q].bits.end());
         rank.insert(rank.end(), work[q].rank.begin(), work[q].rank.end());
         ab.insert(ab.end(), work[q].ab.begin(), work[q].ab.end());
@@ -890,8 +900,9 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     // one allocation, regions on 256-byte boundaries
     auto room = [](size_t n) { return (n + 255) / 256 * 256; };
     const size_t tb = sizeof(RedTile) * tl.size(), abb = sizeof(AbRec) * ab.size(),
-                 cb = sizeof(CellRec) * cell.size(), bb = sizeof(uint64_t) * bits.size(), rb = sizeof(uint32_t) * rank.size();
-    HIPCHK(hipMalloc(&d_work_, room(tb) + room(abb) + room(cb) + room(bb) + room(rb)));
+                 cb = sizeof(CellRec) * cell.size(), bb = sizeof(uint64_t) * bits.size(), rb = sizeof(uint32_t) * rank.size(),
+                 wb = sizeof(int32_t) * rowtab.size();
+    HIPCHK(hipMalloc(&d_work_, room(tb) + room(abb) + room(cb) + room(bb) + room(rb) + room(wb)));
     char *at = static_cast<char *>(d_work_);
     auto put = [&](const void *src, size_t n) {
         char *p = at;
@@ -904,7 +915,9 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     const CellRec *dc = reinterpret_cast<const CellRec *>(put(cell.data(), cb));
     const uint64_t *db = reinterpret_cast<const uint64_t *>(put(bits.data(), bb));
     const uint32_t *dr = reinterpret_cast<const uint32_t *>(put(rank.data(), rb));
+    const int32_t *dw = reinterpret_cast<const int32_t *>(put(rowtab.data(), wb));
     for (int q = 0; q < np_; q++) {
+        prob[q].R.rowtab = dw + ro[q];
         for (int k = 0; k < 4; k++) prob[q].tile[k] = dt + to[4 * q + k];
         prob[q].ab = da + ao[q];
         prob[q].cell = dc + co[q];

@@ -33,11 +33,12 @@ struct RedWork {
     std::vector<CellRec> cell;
     std::vector<uint64_t> bits;             // one a cell, set for those with a CellRec; every
                                             // irrep starts on a word (Segment::aux of RK_CELLS)
+    std::vector<int32_t> rowtab;            // RedLayout::rowtab
     std::vector<uint32_t> rank;             // CellRecs before each word's first
 };
 
 // false: the layout has rows the reduced form does not cover (T1, T2,
-// spin-adapted Q2 / G2).  dev: the layout's device view (tables of either side)
+// spin-adapted Q2 / G2), or sizes beyond its 32-bit places.  R.rowtab is left to the caller.  dev: the layout's device view (tables of either side)
 bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWork &w);
 
 #if defined(__HIPCC__)

@@ -134,6 +134,28 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
         n += (size_t)__builtin_popcountll(w.bits[i]);
     }
 
+    // the places of the full layout's rows
+    const int amo = Lt.amo;
+    w.rowtab.assign((size_t)RT_COUNT * amo * amo, 0);
+    for (int x = 0; x < amo; x++)
+        for (int y = 0; y < amo; y++) {
+            const int h = Lt.sym[x] ^ Lt.sym[y];
+            const int64_t n = Lt.gab[x * amo + y], g = Lt.gems_ab[h];
+            auto put = [&](int tab, int64_t row, int64_t len, int64_t i) {
+                if (row < 0) return true;
+                const int64_t v = row + i * len;
+                w.rowtab[((size_t)tab * amo + x) * amo + y] = (int32_t)v;
+                return v <= INT32_MAX - 2 * g;
+            };
+            const auto &ro = dev.rowoff;
+            if (!put(RT_AB, 0, 1, n) || !put(RT_GG, 0, 1, g + n) || !put(RT_Q2, ro[RF_Q2AB][0][h], g, n) ||
+                !put(RT_G2AB, ro[RF_G2AB][0][h], g, n) || !put(RT_G2BA, ro[RF_G2AB][1][h], g, n) ||
+                !put(RT_GA, ro[RF_G2AA][0][h], 2 * g, n) || !put(RT_GB, ro[RF_G2AA][0][h], 2 * g, g + n) ||
+                !put(RT_D0, ro[Lt.singlet ? RF_SPIN_D200 : RF_SPIN_D200_4][0][h], Lt.singlet ? g : 2 * g, n) ||
+                !put(RT_D1, ro[RF_SPIN_D200_4][0][h], 2 * g, g + n))
+                return false;
+        }
+
     // passes: the long rows first, so that no workgroup is left with one at the end
     auto cat = [](std::vector<Segment> &a, const std::vector<Segment> &b) { a.insert(a.end(), b.begin(), b.end()); };
     std::vector<Segment> ms;

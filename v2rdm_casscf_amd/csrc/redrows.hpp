@@ -61,6 +61,17 @@ struct RedLayout {
     int nM;          // maximal-spin rows (2 gems_ab[0], or 0)
     int lanes;       // threads that share a row summed over the orbitals: 16, 32 or 64
     int nblk_d;      // D200 quadrants: 0 (spin off), 1 (singlet), 4
+    const int32_t *rowtab;   // RT_COUNT tables of amo^2 entries (RowTab)
+};
+
+// A row of the full layout is the sum of two entries, by the row pair and by the column
+// pair: the first with the block's offset and row length worked in.  (From the geminal
+// numbers, with the irreps' offsets and lengths to look up as well, the start and the end of a
+// solve spent 120 loads on an entry's 14 rows.)
+enum RowTab : int {
+    RT_AB,                 // column: the pair's number
+    RT_GG,                 // column: behind the first half
+    RT_Q2, RT_G2AB, RT_G2BA, RT_GA, RT_GB, RT_D0, RT_D1, RT_COUNT   // rows
 };
 
 // a D2ab entry outside the cells (p == q or r == s): where everything lies that its rows read, -1 never occurs (the
@@ -92,6 +103,11 @@ namespace rows {
 struct AbEntry {
     int p, q, r, s;
     int64_t pos;
+    // of an entry inside a cell (cc = 0: outside): the cell's first entry, cells of the
+    // irrep, orientation, place among the cells
+    int64_t base = 0, cc = 0;
+    int o = 0;
+    int64_t k = 0;
 };
 
 V2G_HD inline int64_t ab_pos(const RedLayout &R, int p, int q, int r, int s)
@@ -112,11 +128,6 @@ V2G_HD inline int64_t aa_pos(const RedLayout &R, int p, int q, int r, int s)
     return R.aa0[h] + (int64_t)L.gaa[p * L.amo + q] * L.gems_aa[h] + L.gaa[r * L.amo + s];
 }
 
-V2G_HD inline AbEntry ab_entry(const RedLayout &R, int p, int q, int r, int s)
-{
-    return {p, q, r, s, ab_pos(R, p, q, r, s)};
-}
-
 // the pairs p > q, r > s of cell c of irrep h
 V2G_HD inline AbEntry cell_entry(const RedLayout &R, int h, int64_t c)
 {
@@ -124,24 +135,34 @@ V2G_HD inline AbEntry cell_entry(const RedLayout &R, int h, int64_t c)
     int I, K;
     split_index(c, L.gems_aa[h], I, K);
     const int b = L.baa[L.baa_off[h] + I], k = L.baa[L.baa_off[h] + K];
-    return {P0(b), P1(b), P0(k), P1(k), R.ab0[h] + c};
+    const int64_t pos = R.ab0[h] + c;
+    return {P0(b), P1(b), P0(k), P1(k), pos, pos, (int64_t)L.gems_aa[h] * L.gems_aa[h], 0, R.aa0[h] + c};
 }
 
-V2G_HD inline bool cell_shares(const AbEntry &a)
-{
-    return a.p == a.r || a.p == a.s || a.q == a.r || a.q == a.s;
-}
-
-// entry number i (0 .. 4 gems_aa^2) of irrep h in position order
+// entry number i (0 .. 4 gems_aa^2) of irrep h: by the bra pair in one order, then in the
+// other, with both orders of the ket pair after each bra: together they touch whole lines of the
+// rows, one order alone the r > s part of each
 V2G_HD inline AbEntry cell_ab(const RedLayout &R, int h, int64_t i)
 {
-    const int64_t cc = (int64_t)R.L.gems_aa[h] * R.L.gems_aa[h];
-    const int o = (int)(i / cc);
-    AbEntry a = cell_entry(R, h, i - o * cc);
+    const DevLayout &L = R.L;
+    const int64_t ga = L.gems_aa[h], cc = ga * ga;
+    const int o1 = i >= 2 * cc ? 1 : 0;
+    int I, K;
+    split_index(i - o1 * 2 * cc, 2 * ga, I, K);
+    const int o = o1 + (K >= ga ? 2 : 0);
+    AbEntry a = cell_entry(R, h, I * ga + (K >= ga ? K - ga : K));
     if (o & 1) { const int t = a.p; a.p = a.q; a.q = t; }
     if (o & 2) { const int t = a.r; a.r = a.s; a.s = t; }
     a.pos += o * cc;
+    a.o = o;
     return a;
+}
+
+// position of the entry with the bra pair (x & 1), the ket pair (x & 2) exchanged
+V2G_HD inline int64_t exchanged(const RedLayout &R, const AbEntry &a, int x)
+{
+    if (a.cc) return a.base + (a.o ^ x) * a.cc;
+    return ab_pos(R, x & 1 ? a.q : a.p, x & 1 ? a.p : a.q, x & 2 ? a.s : a.r, x & 2 ? a.r : a.s);
 }
 
 // entry number i (0 .. 2 amo gems_ab[0]) of those with p == q or r == s; false: none
@@ -196,7 +217,7 @@ struct SelfAb {
         g1 = g2 = -x;
         ga = gb = 0.0;
         if (L.g2 && a.p != a.q && a.r != a.s) {
-            const int64_t k = R.nAB + aa_pos(R, a.p, a.q, a.r, a.s);
+            const int64_t k = R.nAB + a.k;
             const double sg = ((a.p < a.q) == (a.r < a.s)) ? -1.0 : 1.0;
             ga = sg * v[k];
             gb = sg * v[k + R.nAA];
@@ -224,9 +245,9 @@ struct D200Ab {
     V2G_HD inline D200Ab(const RedLayout &R, const AbEntry &a, const X &v)
     {
         v0 = v[a.pos];
-        v1 = v[ab_pos(R, a.q, a.p, a.r, a.s)];
-        v2 = v[ab_pos(R, a.p, a.q, a.s, a.r)];
-        v3 = v[ab_pos(R, a.q, a.p, a.s, a.r)];
+        v1 = v[exchanged(R, a, 1)];
+        v2 = v[exchanged(R, a, 2)];
+        v3 = v[exchanged(R, a, 3)];
     }
     V2G_HD inline double row(const RedLayout &R, const AbEntry &a, int blk) const
     {
@@ -307,8 +328,7 @@ V2G_HD inline double self_at_ab(const RedLayout &R, const AbEntry &a, const S &s
         t += (s[R.soff[SF_G2X] + a.pos] + s[R.soff[SF_G2Y] + a.pos]) -
              (s[R.soff[SF_G2AB] + a.pos] + s[R.soff[SF_G2BA] + a.pos]);
     if (R.nblk_d) {
-        const int64_t p1 = ab_pos(R, a.q, a.p, a.r, a.s), p2 = ab_pos(R, a.p, a.q, a.s, a.r),
-                      p3 = ab_pos(R, a.q, a.p, a.s, a.r);
+        const int64_t p1 = exchanged(R, a, 1), p2 = exchanged(R, a, 2), p3 = exchanged(R, a, 3);
         for (int k = 0; k < R.nblk_d; k++) {
             double c[4];
             d200_coef(k, L.singlet, a.p == a.q, a.r == a.s, c);
@@ -434,46 +454,26 @@ V2G_HD inline double long_row(const RedLayout &R, const Segment &sg, int64_t ite
 }
 
 // ---- rows of the full layout -------------------------------------------------
-// the row of the full layout Lo that family f's slot of an aligned entry stands for
-V2G_HD inline int64_t self_row_ab(const DevLayout &Lo, int f, const AbEntry &a)
+V2G_HD inline int64_t row_tab(const RedLayout &R, int tab, int x, int y)
 {
-    const int amo = Lo.amo;
-    const int *gab = Lo.gab, *sym = Lo.sym;
+    return R.rowtab[(tab * R.L.amo + x) * R.L.amo + y];
+}
+
+// the row of the full layout that family f's slot of an aligned entry stands for
+V2G_HD inline int64_t self_row_ab(const RedLayout &R, int f, const AbEntry &a)
+{
     const int p = a.p, q = a.q, r = a.r, s = a.s;
-    auto GAB = [&](int x, int y) -> int64_t { return gab[x * amo + y]; };
     switch (f) {
-    case SF_Q2AB: {
-        const int h = sym[p] ^ sym[q];
-        return Lo.rowoff[RF_Q2AB][0][h] + GAB(p, q) * Lo.gems_ab[h] + GAB(r, s);
-    }
-    case SF_G2AB: {
-        const int h = sym[p] ^ sym[s];
-        return Lo.rowoff[RF_G2AB][0][h] + GAB(p, s) * Lo.gems_ab[h] + GAB(r, q);
-    }
-    case SF_G2BA: {
-        const int h = sym[q] ^ sym[r];
-        return Lo.rowoff[RF_G2AB][1][h] + GAB(q, r) * Lo.gems_ab[h] + GAB(s, p);
-    }
-    case SF_G2X: {
-        const int h = sym[p] ^ sym[r];
-        const int64_t g = Lo.gems_ab[h];
-        return Lo.rowoff[RF_G2AA][0][h] + GAB(p, r) * 2 * g + g + GAB(s, q);
-    }
-    case SF_G2Y: {
-        const int h = sym[q] ^ sym[s];
-        const int64_t g = Lo.gems_ab[h];
-        return Lo.rowoff[RF_G2AA][0][h] + (g + GAB(q, s)) * 2 * g + GAB(r, p);
-    }
-    case SF_G2A: case SF_G2B: {
-        const int h = sym[p] ^ sym[s];
-        const int64_t g = Lo.gems_ab[h], b = f == SF_G2B ? g : 0;
-        return Lo.rowoff[RF_G2AA][0][h] + (b + GAB(p, s)) * 2 * g + b + GAB(r, q);
-    }
+    case SF_Q2AB: return row_tab(R, RT_Q2, p, q) + row_tab(R, RT_AB, r, s);
+    case SF_G2AB: return row_tab(R, RT_G2AB, p, s) + row_tab(R, RT_AB, r, q);
+    case SF_G2BA: return row_tab(R, RT_G2BA, q, r) + row_tab(R, RT_AB, s, p);
+    case SF_G2X: return row_tab(R, RT_GA, p, r) + row_tab(R, RT_GG, s, q);
+    case SF_G2Y: return row_tab(R, RT_GB, q, s) + row_tab(R, RT_AB, r, p);
+    case SF_G2A: return row_tab(R, RT_GA, p, s) + row_tab(R, RT_AB, r, q);
+    case SF_G2B: return row_tab(R, RT_GB, p, s) + row_tab(R, RT_GG, r, q);
     default: {
-        const int h = sym[p] ^ sym[q], k = f - SF_D0;
-        const int64_t g = Lo.gems_ab[h];
-        if (Lo.singlet) return Lo.rowoff[RF_SPIN_D200][0][h] + GAB(p, q) * g + GAB(r, s);
-        return Lo.rowoff[RF_SPIN_D200_4][0][h] + (GAB(p, q) + (k >> 1) * g) * 2 * g + GAB(r, s) + (k & 1) * g;
+        const int k = f - SF_D0;
+        return row_tab(R, k & 2 ? RT_D1 : RT_D0, p, q) + row_tab(R, k & 1 ? RT_GG : RT_AB, r, s);
     }
     }
 }
@@ -486,13 +486,40 @@ V2G_HD inline int64_t self_row_d1(const DevLayout &Lo, int sp, int h, int64_t it
 }
 
 // A^T y on entry a of the D2ab blocks / the cell a of the D2aa, D2bb blocks, from full rows
+// (y's rows of the full layout Lo)
 template <class Y>
-V2G_HD inline double full_at_ab(const DevLayout &Lo, const AbEntry &a, const Y &y)
+V2G_HD inline double full_at_ab(const RedLayout &R, const DevLayout &Lo, const AbEntry &a, const Y &y)
 {
-    Segment sg{};
-    sg.h = Lo.sym[a.p] ^ Lo.sym[a.q];
-    sg.dim = Lo.gems_ab[sg.h];
-    return atu_d2ab(Lo, sg, (int64_t)Lo.gab[a.p * Lo.amo + a.q] * sg.dim + Lo.gab[a.r * Lo.amo + a.s], y);
+    const int p = a.p, q = a.q, r = a.r, s = a.s;
+    double t = 0.0;
+    if (p == r && q == s) t += Lo.sz ? y[Lo.rowoff[RF_TRACE][0][0]] : 2.0 * y[Lo.rowoff[RF_TRACE][3][0]];
+    if (q == s) {   // D2ab -> D1a
+        const int h = Lo.sym[p], n = Lo.amopi[h];
+        t -= y[Lo.rowoff[RF_CONTR][Lo.sz ? 0 : 4][h] + (p - Lo.poff[h]) * n + (r - Lo.poff[h])];
+    }
+    if (p == r) {   // D2ab -> D1b
+        const int h = Lo.sym[q], n = Lo.amopi[h];
+        t -= y[Lo.rowoff[RF_CONTR][Lo.sz ? 1 : 5][h] + (q - Lo.poff[h]) * n + (s - Lo.poff[h])];
+    }
+    if (Lo.spin && p == s && q == r) t += y[Lo.rowoff[RF_S2][0][0]];
+    if (R.cells && a.cc) {
+        const int h = Lo.sym[p] ^ Lo.sym[q];
+        const int64_t k = a.k - R.aa0[h];
+        const double an = 0.5 * (y[Lo.rowoff[RF_SPIN_ANTI][0][h] + k] + y[Lo.rowoff[RF_SPIN_ANTI][1][h] + k]);
+        t += (p > q) == (r > s) ? -an : an;
+    }
+    for (int b = 0; b < R.nblk_d; b++) {
+        double c[4];
+        d200_coef(b, Lo.singlet, p == q, r == s, c);
+        const int tr = b & 2 ? RT_D1 : RT_D0, tc = b & 1 ? RT_GG : RT_AB;
+        const int64_t pq = row_tab(R, tr, p, q), qp = row_tab(R, tr, q, p), rs = row_tab(R, tc, r, s),
+                      sr = row_tab(R, tc, s, r);
+        t += c[0] * y[pq + rs] + c[1] * y[qp + rs] + c[2] * y[pq + sr] + c[3] * y[qp + sr];
+    }
+    auto row = [&](int f) { return y[self_row_ab(R, f, a)]; };
+    if (Lo.q2) t += row(SF_Q2AB);
+    if (Lo.g2) t += (row(SF_G2X) + row(SF_G2Y)) - (row(SF_G2AB) + row(SF_G2BA));
+    return t;
 }
 
 template <class Y>
