@@ -133,7 +133,8 @@ struct v2g_solver {
     int nlanes = 1;
     int lane_off[kMaxLanes] = {}, lane_n[kMaxLanes] = {}, lane_pairs[kMaxLanes] = {},
         lane_nb[kMaxLanes] = {};
-    int64_t lane_tiles[kMaxLanes] = {};
+    v2g::EigTiles lane_tiles[kMaxLanes];
+    DevBuf<int64_t> d_tilestart;   // their prefix sums, lane after lane
     hipStream_t lane_st[kMaxLanes] = {};
     hipEvent_t ev_fork = nullptr, ev_start[kMaxLanes] = {}, ev_join[kMaxLanes] = {};
     std::vector<v2g::EigBlock> large_nat;   // the large blocks in dimensions_ order
@@ -416,7 +417,6 @@ void v2g_solver::configure_lanes(int want)
         lane_off[l] = (int)large.size();
         lane_n[l] = l < nlanes ? (int)g[l].size() : 0;
         lane_pairs[l] = lane_nb[l] = 0;
-        lane_tiles[l] = 0;
         if (l < nlanes) large.insert(large.end(), g[l].begin(), g[l].end());
         if (l < nlanes && nlanes > 1) {
             if (l > 0 && !lane_st[l]) HIPCHK(hipStreamCreateWithFlags(&lane_st[l], hipStreamNonBlocking));
@@ -430,8 +430,13 @@ void v2g_solver::configure_lanes(int want)
             const int np = large[i].N / 64;
             lane_pairs[l] = std::max(lane_pairs[l], np);
             lane_nb[l] = std::max(lane_nb[l], large[i].N / 32);
-            lane_tiles[l] = std::max(lane_tiles[l], (int64_t)np * (np + 1) / 2 + (int64_t)np * np);
         }
+    std::vector<int64_t> ts;
+    for (int l = 0; l < kMaxLanes; l++) {
+        lane_tiles[l] = v2g::EigTiles(large.data() + lane_off[l], lane_n[l]);
+        ts.insert(ts.end(), lane_tiles[l].start.begin(), lane_tiles[l].start.end());
+    }
+    d_tilestart.upload(ts);
     d_large.upload(large.empty() ? std::vector<v2g::EigBlock>{} : large);
     // descriptors of the warm-start products follow the block order
     d_gemm_warm1.alloc(0);
@@ -815,7 +820,8 @@ void v2g_solver::update_xz(double mu, const double *y, const double *c, double *
                 // (every pair is still visited once per sweep): always in a
                 // split that must converge, by option in a capped tracking sweep
                 const int bip = ((capped ? cross_order : 1) && rnd > 0) ? 1 : 0;
-                v2g::eig_pairs(bl, lane_n[l], lane_pairs[l], rnd, Aw.p, Qbuf.p, active.p,
+                const int nb = lane_tiles[l].blocks(rnd);   // the larger blocks' rounds go on longest
+                v2g::eig_pairs(bl, nb, lane_pairs[l], rnd, Aw.p, Qbuf.p, active.p,
                                tol.p + lane_off[l], counter.p, inner, pair_wide ? 1 : 0, bip, s);
                 if (rnd == 0 && l % 2 == 0 && l + 1 < nlanes) {
                     // lane l + 1 starts once lane l's first pair problems are
@@ -824,7 +830,8 @@ void v2g_solver::update_xz(double mu, const double *y, const double *c, double *
                     HIPCHK(hipEventRecord(ev_start[l], s));
                     HIPCHK(hipStreamWaitEvent(lane_st[l + 1], ev_start[l], 0));
                 }
-                v2g::eig_apply(bl, lane_n[l], lane_tiles[l], rnd, Aw.p, Vw.p, Qbuf.p, active.p, s);
+                v2g::eig_apply(bl, nb, d_tilestart.p + lane_off[l] + l, lane_tiles[l].start[nb], rnd, Aw.p,
+                               Vw.p, Qbuf.p, active.p, s);
             }
         for (int l = 1; l < nlanes; l++) {
             HIPCHK(hipEventRecord(ev_join[l], lane_st[l]));

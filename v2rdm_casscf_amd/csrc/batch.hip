@@ -346,7 +346,8 @@ struct v2g_batch {
     DevBuf<int> active, counter;
     DevBuf<v2g::GemmDesc> d_g1, d_g2, d_g3;
     int max_nb = 0, max_N = 0, max_pairs = 0;
-    int64_t max_tiles = 0;
+    v2g::EigTiles eigtiles;          // of the large blocks, and their prefix sums
+    DevBuf<int64_t> d_tilestart;
     bool warm = false, pair_wide = false;
     const double *rec_x = nullptr;
     // CG iterations as a captured graph (fixed arguments: y and the buffers)
@@ -567,12 +568,13 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
         max_nb = std::max(max_nb, e.N / 32);
         max_N = std::max(max_N, e.N);
         max_pairs = std::max(max_pairs, npair);
-        max_tiles = std::max(max_tiles, (int64_t)npair * (npair + 1) / 2 + (int64_t)npair * npair);
     }
     pair_wide = max_N >= 512;
     ntiny = v2g::eig_order_small(small);
     d_small.upload(small);
     d_large.upload(large);
+    eigtiles = v2g::EigTiles(large.data(), (int)large.size());
+    d_tilestart.upload(eigtiles.start);
     if (!large.empty()) {
         Mw.alloc(woff);
         Aw.alloc(woff);
@@ -748,9 +750,11 @@ void v2g_batch::update_xz(const std::vector<double> &mu, const std::vector<int> 
         HIPCHK(hipMemsetAsync(counter.p, 0, sizeof(int), st));
         for (int rnd = 0; rnd < max_nb - 1; rnd++) {
             const int bip = ((capped ? cross_order : 1) && rnd > 0) ? 1 : 0;
-            v2g::eig_pairs(d_large.p, nl, max_pairs, rnd, Aw.p, Qbuf.p, active.p, tol.p, counter.p,
+            const int nb = eigtiles.blocks(rnd);
+            v2g::eig_pairs(d_large.p, nb, max_pairs, rnd, Aw.p, Qbuf.p, active.p, tol.p, counter.p,
                            inner, pair_wide ? 1 : 0, bip, st, eb);
-            v2g::eig_apply(d_large.p, nl, max_tiles, rnd, Aw.p, Vw.p, Qbuf.p, active.p, st, eb);
+            v2g::eig_apply(d_large.p, nb, d_tilestart.p, eigtiles.start[nb], rnd, Aw.p, Vw.p, Qbuf.p, active.p, st,
+                           eb);
         }
         int cnt = 0;
         HIPCHK(hipMemcpyAsync(&cnt, counter.p, sizeof(int), hipMemcpyDeviceToHost, st));

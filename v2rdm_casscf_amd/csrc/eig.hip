@@ -655,21 +655,27 @@ k_pair_eig(const EigBlock *__restrict__ blocks, int round, const double *__restr
 // v_mfma_f64_16x16x4f64: A[i][k] from lane i + 16k, B[k][j] from lane
 // j + 16k, D[i][j] in lane j + 16 (i % 4), element i / 4.
 __global__ void __launch_bounds__(kT, 4)
-k_apply(const EigBlock *__restrict__ blocks, int round, double *__restrict__ Aw,
-        double *__restrict__ Vw, const double *__restrict__ Qbuf, const int *__restrict__ active,
-        EigBatch eb)
+k_apply(const EigBlock *__restrict__ blocks, int nblocks, const int64_t *__restrict__ tile_start, int round,
+        double *__restrict__ Aw, double *__restrict__ Vw, const double *__restrict__ Qbuf,
+        const int *__restrict__ active, EigBatch eb)
 {
     // only the tile lives in LDS; the pair rotations Q_P, Q_R are read from
     // global memory (L2-resident: each one serves a row of tiles), which
     // halves the LDS footprint and doubles the workgroups per CU
     __shared__ double T[kP * kLd];
-    const EigBlock B = blocks[blockIdx.y];
+    // the tiles of all blocks in one line: a grid of the largest block's by the number of
+    // blocks is three quarters empty workgroups at H50
+    int lo = 0, hi = nblocks;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (tile_start[mid] <= (int64_t)blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    const EigBlock B = blocks[lo];
     const int nbk = B.N / 32, np = nbk / 2;
-    if (round >= nbk - 1) return;
     if (eb.active && !eb.active[B.prob]) return;
-    const int64_t ntA = (int64_t)np * (np + 1) / 2, ntV = (int64_t)(B.N / kP) * np;
-    const int64_t t = blockIdx.x;
-    if (t >= ntA + ntV) return;
+    const int64_t ntA = (int64_t)np * (np + 1) / 2;
+    const int64_t t = (int64_t)blockIdx.x - tile_start[lo];
     const bool isA = t < ntA;
     int P = -1, R, rt = 0;
     if (isA) {
@@ -969,10 +975,10 @@ void eig_pairs(const EigBlock *blocks, int nblocks, int maxpairs, int round, con
                        active, tol, counter, inner_sweeps, eb);
 }
 
-void eig_apply(const EigBlock *blocks, int nblocks, int64_t maxtiles, int round, double *Aw,
-               double *Vw, const double *Qbuf, const int *active, hipStream_t st, EigBatch eb)
+void eig_apply(const EigBlock *blocks, int nblocks, const int64_t *tile_start, int64_t ntiles, int round,
+               double *Aw, double *Vw, const double *Qbuf, const int *active, hipStream_t st, EigBatch eb)
 {
-    hipLaunchKernelGGL(k_apply, dim3((unsigned)maxtiles, nblocks), dim3(kT), 0, st, blocks, round, Aw,
+    hipLaunchKernelGGL(k_apply, dim3((unsigned)ntiles), dim3(kT), 0, st, blocks, nblocks, tile_start, round, Aw,
                        Vw, Qbuf, active, eb);
 }
 

@@ -69,8 +69,34 @@ void eig_tol(const EigBlock *blocks, int nblocks, const double *Mw, double *tol,
 void eig_pairs(const EigBlock *blocks, int nblocks, int maxpairs, int round, const double *Aw,
                double *Qbuf, int *active, const double *tol, int *counter, int inner_sweeps,
                int wide, int bip, hipStream_t st, EigBatch eb = {});
-void eig_apply(const EigBlock *blocks, int nblocks, int64_t maxtiles, int round, double *Aw,
-               double *Vw, const double *Qbuf, const int *active, hipStream_t st, EigBatch eb = {});
+// blocks with N descending; tile_start (device): prefix sums of eig_tiles; ntiles: the
+// tiles of the blocks that have this round
+void eig_apply(const EigBlock *blocks, int nblocks, const int64_t *tile_start, int64_t ntiles, int round,
+               double *Aw, double *Vw, const double *Qbuf, const int *active, hipStream_t st, EigBatch eb = {});
+inline int64_t eig_tiles(const EigBlock &b)
+{
+    const int64_t np = b.N / 64;
+    return np * (np + 1) / 2 + np * np;
+}
+// host side of a list of blocks with N descending: tiles and the blocks and tiles of a round
+struct EigTiles {
+    std::vector<int64_t> start;   // prefix sums
+    std::vector<int> rounds;      // N / 32 - 1 of each block
+    explicit EigTiles(const EigBlock *b = nullptr, int n = 0)
+    {
+        start.assign(1, 0);
+        for (int i = 0; i < n; i++) {
+            start.push_back(start.back() + eig_tiles(b[i]));
+            rounds.push_back(b[i].N / 32 - 1);
+        }
+    }
+    int blocks(int round) const   // the first ones
+    {
+        int n = 0;
+        while (n < (int)rounds.size() && rounds[n] > round) n++;
+        return n;
+    }
+};
 // T = the columns of V with a positive eigenvalue, scaled to x = T T^T, side by side;
 // count[b]: how many (a multiple of kGemmK, zeros beyond the last)
 void eig_scale(const EigBlock *blocks, int nblocks, int max_N, const double *Aw, const double *Vw, double *Tw,
