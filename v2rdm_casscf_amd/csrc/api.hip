@@ -217,7 +217,7 @@ struct v2g_solver {
     {
         return std::max<int64_t>(1, plan.x_parts() + 3 * plan.row_parts());
     }
-    int64_t all_x_tiles = 0;   // of every primal segment, those of t2maps too
+    int64_t default_tiles = 0;   // of all primal segments and three times all rows, at the default cut
     // general = true: the final residual stays in own_cg_bufs().r
     int cg(const double *rhs, double *y, double tol, int maxiter, int precond, int flexible,
            double *res, bool general = false);
@@ -253,9 +253,13 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
         *L, {d_sym.p, d_gab.p, d_gaa.p, d_bab.p, d_baa.p, d_baab.p, d_baba.p, d_baaa.p, d_b00.p});
     d_lay.upload(std::vector<v2g::DevLayout>{dl});
 
-    auto tiles = [](const std::vector<v2g::Segment> &segs, std::vector<int64_t> &ts) {
+    int64_t erows = 0;   // not those of t2maps
+    for (const auto &s : L->rowsegs)
+        if (!s.wave && s.kind != v2g::RF_T2AAB && s.kind != v2g::RF_T2BIG) erows += s.count;
+    plan.per_thread = v2g::map_items_per_thread(erows);
+    auto tiles = [&](const std::vector<v2g::Segment> &segs, std::vector<int64_t> &ts) {
         ts.assign(1, 0);
-        for (const auto &s : segs) ts.push_back(ts.back() + v2g::tiles_for(s));
+        for (const auto &s : segs) ts.push_back(ts.back() + v2g::tiles_for(s, plan.per_thread));
         return ts.back();
     };
     std::vector<int64_t> ts;
@@ -277,7 +281,8 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
     plan.nrowsegs = (int)L->rowsegs.size();
     // T2 rows: t2maps takes them and, in A^T, the D2 and D1 entries
     std::vector<v2g::Segment> xs = L->xsegs, x2 = L->xsegs_t2;
-    all_x_tiles = tiles(xs, ts);
+    for (const auto &s : L->xsegs) default_tiles += v2g::tiles_for(s);
+    for (const auto &s : L->rowsegs) default_tiles += 3 * v2g::tiles_for(s);
     if (L->opt.t2) {
         auto drop = [](std::vector<v2g::Segment> &v, std::initializer_list<int> kinds) {
             v.erase(std::remove_if(v.begin(), v.end(), [&](const v2g::Segment &s) {
@@ -288,7 +293,7 @@ v2g_solver::v2g_solver(const v2g_layout_desc &d)
         t2maps.build(*L, d_lay.p);
         plan.t2maps = &t2maps;
         for (const auto &s : L->rowsegs)
-            if (s.kind == v2g::RF_T2AAB || s.kind == v2g::RF_T2BIG) plan.row_tiles_t2 += v2g::tiles_for(s);
+            if (s.kind == v2g::RF_T2AAB || s.kind == v2g::RF_T2BIG) plan.row_tiles_t2 += v2g::tiles_for(s, plan.per_thread);
     }
     plan.x_tiles = tiles(xs, ts);
     d_xsegs.upload(xs);
@@ -1011,7 +1016,7 @@ int v2g_cg_solve_noalloc(v2g_handle h, const double *rhs, double *y, double tol,
     const int64_t ncon = h->L->ncon, dimx = h->L->dimx;
     // (a plan with more partial sums than tiles keeps them in the handle's own array, so
     // what fits does not depend on how the rows are dealt out)
-    const int64_t tiles = std::max<int64_t>(1, h->all_x_tiles + 3 * h->plan.row_tiles);
+    const int64_t tiles = std::max<int64_t>(1, h->default_tiles);
     const int64_t need = 3 * up(ncon) + up(dimx) + up(v2g::kPartialArrays * v2g::kRedBlocks) +
                          up(v2g::CG_NSLOTS) + up(tiles);
     if (need > (int64_t)kScratchDoubles)

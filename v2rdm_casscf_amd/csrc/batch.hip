@@ -377,9 +377,9 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
 {
     HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     std::vector<v2g::DevLayout> dls;
-    auto tiles = [](const std::vector<v2g::Segment> &segs, std::vector<int64_t> &ts) {
+    auto tiles = [&](const std::vector<v2g::Segment> &segs, std::vector<int64_t> &ts) {
         ts.assign(1, 0);
-        for (const auto &s : segs) ts.push_back(ts.back() + v2g::tiles_for(s));
+        for (const auto &s : segs) ts.push_back(ts.back() + v2g::tiles_for(s, plan.per_thread));
         return ts.back();
     };
     std::vector<v2g::Segment> xsegs, t2segs;
@@ -454,6 +454,7 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
     d_lay.upload(dls);
     std::vector<int64_t> ts;
     plan.dlay = d_lay.p;
+    plan.per_thread = v2g::map_items_per_thread(ncon);
     plan.row_tiles = tiles(rowsegs, ts);
     d_rowsegs.upload(rowsegs);
     d_rowtiles.upload(ts);

@@ -33,6 +33,7 @@ struct MapPlan {
     // dlay holds one layout per problem (Segment::prob picks it); the done flag
     // of problem p is done[p * done_stride] (0: one flag for the whole plan)
     int done_stride = 0;
+    int per_thread = 0;   // elementwise items per thread the tiles are cut for (0: the default)
     bool tiled = false;   // some G2 block is visited by tiles (rowterms.hpp, kTileDim)
     // the T2 rows and the D2 / D1 entries of A^T they enter (null: with the other rows, and
     // xsegs / t2segs hold them); the last row_tiles_t2 tiles of rowsegs are these rows'
@@ -42,7 +43,8 @@ struct MapPlan {
     int64_t x_parts() const;     // of launch_atu
 };
 
-int64_t tiles_for(const Segment &s);
+int map_items_per_thread(int64_t rows);   // rows of A.x that take a thread each
+int64_t tiles_for(const Segment &s, int per_thread = 0);   // 0: the default number
 // fill the G2 column table for the row segments whose aux is >= 0; D1 columns
 // of x are [d1lo, d1hi)
 void build_g2_index(const MapPlan &p, const std::vector<Segment> &rowsegs, int64_t d1lo,

@@ -48,8 +48,7 @@ using namespace rows;
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / 64;
-constexpr int kPerThread = V2G_MAP_ITEMS_PER_THREAD;   // independent elementwise items per thread
-constexpr int kElemTile = kBlock * kPerThread;
+constexpr int kMany = V2G_MAP_ITEMS_PER_THREAD;   // elementwise items per thread (MapPlan::per_thread: this or 1)
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -161,7 +160,7 @@ k_g2_index(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs, i
 
 // fz.r (optional): the CG residual update fused in, r -= alpha (A.x) with the
 // tile sums of the new residual's dot products instead of A.x itself
-template <bool TILED>
+template <bool TILED, int kPerThread>
 __global__ void __launch_bounds__(kBlock, V2G_AU_WAVES_PER_EU)
 k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
      const int64_t *__restrict__ tile_start, int nseg, const double *__restrict__ x,
@@ -211,7 +210,7 @@ k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
         int2 ci[kPerThread];
 #pragma unroll
         for (int u = 0; u < kPerThread; u++) {
-            const int64_t pos = t * kElemTile + u * kBlock + threadIdx.x;
+            const int64_t pos = t * (kBlock * kPerThread) + u * kBlock + threadIdx.x;
             row[u] = -1;
             if (pos < sg.count) {
                 ci[u] = g2idx[sg.aux + pos];
@@ -240,7 +239,7 @@ k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
         int64_t row[kPerThread];
 #pragma unroll
         for (int u = 0; u < kPerThread; u++) {
-            const int64_t pos = t * kElemTile + u * kBlock + threadIdx.x;
+            const int64_t pos = t * (kBlock * kPerThread) + u * kBlock + threadIdx.x;
             Gather f{x, 0.0};
             row[u] = pos < sg.count ? row_of<TILED>(L, sg, pos) : -1;
             if (row[u] >= 0) elem_terms(L, sg, row[u], f);
@@ -270,6 +269,7 @@ k_au(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
 // diag(A A^T): squared norm of every constraint row (Jacobi preconditioner,
 // features of the learned preconditioner).  Trace rows repeat columns across
 // lanes and are given in closed form.
+template <int kPerThread>
 __global__ void __launch_bounds__(kBlock)
 k_row_norm2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
             const int64_t *__restrict__ tile_start, int nseg, double *__restrict__ d)
@@ -299,7 +299,7 @@ k_row_norm2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
         if (lane == 0) d[sg.start + item] = v;
     } else {
         for (int u = 0; u < kPerThread; u++) {
-            const int64_t pos = t * kElemTile + u * kBlock + threadIdx.x;
+            const int64_t pos = t * (kBlock * kPerThread) + u * kBlock + threadIdx.x;
             if (pos >= sg.count) return;
             const int64_t e = row_of(L, sg, pos);
             Collect f;
@@ -312,6 +312,7 @@ k_row_norm2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
 // eight waves per SIMD (57 VGPRs) to hide the gathers' latency.  sqpart
 // (optional): sqpart[tile] = sum of the squares of the tile's entries of
 // A^T.y, so that p.(A A^T p) = ||A^T p||^2 needs no second read of p
+template <int kPerThread>
 __global__ void __launch_bounds__(kBlock, 8)
 k_atu(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
       const int64_t *__restrict__ tile_start, int nseg, const double *__restrict__ y,
@@ -345,7 +346,7 @@ k_atu(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
         int64_t ent[kPerThread];
 #pragma unroll
         for (int u = 0; u < kPerThread; u++) {
-            const int64_t pos = t * kElemTile + u * kBlock + threadIdx.x;
+            const int64_t pos = t * (kBlock * kPerThread) + u * kBlock + threadIdx.x;
             v[u] = 0.0;
             ent[u] = pos < sg.count ? entry_of(L, sg, pos) : -1;
             if (ent[u] >= 0) {
@@ -371,6 +372,7 @@ k_atu(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
 
 // second-pass rows (T1, T2, spin-adapted Q2 / G2): self entry written, the
 // other terms accumulated
+template <int kPerThread>
 __global__ void __launch_bounds__(kBlock)
 k_atu_t2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
          const int64_t *__restrict__ tile_start, int nseg, const double *__restrict__ y,
@@ -382,7 +384,7 @@ k_atu_t2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
     if (done && done[(int64_t)sg.prob * done_stride] != 0.0) return;
     const DevLayout &L = Lp[sg.prob];
     for (int u = 0; u < kPerThread; u++) {
-        const int64_t e = (tile - tile_start[si]) * kElemTile + u * kBlock + threadIdx.x;
+        const int64_t e = (tile - tile_start[si]) * (kBlock * kPerThread) + u * kBlock + threadIdx.x;
         if (e >= sg.count) return;
         const double yv = y[sg.aux + e];
         ATy[sg.start + e] = -yv;
@@ -391,14 +393,22 @@ k_atu_t2(const DevLayout *__restrict__ Lp, const Segment *__restrict__ segs,
     }
 }
 
+// Below this many rows a launch waits for one thread's items in turn, and one item a thread
+// shortens it (15 orbitals, 0.7 million rows, A x and A^T y: 16 to 20 and 21 to 29 us with
+// four, 14.8 and 9.6 with one; 24 orbitals, 4 million: 37 and 25 us either way).  Above,
+// several a thread spare workgroups (H50 287 and 224 us against 346 and 238).
+constexpr int64_t kFewItems = 1 << 21;
+
 }  // namespace
 
 void launch_au(const MapPlan &p, const double *x, double *Ax, hipStream_t st, const double *done,
                const double *dotv, double *rowpart, CgFuse fz)
 {
     const int64_t tiles = p.row_tiles - p.row_tiles_t2;
+    const bool one = p.per_thread == 1;
     if (tiles > 0)
-        hipLaunchKernelGGL(p.tiled ? k_au<true> : k_au<false>, dim3((unsigned)tiles), dim3(kBlock), 0, st, p.dlay,
+        hipLaunchKernelGGL(p.tiled ? (one ? k_au<true, 1> : k_au<true, kMany>)
+                                   : (one ? k_au<false, 1> : k_au<false, kMany>), dim3((unsigned)tiles), dim3(kBlock), 0, st, p.dlay,
                            p.rowsegs, p.row_tile_start, p.nrowsegs, x, Ax, done, dotv, rowpart,
                            p.g2idx, p.done_stride, fz);
     if (p.t2maps) p.t2maps->au(x, Ax, done, dotv, rowpart ? rowpart + tiles : nullptr, fz, tiles, st);
@@ -419,7 +429,7 @@ void build_g2_index(const MapPlan &p, const std::vector<Segment> &rowsegs, int64
 void launch_row_norm2(const MapPlan &p, double *d, hipStream_t st)
 {
     if (p.row_tiles > 0)
-        hipLaunchKernelGGL(k_row_norm2, dim3((unsigned)p.row_tiles), dim3(kBlock), 0, st, p.dlay,
+        hipLaunchKernelGGL(p.per_thread == 1 ? k_row_norm2<1> : k_row_norm2<kMany>, dim3((unsigned)p.row_tiles), dim3(kBlock), 0, st, p.dlay,
                            p.rowsegs, p.row_tile_start, p.nrowsegs, d);
 }
 
@@ -431,21 +441,23 @@ void launch_atu(const MapPlan &p, const double *y, double *ATy, hipStream_t st, 
     if (sqpart && p.t2_tiles > 0)
         throw std::logic_error("||A^T y||^2 partials need a layout without second-pass rows");
     if (p.x_tiles > 0)
-        hipLaunchKernelGGL(k_atu, dim3((unsigned)chunk_grid(p.x_tiles)), dim3(kBlock), 0, st, p.dlay,
+        hipLaunchKernelGGL(p.per_thread == 1 ? k_atu<1> : k_atu<kMany>, dim3((unsigned)chunk_grid(p.x_tiles)), dim3(kBlock), 0, st, p.dlay,
                            p.xsegs, p.x_tile_start, p.nxsegs, y, ATy, done, p.x_tiles, p.done_stride,
                            sqpart);
     if (p.t2maps) p.t2maps->atu(y, ATy, done, sqpart ? sqpart + p.x_tiles : nullptr, st);
     if (p.t2_tiles > 0)
-        hipLaunchKernelGGL(k_atu_t2, dim3((unsigned)p.t2_tiles), dim3(kBlock), 0, st, p.dlay,
+        hipLaunchKernelGGL(p.per_thread == 1 ? k_atu_t2<1> : k_atu_t2<kMany>, dim3((unsigned)p.t2_tiles), dim3(kBlock), 0, st, p.dlay,
                            p.t2segs, p.t2_tile_start, p.nt2segs, y, ATy, done, p.done_stride);
 }
 
 int64_t MapPlan::row_parts() const { return row_tiles - row_tiles_t2 + (t2maps ? t2maps->au_blocks() : 0); }
 int64_t MapPlan::x_parts() const { return x_tiles + (t2maps ? t2maps->atu_blocks() : 0); }
 
-int64_t tiles_for(const Segment &s)
+int map_items_per_thread(int64_t rows) { return rows < kFewItems ? 1 : kMany; }
+
+int64_t tiles_for(const Segment &s, int per_thread)
 {
-    const int64_t per = s.wave ? kWavesPerBlock : kElemTile;
+    const int64_t per = s.wave ? kWavesPerBlock : kBlock * (per_thread > 0 ? per_thread : kMany);
     return (s.count + per - 1) / per;
 }
 
