@@ -13,7 +13,8 @@
 //   * D2ab / D2aa / D2bb entries invert each family's index rule in closed
 //     form (the particle-hole G2 maps are permutations per irrep);
 //   * D1 entries sum O(amo) rows -> one wavefront per entry.
-// With T1, T2 or spin-adapted Q2 / G2 on, a second launch walks those rows:
+// The T2 rows of a single problem have kernels of their own (t2maps.hip), gathers too.  With
+// T1 or spin-adapted Q2 / G2 on (and T2 in a batch), a second launch walks those rows:
 // each row's own block entry is a self term, and the terms the rows put into
 // Q2 / D2 / G2 / D1 / Q1 entries are added with hardware FP64 atomics, so
 // A^T.y with any of them is not bitwise reproducible from run to run (it is

@@ -165,15 +165,6 @@ struct Ptr {
     __device__ __forceinline__ double operator[](int64_t i) const { return a[i]; }
 };
 
-__device__ __forceinline__ void store_cell(const RedLayout &R, int64_t pos, int64_t cc, int64_t k, double *x,
-                                           const Cell &c)
-{
-#pragma unroll
-    for (int o = 0; o < 4; o++) x[pos + o * cc] = c.ab[o];
-    x[R.nAB + k] = c.aa;
-    x[R.nAB + R.nAA + k] = c.bb;
-}
-
 __device__ __forceinline__ double cell_sq(const Cell &t)
 {
     return ((t.ab[0] * t.ab[0] + t.ab[1] * t.ab[1]) + (t.ab[2] * t.ab[2] + t.ab[3] * t.ab[3])) +
