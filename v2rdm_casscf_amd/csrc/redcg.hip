@@ -855,13 +855,28 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     std::vector<uint32_t> rank;
     std::vector<int32_t> rowtab;
     std::vector<size_t> to(4 * np_), ao(np_), co(np_), bo(np_), ro(np_);
+    auto list = [&](int q, int k) -> const std::vector<Segment> & {
+        return k == 0 ? work[q].start : k == 1 ? work[q].dir : k == 2 ? work[q].res : work[q].norm;
+    };
+    auto items = [&](int q, const Segment &s) -> int64_t {
+        return s.wave == 0 ? kNT : s.wave == 1 ? kWaves : s.wave == 3 ? kNT / prob[q].R.lanes : 1;
+    };
+    size_t ntl = 0;
+    for (int q = 0; q < np_; q++)
+        for (int k = 0; k < 4; k++)
+            for (const Segment &s : list(q, k)) ntl += (size_t)((s.count + items(q, s) - 1) / items(q, s));
+    tl.reserve(ntl);
+    // a problem's lists follow each other's; the first's are taken as they are
+    auto join = [](auto &all, auto &one) {
+        if (all.empty()) all = std::move(one);
+        else all.insert(all.end(), one.begin(), one.end());
+    };
     for (int q = 0; q < np_; q++) {
         tiles[q] = 1;
         for (int k = 0; k < 4; k++) {
-            const auto &v = k == 0 ? work[q].start : k == 1 ? work[q].dir : k == 2 ? work[q].res : work[q].norm;
             to[4 * q + k] = tl.size();
-            for (const Segment &s : v) {
-                const int64_t per = s.wave == 0 ? kNT : s.wave == 1 ? kWaves : s.wave == 3 ? kNT / prob[q].R.lanes : 1;
+            for (const Segment &s : list(q, k)) {
+                const int64_t per = items(q, s);
                 for (int64_t i = 0; i < s.count; i += per) tl.push_back({s, i});
             }
             prob[q].ntile[k] = (int)(tl.size() - to[4 * q + k]);
@@ -872,11 +887,11 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
         co[q] = cell.size();
         bo[q] = bits.size();
         ro[q] = rowtab.size();
-        rowtab.insert(rowtab.end(), work[q].rowtab.begin(), work[q].rowtab.end());
-        bits.insert(bits.end(), work[q].bits.begin(), work[q].bits.end());
-        rank.insert(rank.end(), work[q].rank.begin(), work[q].rank.end());
-        ab.insert(ab.end(), work[q].ab.begin(), work[q].ab.end());
-        cell.insert(cell.end(), work[q].cell.begin(), work[q].cell.end());
+        join(rowtab, work[q].rowtab);
+        join(bits, work[q].bits);
+        join(rank, work[q].rank);
+        join(ab, work[q].ab);
+        join(cell, work[q].cell);
     }
     // workgroups in proportion to the tiles, at least one a problem
     std::vector<int> blk;
