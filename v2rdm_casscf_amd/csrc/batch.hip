@@ -405,8 +405,6 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
         r.nr = Lq.ncon;
         r.x0 = dimx;
         r.nx = Lq.dimx;
-        r.t0 = 0;
-        for (const auto &s : rowsegs) r.t0 += v2g::tiles_for(s);
         for (auto s : Lq.rowsegs) {
             s.start += ncon;
             s.prob = q;
@@ -415,8 +413,6 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
             if (s.aux >= 0) g2rows += s.count;
             rowsegs.push_back(s);
         }
-        r.nt = 0;
-        for (const auto &s : Lq.rowsegs) r.nt += v2g::tiles_for(s);
         for (auto s : Lq.xsegs) {
             s.start += dimx;
             if (s.kind == v2g::XS_SELF) s.aux += ncon;
@@ -456,6 +452,18 @@ v2g_batch::v2g_batch(const v2g_layout_desc *descs, int n) : np(n)
     plan.dlay = d_lay.p;
     plan.per_thread = v2g::map_items_per_thread(ncon);
     plan.row_tiles = tiles(rowsegs, ts);
+    // each problem's tiles, as the launch is cut (the cut follows from all rows together)
+    for (size_t i = 0; i < rowsegs.size(); i++) {
+        v2g::ProbRange &r = pr[rowsegs[i].prob];
+        if (r.nt == 0) r.t0 = ts[i];
+        r.nt = ts[i + 1] - r.t0;
+    }
+    int64_t dealt = 0;
+    for (const auto &r : pr) {
+        if (r.nt > 0 && r.t0 != dealt) throw std::logic_error("batch: row tiles out of order");
+        dealt += r.nt;
+    }
+    if (dealt != plan.row_tiles) throw std::logic_error("batch: row tiles not all dealt out");
     d_rowsegs.upload(rowsegs);
     d_rowtiles.upload(ts);
     plan.rowsegs = d_rowsegs.p;
