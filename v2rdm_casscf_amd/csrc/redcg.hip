@@ -804,6 +804,9 @@ k_red_y(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B
     const Place pl = place(prob, blk);
     if (active && !active[pl.prob]) return;
     const View V = view(B, *pl.pr, pl.prob, 0);
+    // no iterations: y keeps every bit (0 times a residual that is not finite is no zero,
+    // and -0 + 0 is not -0)
+    if (V.scal[RS_MAXIT] <= 0.0) return;
     const double e = V.scal[RS_B + 3 + 1];
     const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
