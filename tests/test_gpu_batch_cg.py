@@ -27,6 +27,14 @@ BATCHES = {
     "t1 and plain": [D2H, dict(C1, positivity="DQGT1"), dict(amopi=[9], nalpha=4, nbeta=4)],
     "spin adapted": [dict(amopi=[5], nalpha=2, nbeta=2, spin_adapt_q2=True), C1,
                      dict(D2H, constrain_spin=False, spin_adapt_q2=True, spin_adapt_g2=True)],
+    # batches of the reduced form: closed shells with every condition, and one problem or
+    # more without, which takes all of the batch to the kernels that ask the layout
+    "reduced": [dict(amopi=[4], nalpha=2, nbeta=2), D2H, dict(amopi=[7], nalpha=3, nbeta=3)],
+    "reduced, mixed": [D2H, C1, dict(amopi=[3, 2], nalpha=3, nbeta=2, positivity="DQ"),
+                       dict(amopi=[5], nalpha=2, nbeta=2, positivity="DG"),
+                       dict(amopi=[4], nalpha=3, nbeta=1, positivity="DG", constrain_spin=False),
+                       dict(amopi=[0, 3, 2, 1], nalpha=3, nbeta=1, constrain_sz=False),
+                       dict(amopi=[6], nalpha=4, nbeta=2), dict(amopi=[7], nalpha=3, nbeta=3)],
 }
 
 
@@ -97,3 +105,16 @@ def test_batch_iteration_matches_recurrence(name, n):
 def test_batch_of_many_problems():
     """More problems than the reduced form of the CG takes in one batch (1 024)."""
     _run([SMALL] * 1025, (0, 511, 1024), 3)
+
+
+def test_batch_of_many_mid_sized_blocks():
+    """More blocks of 33 to 64 indices in a launch than its 1 024-thread workgroups take
+    (kFewMid, 512): even and odd sizes from 33 to 64, with 256 threads each."""
+    probs = ([dict(amopi=[5, 4], nalpha=4, nbeta=4)] * 50 + [dict(amopi=[6], nalpha=3, nbeta=3)]
+             + [dict(amopi=[7], nalpha=4, nbeta=3), dict(amopi=[8], nalpha=4, nbeta=4),
+                dict(amopi=[11, 3], nalpha=4, nbeta=4, positivity="D"),
+                dict(amopi=[9, 7], nalpha=4, nbeta=4, positivity="D")]
+             + [dict(amopi=[7], nalpha=3, nbeta=3)] * 10)
+    mid = [n for pb in probs for n in _layout(pb).block_dims if 32 < n <= 64]
+    assert len(mid) > 512 and {33, 36, 40, 41, 49, 57, 63, 64} <= set(mid)
+    _run(probs, (0, 49, 50, 51, 52, 53, 54, 64), 2)

@@ -1,5 +1,6 @@
-"""Update_xz of small blocks at the edges of their kernels: one wavefront up to 32 indices,
-256 threads up to 64, the block Jacobi above; odd sizes, a block of one index, matrices whose
+"""Update_xz of small blocks at the edges of their kernels: 256 threads up to 32 indices,
+1 024 up to 64 (256 where a launch has more than 512 such blocks: test_gpu_batch_cg.py),
+the block Jacobi above; odd sizes, a block of one index, matrices whose
 squares leave the range of the fast rotation, and ones with nothing to rotate.  Against the
 oracle (LAPACK), 1e-10 relative, as the other splits."""
 import numpy as np
