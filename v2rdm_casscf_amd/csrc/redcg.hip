@@ -338,10 +338,9 @@ k_red_aty(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
         a[2] = 0.0;                         // d
         a[3] = 0.0;
         a[4] = 0.0;                         // iterations begun
-        double *b = V.scal + RS_B + 3;
+        double *b = V.scal + RS_B + 2;
         b[0] = 1.0;                         // c
         b[1] = 0.0;                         // e
-        b[2] = 0.0;
         V.scal[RS_DONE] = 0.0;
         V.scal[RS_NRM] = 0.0;
         V.scal[RS_ITER] = 0.0;
@@ -488,7 +487,7 @@ k_red_dir(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
     const Place pl = place(prob, blk);
     const View V = view(B, *pl.pr, pl.prob, par);
     double *a1 = V.scal + RS_A + 6 * par;
-    const double *a0 = V.scal + RS_A + 6 * (par ^ 1), *b0 = V.scal + RS_B + 3 * (par ^ 1);
+    const double *a0 = V.scal + RS_A + 6 * (par ^ 1), *b0 = V.scal + RS_B + 2 * (par ^ 1);
     if (a0[0] != 0.0) {
         if (pl.lb == 0 && threadIdx.x == 0) a1[0] = 1.0;
         return;
@@ -581,8 +580,8 @@ k_red_res(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
     __shared__ double sh[kWaves];
     const Place pl = place(prob, blk);
     const View V = view(B, *pl.pr, pl.prob, par);
-    const double *a = V.scal + RS_A + 6 * par, *b0 = V.scal + RS_B + 3 * (par ^ 1);
-    double *b1 = V.scal + RS_B + 3 * par;
+    const double *a = V.scal + RS_A + 6 * par, *b0 = V.scal + RS_B + 2 * (par ^ 1);
+    double *b1 = V.scal + RS_B + 2 * par;
     if (a[0] != 0.0) {
         if (pl.lb == 0 && threadIdx.x == 0) { b1[0] = b0[0]; b1[1] = b0[1]; }
         return;
@@ -594,7 +593,6 @@ k_red_res(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
     if (pl.lb == 0 && threadIdx.x == 0) {
         b1[0] = fma(-alpha, d, b0[0]);
         b1[1] = fma(alpha, d, b0[1]);
-        b1[2] = alpha;
     }
     const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
@@ -671,7 +669,7 @@ k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     const Place pl = place(prob, blk);
     const View V = view(B, *pl.pr, pl.prob, par);
     if (V.scal[RS_A + 6 * par] != 0.0) return;
-    const double c = V.scal[RS_B + 3 * par], d = V.scal[RS_A + 6 * par + 2];
+    const double c = V.scal[RS_B + 2 * par], d = V.scal[RS_A + 6 * par + 2];
     const RedLayout &R = pl.pr->R;
     const bool q2 = FULL || R.L.q2, g2 = FULL || R.L.g2;
     const int nd = FULL ? 1 : R.nblk_d;
@@ -807,7 +805,7 @@ k_red_y(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B
     // no iterations: y keeps every bit (0 times a residual that is not finite is no zero,
     // and -0 + 0 is not -0)
     if (V.scal[RS_MAXIT] <= 0.0) return;
-    const double e = V.scal[RS_B + 3 + 1];
+    const double e = V.scal[RS_B + 2 + 1];
     const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
     const Ptr w{V.w}, om{V.om};

@@ -80,7 +80,7 @@ struct RedBufs {
 // ping-pong pairs indexed by the iteration parity; the rest is read by the host
 enum RedSlot : int {
     RS_A = 0,        // + 6 parity: done, r.z, d, ||p_self||^2, iterations begun
-    RS_B = 12,       // + 3 parity: c, e, alpha
+    RS_B = 12,       // + 2 parity: c, e
     RS_DONE = 18, RS_NRM = 20, RS_ITER = 21, RS_TOL = 25, RS_MAXIT = 26, RS_NRM0 = 29
 };
 constexpr int kRedScal = 32;

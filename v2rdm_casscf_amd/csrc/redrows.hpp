@@ -74,17 +74,17 @@ enum RowTab : int {
     RT_Q2, RT_G2AB, RT_G2BA, RT_GA, RT_GB, RT_D0, RT_D1, RT_COUNT   // rows
 };
 
-// a D2ab entry outside the cells (p == q or r == s): where everything lies that its rows read, -1 never occurs (the
-// zero at the end of the vector stands for an absent entry)
+// a D2ab entry outside the cells (p == q or r == s): where everything lies that its rows
+// read, -1 never occurs (the zero at the end of the vector stands for an absent entry).  It
+// has no D2aa entry and no antisymmetry row
 struct AbRec {
     int32_t pos, p1, p2, p3;   // (pq|rs), (qp|rs), (pq|sr), (qp|sr)
-    int32_t ka;                // its D2aa entry
     int32_t pr, rp;            // D1a entries (p,r), (r,p) when q == s
     int32_t qs, sq;            // D1b entries (q,s), (s,q) when p == r
     int32_t m0, m1;            // maximal-spin rows when s == p, q == r
     int32_t flags;             // AbFlag
 };
-enum AbFlag : int { AF_NEG = 1, AF_BRA = 2, AF_KET = 4, AF_QS = 8, AF_PR = 16, AF_S2 = 32 };
+enum AbFlag : int { AF_BRA = 1, AF_KET = 2, AF_QS = 4, AF_PR = 8, AF_S2 = 16 };
 
 // a listed cell: its pairs share an orbital k, or both orbitals.  With i and j the others
 // of the two pairs, a shared orbital puts D1a(i,j) into the rows of (ik|jk), D1b(i,j) into
@@ -93,7 +93,7 @@ struct CellRec {
     int32_t pos, k;            // first D2ab entry, place among the cells
     int32_t ij[2], ji[2];      // D1a entries (i,j), (j,i)
     int32_t m0[2], m1[2];      // maximal-spin rows of (ki|jk), (ik|kj)
-    int32_t row;               // place within the irrep
+    int32_t row;               // place within the irrep (for checks)
     int32_t flags;             // orientation of (ik|jk) in bits 0-1 and 2-3, CellFlag, irrep << 8
 };
 enum CellFlag : int { CF_TWO = 16 };
@@ -533,6 +533,7 @@ V2G_HD inline double full_at_aa(const DevLayout &Lo, int sp, const AbEntry &a, c
 }
 
 // ---- listed entries ------------------------------------------------------------
+// p == q or r == s
 V2G_HD inline AbRec make_ab_rec(const RedLayout &R, int p, int q, int r, int s)
 {
     const DevLayout &L = R.L;
@@ -541,16 +542,14 @@ V2G_HD inline AbRec make_ab_rec(const RedLayout &R, int p, int q, int r, int s)
     a.p1 = (int32_t)ab_pos(R, q, p, r, s);
     a.p2 = (int32_t)ab_pos(R, p, q, s, r);
     a.p3 = (int32_t)ab_pos(R, q, p, s, r);
-    const bool diag = p == q || r == s;
-    a.ka = (int32_t)(diag ? R.nD : R.nAB + aa_pos(R, p, q, r, s));
     a.pr = (int32_t)(q == s ? d1_col(L, XB_D1A, p, r) : R.nD);
     a.rp = (int32_t)(q == s ? d1_col(L, XB_D1A, r, p) : R.nD);
     a.qs = (int32_t)(p == r ? d1_col(L, XB_D1B, q, s) : R.nD);
     a.sq = (int32_t)(p == r ? d1_col(L, XB_D1B, s, q) : R.nD);
     a.m0 = R.nM && s == p ? L.gab[q * L.amo + r] : R.nM;
     a.m1 = R.nM && q == r ? L.gems_ab[0] + L.gab[s * L.amo + p] : R.nM;
-    a.flags = ((p < q) == (r < s) ? 0 : AF_NEG) | (p == q ? AF_BRA : 0) | (r == s ? AF_KET : 0) |
-              (q == s ? AF_QS : 0) | (p == r ? AF_PR : 0) | (p == s && q == r ? AF_S2 : 0);
+    a.flags = (p == q ? AF_BRA : 0) | (r == s ? AF_KET : 0) | (q == s ? AF_QS : 0) | (p == r ? AF_PR : 0) |
+              (p == s && q == r ? AF_S2 : 0);
     return a;
 }
 
@@ -589,7 +588,7 @@ V2G_HD inline CellRec make_cell_rec(const RedLayout &R, int p, int q, int r, int
 
 // what a listed D2ab entry reads of a D vector
 struct AbVals {
-    double x0, x1, x2, x3, aa, bb, arp, apr, bpr, bsq, bqs;
+    double x0, x1, x2, x3, arp, apr, bpr, bsq, bqs;
     template <class X>
     V2G_HD inline AbVals(const RedLayout &R, const AbRec &a, const X &x)
     {
@@ -597,8 +596,6 @@ struct AbVals {
         x1 = x[a.p1];
         x2 = x[a.p2];
         x3 = x[a.p3];
-        aa = x[a.ka];
-        bb = x[a.flags & (AF_BRA | AF_KET) ? a.ka : a.ka + (int32_t)R.nAA];
         arp = x[a.rp];
         apr = x[a.pr];
         bpr = x[a.flags & AF_QS ? a.pr + (int32_t)R.nD1 : a.pr];
@@ -608,15 +605,15 @@ struct AbVals {
     V2G_HD inline double q2() const { return x0 - arp - bsq; }
     V2G_HD inline double g1() const { return apr - x0; }
     V2G_HD inline double g2() const { return bqs - x0; }
-    V2G_HD inline double ga(const AbRec &a) const { return a.flags & AF_NEG ? apr + aa : apr - aa; }
-    V2G_HD inline double gb(const AbRec &a) const { return a.flags & AF_NEG ? bpr + bb : bpr - bb; }
+    V2G_HD inline double ga(const AbRec &) const { return apr; }
+    V2G_HD inline double gb(const AbRec &) const { return bpr; }
     V2G_HD inline double d200(const RedLayout &R, const AbRec &a, int blk) const
     {
         double c[4];
         d200_coef(blk, R.L.singlet, (a.flags & AF_BRA) != 0, (a.flags & AF_KET) != 0, c);
         return c[0] * x0 + c[1] * x1 + c[2] * x2 + c[3] * x3;
     }
-    // B2^T B2 x (gram_ab without its maximal-spin part)
+    // B2^T B2 x (the maximal-spin part, nu[m0] + nu[m1], is the caller's)
     V2G_HD inline double gram(const RedLayout &R, const AbRec &a) const
     {
         double t = (R.L.q2 ? x0 - arp - bsq : 0.0) + (R.L.g2 ? 4.0 * x0 - apr - bqs : 0.0);
@@ -644,11 +641,6 @@ V2G_HD inline double rec_expl_ab(const RedLayout &R, const AbRec &a, const Y &y)
     const int64_t tr = L.rowoff[RF_TRACE][L.sz ? 0 : 3][0];
     double v = (L.sz ? 1.0 : 2.0) * y[A && B ? tr : R.nR] - y[A ? ca : R.nR] - y[B ? cb : R.nR];
     if (L.spin) v += y[a.flags & AF_S2 ? L.rowoff[RF_S2][0][0] : R.nR];
-    if (R.cells && !(a.flags & (AF_BRA | AF_KET))) {
-        const int64_t k = a.ka - R.nAB;
-        const double an = 0.5 * (y[R.nAA + k] + y[2 * R.nAA + k]);
-        v += a.flags & AF_NEG ? an : -an;
-    }
     return v;
 }
 

@@ -524,18 +524,18 @@ V2G_HD inline void elem_terms(const DevLayout &L, const Segment &sg, int64_t e, 
     }
 }
 
-// one wavefront (or `lanes` threads) per row (traces, S^2, contractions,
-// maximal-spin rows): the lane-strided share of the row's terms.  Columns are distinct across the
+// one wavefront per row (traces, S^2, contractions, maximal-spin rows): the
+// lane-strided share of the row's terms.  Columns are distinct across the
 // terms of one row except in the trace rows (handled in the diagonal pass).
 template <class F>
 V2G_HD inline void wave_terms(const DevLayout &L, const Segment &sg, int64_t item,
-                                           int lane, F &f, int lanes = 64)
+                                           int lane, F &f)
 {
     const int amo = L.amo;
     const int *gab = L.gab, *gaa = L.gaa, *sym = L.sym;
     switch (sg.kind) {
     case RF_TRACE: {  // d2.cc:303-366
-        for (int pq = lane; pq < amo * amo; pq += lanes) {
+        for (int pq = lane; pq < amo * amo; pq += 64) {
             const int i = pq / amo, j = pq % amo, h = sym[i] ^ sym[j];
             const int64_t gb = L.gems_ab[h], ga = L.gems_aa[h];
             if (sg.sub == 0) {
@@ -557,7 +557,7 @@ V2G_HD inline void wave_terms(const DevLayout &L, const Segment &sg, int64_t ite
         return;
     }
     case RF_S2: {  // spin.cc:281-292
-        for (int pq = lane; pq < amo * amo; pq += lanes) {
+        for (int pq = lane; pq < amo * amo; pq += 64) {
             const int i = pq / amo, j = pq % amo, h = sym[i] ^ sym[j];
             f(L.xoff[XB_D2AB][h] + (int64_t)gab[i * amo + j] * L.gems_ab[h] + gab[j * amo + i], 1.0);
         }
@@ -582,7 +582,7 @@ V2G_HD inline void wave_terms(const DevLayout &L, const Segment &sg, int64_t ite
             }
             f(L.xoff[beta ? XB_D1B : XB_D1A][h] + i * n + j, coef);
         }
-        for (int k = lane; k < amo; k += lanes) {
+        for (int k = lane; k < amo; k += 64) {
             const int h2 = sym[ii] ^ sym[k];
             if (use_ab) {
                 const int64_t ik = beta ? gab[k * amo + ii] : gab[ii * amo + k];
@@ -599,7 +599,7 @@ V2G_HD inline void wave_terms(const DevLayout &L, const Segment &sg, int64_t ite
     }
     case RF_MAXSPIN: {  // spin.cc:471-491
         const int64_t g0 = L.gems_ab[0], kl = item;
-        for (int i = lane; i < amo; i += lanes) {
+        for (int i = lane; i < amo; i += 64) {
             const int64_t ii = gab[i * amo + i];
             f(L.xoff[XB_G2BA][0] + (sg.sub == 0 ? kl * g0 + ii : ii * g0 + kl), 1.0);
         }
@@ -718,11 +718,11 @@ V2G_HD inline int64_t entry_of(const DevLayout &L, const Segment &sg, int64_t po
 // A^T.y gathers.  The rows of A fall in two groups: a self row holds one entry
 // +-1 in a block of its own (D200, Q1, Q2, G2), an explicit row (traces,
 // contractions, S^2, the D1 / D2 spin rows) holds D2 and D1 entries only.
-// SELF / EXPL select which groups a gather of a D2 or D1 entry takes; y is
-// anything that can be indexed by the row.
+// SELF / EXPL select which groups a gather of a D1 entry takes; y is anything
+// that can be indexed by the row.
 // ----------------------------------------------------------------------------
 
-template <bool SELF = true, bool EXPL = true, class Y = const double *>
+template <class Y>
 V2G_HD inline double atu_d2ab(const DevLayout &L, const Segment &sg, int64_t e, const Y &y)
 {
     const int amo = L.amo, h = sg.h, g = sg.dim;
@@ -733,43 +733,36 @@ V2G_HD inline double atu_d2ab(const DevLayout &L, const Segment &sg, int64_t e, 
     const int pij = L.bab[L.bab_off[h] + IJ], pkl = L.bab[L.bab_off[h] + KL];
     const int p = P0(pij), q = P1(pij), r = P0(pkl), s = P1(pkl);
     double v = 0.0;
-    if constexpr (EXPL) {
-        // trace rows
-        if (IJ == KL) v += L.sz ? y[L.rowoff[RF_TRACE][0][0]] : 2.0 * y[L.rowoff[RF_TRACE][3][0]];
-        // D2ab -> D1a : row (p, r) of irrep sym p when q == s
-        if (q == s) {
-            const int hp = sym[p], n = L.amopi[hp];
-            v -= y[L.rowoff[RF_CONTR][L.sz ? 0 : 4][hp] + (p - L.poff[hp]) * n + (r - L.poff[hp])];
-        }
-        // D2ab -> D1b : row (q, s) when p == r
-        if (p == r) {
-            const int hq = sym[q], n = L.amopi[hq];
-            v -= y[L.rowoff[RF_CONTR][L.sz ? 1 : 5][hq] + (q - L.poff[hq]) * n + (s - L.poff[hq])];
-        }
+    // trace rows
+    if (IJ == KL) v += L.sz ? y[L.rowoff[RF_TRACE][0][0]] : 2.0 * y[L.rowoff[RF_TRACE][3][0]];
+    // D2ab -> D1a : row (p, r) of irrep sym p when q == s
+    if (q == s) {
+        const int hp = sym[p], n = L.amopi[hp];
+        v -= y[L.rowoff[RF_CONTR][L.sz ? 0 : 4][hp] + (p - L.poff[hp]) * n + (r - L.poff[hp])];
+    }
+    // D2ab -> D1b : row (q, s) when p == r
+    if (p == r) {
+        const int hq = sym[q], n = L.amopi[hq];
+        v -= y[L.rowoff[RF_CONTR][L.sz ? 1 : 5][hq] + (q - L.poff[hq]) * n + (s - L.poff[hq])];
     }
     if (L.spin) {
-        if constexpr (EXPL)
-            if (p == s && q == r) v += y[L.rowoff[RF_S2][0][0]];
+        if (p == s && q == r) v += y[L.rowoff[RF_S2][0][0]];
         const int64_t qp = GAB(q, p), sr = GAB(s, r);
         const double dpq = (p == q) ? 1.4142135623730951 : 1.0;
         const double drs = (r == s) ? 1.4142135623730951 : 1.0;
         if (L.singlet) {
-            if constexpr (EXPL) {
-                if (p != q && r != s) {
-                    const int64_t ga = L.gems_aa[h];
-                    const int64_t ia = gaa[p * amo + q], ka = gaa[r * amo + s];
-                    const double sg2 = ((p > q) == (r > s)) ? 1.0 : -1.0;
-                    v += -0.5 * sg2 *
-                         (y[L.rowoff[RF_SPIN_ANTI][0][h] + ia * ga + ka] + y[L.rowoff[RF_SPIN_ANTI][1][h] + ia * ga + ka]);
-                }
+            if (p != q && r != s) {
+                const int64_t ga = L.gems_aa[h];
+                const int64_t ia = gaa[p * amo + q], ka = gaa[r * amo + s];
+                const double sg2 = ((p > q) == (r > s)) ? 1.0 : -1.0;
+                v += -0.5 * sg2 *
+                     (y[L.rowoff[RF_SPIN_ANTI][0][h] + ia * ga + ka] + y[L.rowoff[RF_SPIN_ANTI][1][h] + ia * ga + ka]);
             }
-            if constexpr (SELF) {
-                const int64_t R0 = L.rowoff[RF_SPIN_D200][0][h];
-                const double c = -0.5 / (dpq * drs);
-                v += c * (y[R0 + (int64_t)IJ * g + KL] + y[R0 + qp * g + KL] + y[R0 + (int64_t)IJ * g + sr] +
-                          y[R0 + qp * g + sr]);
-            }
-        } else if constexpr (SELF) {
+            const int64_t R0 = L.rowoff[RF_SPIN_D200][0][h];
+            const double c = -0.5 / (dpq * drs);
+            v += c * (y[R0 + (int64_t)IJ * g + KL] + y[R0 + qp * g + KL] + y[R0 + (int64_t)IJ * g + sr] +
+                      y[R0 + qp * g + sr]);
+        } else {
             const int64_t G = 2 * (int64_t)g;
             const int64_t R4 = L.rowoff[RF_SPIN_D200_4][0][h];
             for (int blk = 0; blk < 4; blk++) {
@@ -785,7 +778,6 @@ V2G_HD inline double atu_d2ab(const DevLayout &L, const Segment &sg, int64_t e, 
             }
         }
     }
-    if constexpr (!SELF) return v;
     if (L.q2) v += y[L.rowoff[RF_Q2AB][0][h] + e];
     if (L.g2) {
         {   // G2ab row ((p,s),(r,q))
@@ -810,7 +802,7 @@ V2G_HD inline double atu_d2ab(const DevLayout &L, const Segment &sg, int64_t e, 
     return v;
 }
 
-template <bool SELF = true, bool EXPL = true, class Y = const double *>
+template <class Y>
 V2G_HD inline double atu_d2aa(const DevLayout &L, const Segment &sg, int64_t e, const Y &y)
 {
     const int amo = L.amo, h = sg.h, ga = sg.dim, sp = sg.sub;
@@ -820,26 +812,23 @@ V2G_HD inline double atu_d2aa(const DevLayout &L, const Segment &sg, int64_t e, 
     const int pij = L.baa[L.baa_off[h] + IJ], pkl = L.baa[L.baa_off[h] + KL];
     const int p1 = P0(pij), p2 = P1(pij), r1 = P0(pkl), r2 = P1(pkl);
     double v = 0.0;
-    if constexpr (EXPL) {
-        if (IJ == KL) v += 2.0 * y[L.rowoff[RF_TRACE][L.sz ? 1 + sp : 3][0]];
-        // contraction rows: common orbital k of the two pairs
-        const int csub = L.sz ? 2 + sp : 4 + sp;
-        for (int a = 0; a < 2; a++) {
-            const int k = a ? p2 : p1, ii = a ? p1 : p2;
-            int jj = -1;
-            if (r1 == k) jj = r2;
-            else if (r2 == k) jj = r1;
-            if (jj < 0) continue;
-            const int hi = sym[ii], n = L.amopi[hi];
-            const double sg2 = ((ii < k) == (jj < k)) ? 1.0 : -1.0;
-            v -= sg2 * y[L.rowoff[RF_CONTR][csub][hi] + (ii - L.poff[hi]) * n + (jj - L.poff[hi])];
-        }
-        if (L.spin && L.singlet) {
-            v += (sp ? -1.0 : 1.0) * y[L.rowoff[RF_SPIN_D2][0][h] + e];
-            v += y[L.rowoff[RF_SPIN_ANTI][sp][h] + e];
-        }
+    if (IJ == KL) v += 2.0 * y[L.rowoff[RF_TRACE][L.sz ? 1 + sp : 3][0]];
+    // contraction rows: common orbital k of the two pairs
+    const int csub = L.sz ? 2 + sp : 4 + sp;
+    for (int a = 0; a < 2; a++) {
+        const int k = a ? p2 : p1, ii = a ? p1 : p2;
+        int jj = -1;
+        if (r1 == k) jj = r2;
+        else if (r2 == k) jj = r1;
+        if (jj < 0) continue;
+        const int hi = sym[ii], n = L.amopi[hi];
+        const double sg2 = ((ii < k) == (jj < k)) ? 1.0 : -1.0;
+        v -= sg2 * y[L.rowoff[RF_CONTR][csub][hi] + (ii - L.poff[hi]) * n + (jj - L.poff[hi])];
     }
-    if constexpr (!SELF) return v;
+    if (L.spin && L.singlet) {
+        v += (sp ? -1.0 : 1.0) * y[L.rowoff[RF_SPIN_D2][0][h] + e];
+        v += y[L.rowoff[RF_SPIN_ANTI][sp][h] + e];
+    }
     if (L.q2) v += y[L.rowoff[RF_Q2AA][sp][h] + e];
     if (L.g2) {
         // G2aaaa / G2bbbb rows ((i,j),(k,l)) with {i,l} = pair 1, {k,j} = pair 2
