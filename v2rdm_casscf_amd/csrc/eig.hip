@@ -918,10 +918,14 @@ k_z(const EigBlock *__restrict__ blocks, const double *__restrict__ x,
 }  // namespace
 
 namespace {
-// Blocks of 33 to 64 that the chip holds at once with 1024 threads each, two a CU: up to
-// there a launch waits for one block's latency (about 400 blocks of 64 chains: 715 against
-// 786 us), beyond for the throughput, which 256 threads have (about 800: 1295 against 1055
-// us).  Blocks up to 32 take 256 threads at any count (128 chains: 201 against 328 us with a
+// Blocks of 33 to 64 take 1024 threads each up to this many in a launch, 256 beyond.  One
+// workgroup of 1024 fits a CU (80 registers a thread), four of 256 do.  Up to 256 blocks, one
+// a CU, a launch waits for one block's latency: blocks of 50 indices 365 us against 565 with
+// 256 threads, of 64 513 against 731.  Above 512 the throughput counts, which 256 threads
+// have: 520 blocks of 50 1052 against 837 us, 550 of 64 1528 against 1213.  Between them it
+// depends on the sizes: the 400 or so of 64 chains, 33 to 64 mixed and the largest first, 715
+// against 786 us, but 400 equal blocks of 50 726 against 622, 350 of 64 1024 against 920.
+// Blocks up to 32 take 256 threads at any count (128 chains: 201 against 328 us with a
 // wavefront each).
 constexpr int kFewMid = 512;
 }

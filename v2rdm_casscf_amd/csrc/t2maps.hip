@@ -27,8 +27,9 @@ struct AddTo {
 // orbitals, with the residual update: 162 us with the entries streamed in first, 87 us; a
 // row a thread of rowterms.hpp, without the update: 168 us; the bytes 75 us).  The lists
 // follow each other in program order within the wavefront, so the sums have one order.  A
-// list is a chain of item, pair tables and D2 entry: latency, hence five workgroups a CU.
-__global__ void __launch_bounds__(kBlock, 5)
+// list is a chain of item, pair tables and D2 entry: latency, hence four workgroups a CU,
+// what the sums' 32 KB of LDS allow.
+__global__ void __launch_bounds__(kBlock, 4)
 k_t2_au(const DevLayout *__restrict__ Lp, T2Tab T, const double *__restrict__ x, double *__restrict__ Ax,
         const double *__restrict__ done, const double *__restrict__ dotv, double *__restrict__ rowpart, CgFuse fz,
         int64_t part0)
