@@ -285,6 +285,24 @@ __device__ __forceinline__ Eval evaluate(const RedBufs &B, const Place &pl, cons
     return e;
 }
 
+// ---- plan -------------------------------------------------------------------
+// The records of the listed entries and cells from their orbitals: on the host, with the
+// upload, they were most of the plan (H50: 1.5 of 1.9 ms).
+__global__ void __launch_bounds__(kNT)
+k_red_records(const RedProb *__restrict__ prob)
+{
+    const RedProb &p = prob[blockIdx.y];
+    const int first = blockIdx.x * kNT + threadIdx.x, step = gridDim.x * kNT;
+    for (int i = first; i < p.nab; i += step) {
+        const RedKey k(p.ab_key[i]);
+        p.ab[i] = make_ab_rec(p.R, k.p, k.q, k.r, k.s);
+    }
+    for (int i = first; i < p.ncell; i += step) {
+        const RedKey k(p.cell_key[i]);
+        p.cell[i] = make_cell_rec(p.R, k.p, k.q, k.r, k.s);
+    }
+}
+
 // ---- start of a solve -------------------------------------------------------
 // These passes and the last one, k_red_y, meet the full rows of rhs and y, where the rows of
 // neighbouring entries lie apart: lines that several wavefronts touch bound them (H50: 258, 345,
@@ -836,7 +854,7 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     int64_t total = 0;
     for (int q = 0; q < np_; q++) {
         RedProb &p = prob[q];
-        if (!make_red_layout(*L[q], dev[q], p.R, work[q])) return false;
+        if (!make_red_layout(*L[q], dev[q], p.R, work[q], false)) return false;
         p.full = d_dev + q;
         full_ = full_ && p.R.L.q2 && p.R.L.g2 && p.R.cells;
         p.oD = nD_;
@@ -848,14 +866,9 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
         nS_ += p.R.nS;
         nM_ += p.R.nM + 1;
     }
-    // the tiles of every problem's three lists, in one array, and the listed entries
+    // the tiles of every problem's four lists, in one array
     std::vector<RedTile> tl;
-    std::vector<AbRec> ab;
-    std::vector<CellRec> cell;
-    std::vector<uint64_t> bits;
-    std::vector<uint32_t> rank;
-    std::vector<int32_t> rowtab;
-    std::vector<size_t> to(4 * np_), ao(np_), co(np_), bo(np_), ro(np_);
+    std::vector<size_t> to(4 * np_);
     auto list = [&](int q, int k) -> const std::vector<Segment> & {
         return k == 0 ? work[q].start : k == 1 ? work[q].dir : k == 2 ? work[q].res : work[q].norm;
     };
@@ -867,11 +880,6 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
         for (int k = 0; k < 4; k++)
             for (const Segment &s : list(q, k)) ntl += (size_t)((s.count + items(q, s) - 1) / items(q, s));
     tl.reserve(ntl);
-    // a problem's lists follow each other's; the first's are taken as they are
-    auto join = [](auto &all, auto &one) {
-        if (all.empty()) all = std::move(one);
-        else all.insert(all.end(), one.begin(), one.end());
-    };
     for (int q = 0; q < np_; q++) {
         tiles[q] = 1;
         for (int k = 0; k < 4; k++) {
@@ -884,15 +892,6 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
             tiles[q] = std::max<int64_t>(tiles[q], prob[q].ntile[k]);
         }
         total += tiles[q];
-        ao[q] = ab.size();
-        co[q] = cell.size();
-        bo[q] = bits.size();
-        ro[q] = rowtab.size();
-        join(rowtab, work[q].rowtab);
-        join(bits, work[q].bits);
-        join(rank, work[q].rank);
-        join(ab, work[q].ab);
-        join(cell, work[q].cell);
     }
     // workgroups in proportion to the tiles, at least one a problem
     std::vector<int> blk;
@@ -904,37 +903,56 @@ bool RedCG::build(const std::vector<const Layout *> &L, const std::vector<DevLay
     }
     nblk_ = (int)blk.size();
     if (nblk_ > kRedMaxBlocks) throw std::logic_error("reduced CG: more workgroups than partial sums");
-    // one allocation, regions on 256-byte boundaries
+    // one allocation, regions on 256-byte boundaries: the tiles, then what is uploaded beside
+    // them in one piece, then the records
     auto room = [](size_t n) { return (n + 255) / 256 * 256; };
-    const size_t tb = sizeof(RedTile) * tl.size(), abb = sizeof(AbRec) * ab.size(),
-                 cb = sizeof(CellRec) * cell.size(), bb = sizeof(uint64_t) * bits.size(), rb = sizeof(uint32_t) * rank.size(),
-                 wb = sizeof(int32_t) * rowtab.size();
-    HIPCHK(hipMalloc(&d_work_, room(tb) + room(abb) + room(cb) + room(bb) + room(rb) + room(wb)));
-    char *at = static_cast<char *>(d_work_);
-    auto put = [&](const void *src, size_t n) {
-        char *p = at;
-        if (n) HIPCHK(hipMemcpy(p, src, n, hipMemcpyHostToDevice));
-        at += room(n);
+    const size_t tb = room(sizeof(RedTile) * tl.size());
+    size_t sb = 0, nb = 0;
+    auto bytes = [](const auto &v) { return sizeof(v[0]) * v.size(); };
+    for (int q = 0; q < np_; q++) {
+        const RedWork &w = work[q];
+        sb += room(bytes(w.ab_key)) + room(bytes(w.cell_key)) + room(bytes(w.bits)) + room(bytes(w.rank)) +
+              room(bytes(w.rowtab));
+        nb += room(sizeof(AbRec) * w.ab_key.size()) + room(sizeof(CellRec) * w.cell_key.size());
+    }
+    HIPCHK(hipMalloc(&d_work_, tb + sb + nb));
+    char *const base = static_cast<char *>(d_work_);
+    std::vector<char> stage(sb);
+    size_t at = 0;
+    auto put = [&](const auto &v) {
+        using T = std::decay_t<decltype(v[0])>;
+        if (!v.empty()) std::memcpy(stage.data() + at, v.data(), bytes(v));
+        const T *p = reinterpret_cast<const T *>(base + tb + at);
+        at += room(bytes(v));
         return p;
     };
-    const RedTile *dt = reinterpret_cast<const RedTile *>(put(tl.data(), tb));
-    const AbRec *da = reinterpret_cast<const AbRec *>(put(ab.data(), abb));
-    const CellRec *dc = reinterpret_cast<const CellRec *>(put(cell.data(), cb));
-    const uint64_t *db = reinterpret_cast<const uint64_t *>(put(bits.data(), bb));
-    const uint32_t *dr = reinterpret_cast<const uint32_t *>(put(rank.data(), rb));
-    const int32_t *dw = reinterpret_cast<const int32_t *>(put(rowtab.data(), wb));
+    char *rec = base + tb + sb;
     for (int q = 0; q < np_; q++) {
-        prob[q].R.rowtab = dw + ro[q];
-        for (int k = 0; k < 4; k++) prob[q].tile[k] = dt + to[4 * q + k];
-        prob[q].ab = da + ao[q];
-        prob[q].cell = dc + co[q];
-        prob[q].bits = db + bo[q];
-        prob[q].rank = dr + bo[q];
+        RedProb &p = prob[q];
+        const RedWork &w = work[q];
+        for (int k = 0; k < 4; k++) p.tile[k] = reinterpret_cast<const RedTile *>(base) + to[4 * q + k];
+        p.ab_key = put(w.ab_key);
+        p.cell_key = put(w.cell_key);
+        p.bits = put(w.bits);
+        p.rank = put(w.rank);
+        p.R.rowtab = put(w.rowtab);
+        p.nab = (int)w.ab_key.size();
+        p.ncell = (int)w.cell_key.size();
+        p.ab = reinterpret_cast<AbRec *>(rec);
+        rec += room(sizeof(AbRec) * p.nab);
+        p.cell = reinterpret_cast<CellRec *>(rec);
+        rec += room(sizeof(CellRec) * p.ncell);
     }
+    HIPCHK(hipMemcpy(base, tl.data(), sizeof(RedTile) * tl.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(base + tb, stage.data(), sb, hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&d_blk_, sizeof(int) * blk.size()));
     HIPCHK(hipMemcpy(d_blk_, blk.data(), sizeof(int) * blk.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMalloc(&d_prob_, sizeof(RedProb) * prob.size()));
     HIPCHK(hipMemcpy(d_prob_, prob.data(), sizeof(RedProb) * prob.size(), hipMemcpyHostToDevice));
+    // (the solves' streams do not wait for this one)
+    hipLaunchKernelGGL(k_red_records, dim3(std::max(1, kRedMaxBlocks / np_), np_), dim3(kNT), 0, nullptr, d_prob_);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(nullptr));
     return true;
 }
 

@@ -29,6 +29,8 @@ enum RedKind : int {
 struct RedWork {
     // start and end of a solve, direction, residual, norms
     std::vector<Segment> start, dir, res, norm;
+    // the orbitals of the listed D2ab entries and cells (RedKey), in order, and their records
+    std::vector<uint32_t> ab_key, cell_key;
     std::vector<AbRec> ab;
     std::vector<CellRec> cell;
     std::vector<uint64_t> bits;             // one a cell, set for those with a CellRec; every
@@ -37,9 +39,17 @@ struct RedWork {
     std::vector<uint32_t> rank;             // CellRecs before each word's first
 };
 
+// (pq|rs) of a listed entry or cell, eight bits an orbital (at most 255, layout.cc)
+struct RedKey {
+    static V2G_HD uint32_t of(int p, int q, int r, int s) { return (uint32_t)p | (uint32_t)q << 8 | (uint32_t)r << 16 | (uint32_t)s << 24; }
+    int p, q, r, s;
+    explicit V2G_HD RedKey(uint32_t k) : p(k & 255), q(k >> 8 & 255), r(k >> 16 & 255), s(k >> 24) {}
+};
+
 // false: the layout has rows the reduced form does not cover (T1, T2,
-// spin-adapted Q2 / G2), or sizes beyond its 32-bit places.  R.rowtab is left to the caller.  dev: the layout's device view (tables of either side)
-bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWork &w);
+// spin-adapted Q2 / G2), or sizes beyond its 32-bit places.  R.rowtab is left to the caller.  dev: the layout's
+// device view (tables of either side).  records = false: RedWork::ab and cell stay empty
+bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWork &w, bool records = true);
 
 #if defined(__HIPCC__)
 
@@ -58,11 +68,13 @@ struct RedProb {
     int64_t oD, oR, oS, oM;
     const RedTile *tile[4];             // RedWork's lists, cut into tiles
     int ntile[4];
-    const AbRec *ab;
-    const CellRec *cell;
+    AbRec *ab;
+    CellRec *cell;
     const uint64_t *bits;
     const uint32_t *rank;
     int b0, nb;
+    const uint32_t *ab_key, *cell_key;  // where the records come from
+    int nab, ncell;
 };
 
 // the vectors of a solve (concatenated over the problems); pairs are indexed by the
@@ -112,7 +124,7 @@ public:
 private:
     RedProb *d_prob_ = nullptr;
     int *d_blk_ = nullptr;              // problem of each workgroup
-    void *d_work_ = nullptr;            // segments and tile prefixes
+    void *d_work_ = nullptr;            // tiles, lists and tables
     int np_ = 0, nblk_ = 0;
     bool full_ = true;
     int64_t nD_ = 0, nR_ = 0, nS_ = 0, nM_ = 0;

@@ -3,7 +3,7 @@
 
 namespace v2g {
 
-bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWork &w)
+bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWork &w, bool records)
 {
     if (!Lt.xsegs_t2.empty() || Lt.dimx >= ((int64_t)1 << 30)) return false;
     R.L = dev;
@@ -117,9 +117,10 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
             with[first(b[K])].push_back(K);
             with[second(b[K])].push_back(K);
         }
-        size_t listed = w.cell.size();
+        size_t listed = w.cell_key.size();
         for (int I = 0; I < Lt.gems_aa[h]; I++) listed += with[first(b[I])].size() + with[second(b[I])].size() - 1;
-        w.cell.reserve(listed);
+        w.cell_key.reserve(listed);
+        if (records) w.cell.reserve(listed);
         for (int I = 0; I < Lt.gems_aa[h]; I++) {
             const int p = first(b[I]), q = second(b[I]);
             const auto &u = with[p], &v = with[q];
@@ -129,19 +130,25 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
                 j += j < v.size() && v[j] == K;
                 const int64_t c = (int64_t)I * Lt.gems_aa[h] + K;
                 w.bits[word + c / 64] |= (uint64_t)1 << (c % 64);
-                w.cell.push_back(rows::make_cell_rec(H, p, q, first(b[K]), second(b[K])));
+                w.cell_key.push_back(RedKey::of(p, q, first(b[K]), second(b[K])));
+                if (records) w.cell.push_back(rows::make_cell_rec(H, p, q, first(b[K]), second(b[K])));
             }
         }
     }
     const int *b0 = Lt.bab.data() + Lt.bab_off[0];
-    w.ab.reserve((size_t)(2 * ndiag));
+    w.ab_key.reserve((size_t)(2 * ndiag));
     for (int d = 0; d < Lt.amo; d++)
         for (int n = 0; n < Lt.gems_ab[0]; n++) {
             const int p = first(b0[n]), q = second(b0[n]);
-            w.ab.push_back(rows::make_ab_rec(H, d, d, p, q));
-            if (p != q) w.ab.push_back(rows::make_ab_rec(H, p, q, d, d));
+            w.ab_key.push_back(RedKey::of(d, d, p, q));
+            if (p != q) w.ab_key.push_back(RedKey::of(p, q, d, d));
         }
-    const int64_t nout = (int64_t)w.ab.size();
+    if (records)
+        for (const uint32_t key : w.ab_key) {
+            const RedKey k(key);
+            w.ab.push_back(rows::make_ab_rec(H, k.p, k.q, k.r, k.s));
+        }
+    const int64_t nout = (int64_t)w.ab_key.size();
     // listed cells before each word's first
     w.rank.resize(w.bits.size());
     for (size_t i = 0, n = 0; i < w.bits.size(); i++) {
@@ -212,7 +219,8 @@ bool make_red_layout(const Layout &Lt, const DevLayout &dev, RedLayout &R, RedWo
         w.norm.push_back(s);
     }
     seg(w.norm, RK_LIST_AB, 0, 0, 0, 0, nout, 0, 0);
-    seg(w.norm, RK_SHARED, 0, 0, (int)w.cell.size(), 0, 4 * (int64_t)w.cell.size(), 0, 0);
+    const int64_t ncell = (int64_t)w.cell_key.size();
+    seg(w.norm, RK_SHARED, 0, 0, (int)ncell, 0, 4 * ncell, 0, 0);
     cat(w.norm, bulk);
     return true;
 }
