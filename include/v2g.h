@@ -189,7 +189,12 @@ typedef struct v2g_stats {
     long long cg_iters;          /* total CG iterations                   */
     int converged;
     double energy_primal, energy_dual, ep, ed, mu;
-    double t_cg, t_xz, t_total;  /* seconds: CG phase, Update_xz, loop    */
+    double t_cg, t_xz, t_total;  /* seconds: CG phase, Update_xz, loop.   */
+                                 /* The phases meet where the host reads  */
+                                 /* the CG's last status; the plain CG's  */
+                                 /* last pass (y of the rows with a       */
+                                 /* primal entry of their own), enqueued  */
+                                 /* after it, counts in t_xz              */
     int eig_sweeps;              /* block-Jacobi sweeps, last Update_xz   */
     int precond_active;          /* preconditioner of the last CG solve   */
     long long cg_iters_train;    /* CG iterations during the training phase */

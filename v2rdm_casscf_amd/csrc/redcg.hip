@@ -14,10 +14,12 @@
 //   norms       r.r, r.p and p.p of the self rows, one read of s
 // ||p_self||^2 of the next direction follows from the three norms (p' = r + beta p).
 //
-// What bounds it: at (50e,50o) the bytes of the cells (redrows.hpp), 85 us for each of
-// the three passes, 255 us an iteration against 590 us with the entries in block order
-// (index chains and a divergent branch for every D1 term) and 796 us for the general
-// form; 58 against 74 us at (24e,24o) without symmetry, latency-bound: 23 us at (10e,8o).
+// What bounds it: at (50e,50o) memory traffic.  By the HBM counters the three passes move
+// 334, 377 and 470 MB in 86, 83 and 82 us (3.9, 4.5 and 5.7 TB/s; a large copy has 4.5): 1.18
+// GB an iteration where its vectors are 0.80, lines of listed cells being fetched twice.
+// 255 us an iteration against 590 us with the entries in block order (index chains and a
+// divergent branch for every D1 term) and 796 us for the general form; 58 against 74 us at
+// (24e,24o) without symmetry; 23 us at (10e,8o), three dependent launches.
 // Norms and residual are two launches because together they need more registers than
 // four workgroups a CU leave (200 us in one, spilling or at three a CU).  Every
 // workgroup re-sums the partials of the pass before (at most kRedMaxBlocks of them, in

@@ -658,7 +658,8 @@ V2G_HD inline int ab_transposed(const DevLayout &L, int h, int pos)
 // chunks of 64 columns, a wavefront on 8 rows x 8 columns of a whole chunk: the G2 rows'
 // D2ab operand runs along the transposed rows in half of the cases, along the columns in
 // the others, and either way a wavefront reads pieces of 64 bytes (H50, A x: 334 -> 287 us
-// against whole rows).  Blocks below kTileDim stay in whole rows: their operands lie in L2
+// against whole rows; A x itself is then written in such pieces too, 351 MB
+// by the HBM counters for 230 MB of rows).  Blocks below kTileDim stay in whole rows: their operands lie in L2
 // anyway, and the tiles' divisions cost 1 - 2 % (15 orbitals, 225 pairs: A x 16.1 against 15.6 us)
 constexpr int kTileDim = 512;
 
