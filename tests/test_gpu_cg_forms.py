@@ -105,3 +105,20 @@ def test_capped_preconditioned_cg_matches_recurrence(amopi, na, nb, pos):
         assert it == n
         assert abs(res - resr) <= 1e-12 * max(r0, resr)
         assert np.linalg.norm(y.cpu().numpy() - yr) <= max(1e-12 * np.linalg.norm(yr), 10 * own)
+
+
+@pytest.mark.parametrize("amopi,na,nb,pos", [([5], 2, 2, "DQG"), ([5], 3, 2, "DQG"), ([5], 2, 2, "DG"),
+                                             ([2, 0, 1, 1, 0, 2, 1, 1], 5, 5, "DQG")])
+def test_cg_past_its_last_digit_stays_finite(amopi, na, nb, pos):
+    """A A^T is singular: iterations beyond the solution's last digit run along directions that
+    A^T maps to zero, where ||A^T p||^2 is what rounding leaves of it.  As a sum of squares that
+    is (eps ||p||)^2, and y stays finite; a difference of squares can be zero or negative."""
+    s, L = _pair(amopi, na, nb, pos, True, True)
+    rng = np.random.default_rng(1)
+    rhs = L.Au(rng.normal(size=L.dimx))
+    for n in (150, 250, 400):
+        y = _dev(np.zeros(L.ncon))
+        it, res = s.cg_solve(_dev(rhs), y, 0.0, n)
+        print(f"[cg {amopi} {pos} n {n}] |r| {res:.1e} |y| {float(y.norm()):.1e}", flush=True)
+        assert it == n and np.isfinite(res)
+        assert bool(torch.isfinite(y).all())

@@ -12,7 +12,12 @@
 //   direction   beta from the last norms; v, nu, p; ||A^T p||^2
 //   residual    alpha; u, w, mu, om; explicit rows of r and y
 //   norms       r.r, r.p and p.p of the self rows, one read of s
-// ||p_self||^2 of the next direction follows from the three norms (p' = r + beta p).
+// ||p_self||^2 of the next direction follows from the three norms (p' = r + beta p) on the
+// rows whose own entry of A^T p is +-p alone.  The G2ba rows that maximal-spin rows read have
+// p_self - P p_ms there, squared entry by entry in the direction pass: on a direction that A^T
+// maps to zero the two cancel, and the squares written out would leave eps ||p||^2 of either
+// sign where the recurrence has (eps ||p||)^2 (a solve that goes on past its last digit then
+// took steps of any size, to NaN within some 40 iterations).
 //
 // What bounds it: at (50e,50o) memory traffic.  By the HBM counters the three passes move
 // 334, 377 and 470 MB in 86, 83 and 82 us (3.9, 4.5 and 5.7 TB/s; a large copy has 4.5): 1.18
@@ -160,6 +165,11 @@ struct Axpy {
     const double *__restrict__ y;
     double b;
     __device__ __forceinline__ double operator[](int64_t i) const { return fma(b, y[i], a[i]); }
+};
+
+struct Sum {
+    Axpy a, b;
+    __device__ __forceinline__ double operator[](int64_t i) const { return a[i] + b[i]; }
 };
 
 struct Ptr {
@@ -370,7 +380,7 @@ k_red_aty(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
 }
 
 // visits the self rows of a start-list item: fn(slot, full row, D2 / D1 part of x
-// minus the maximal-spin part of m)
+// minus the maximal-spin part of m, whether a maximal-spin row reads it)
 template <class X, class M, class F>
 __device__ __forceinline__ void self_slots(const RedLayout &R, const DevLayout &Lo, const Segment &sg,
                                            int64_t i, int lane, const X &x, const M &m, F fn)
@@ -378,12 +388,12 @@ __device__ __forceinline__ void self_slots(const RedLayout &R, const DevLayout &
     if (is_ab(sg)) {
         AbEntry a;
         if (!start_entry(R, sg, i, a)) return;
-        auto one = [&](int f, double o) { fn(R.soff[f] + a.pos, self_row_ab(R, f, a), o); };
+        auto one = [&](int f, double o, bool ms = false) { fn(R.soff[f] + a.pos, self_row_ab(R, f, a), o, ms); };
         const SelfAb<X> o(R, a, x);
         if (R.L.q2) one(SF_Q2AB, o.q2);
         if (R.L.g2) {
             one(SF_G2AB, o.g1);
-            one(SF_G2BA, o.g2 - ms_part(R, a.p, a.q, a.r, a.s, m));
+            one(SF_G2BA, o.g2 - ms_part(R, a.p, a.q, a.r, a.s, m), ms_reads(R, a.p, a.q, a.r, a.s));
             one(SF_G2X, o.x);
             one(SF_G2Y, o.x);
             one(SF_G2A, o.ga);
@@ -397,34 +407,38 @@ __device__ __forceinline__ void self_slots(const RedLayout &R, const DevLayout &
         if (!R.L.q2) return;
         const AbEntry a = cell_entry(R, sg.h, i);
         for (int sp = 0; sp < 2; sp++)
-            fn(R.soff[SF_Q2AA + sp] + sg.start + i, Lo.rowoff[RF_Q2AA][sp][sg.h] + i, self_row_aa(R, sp, a, x));
+            fn(R.soff[SF_Q2AA + sp] + sg.start + i, Lo.rowoff[RF_Q2AA][sp][sg.h] + i, self_row_aa(R, sp, a, x), false);
     } else if (sg.kind == XS_D1 && lane == 0) {
-        fn(q1_slot(R, sg, i), self_row_d1(Lo, sg.sub, sg.h, i), x[sg.start + i]);
+        fn(q1_slot(R, sg, i), self_row_d1(Lo, sg.sub, sg.h, i), x[sg.start + i], false);
     }
 }
 
-// s = rhs - y - B2 t + P y_ms on the self rows, and the sum of its squares
+// s = rhs - y - B2 t + P y_ms on the self rows, and the sums of its squares
 __global__ void __launch_bounds__(kNT, 4)
 k_red_self(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B,
            const double *__restrict__ rhs, const double *__restrict__ y)
 {
-    __shared__ double sh[kWaves];
+    __shared__ double sh[2 * kWaves];
     const Place pl = place(prob, blk);
     const View V = view(B, *pl.pr, pl.prob, 0);
     if (V.scal[RS_DONE] != 0.0) return;
     const RedLayout &R = pl.pr->R;
     const DevLayout &Lo = *pl.pr->full;
     const Ptr t{V.t}, ms{y + (R.nM ? Lo.rowoff[RF_MAXSPIN][0][0] : 0)};
-    double ss[1] = {0.0};
+    double ss[2] = {0.0, 0.0};
     for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
-        self_slots(R, Lo, sg, i, lane, t, ms, [&](int64_t slot, int64_t row, double o) {
+        self_slots(R, Lo, sg, i, lane, t, ms, [&](int64_t slot, int64_t row, double o, bool ms) {
             const double v = rhs[row] - y[row] - o;
             V.s[slot] = v;
-            ss[0] += v * v;
+            ss[0] += ms ? 0.0 : v * v;
+            ss[1] += ms ? v * v : 0.0;
         });
     });
-    block_sums<1>(ss, sh);
-    if (threadIdx.x == 0) *part(B, P_RR2, pl.gb) = ss[0];
+    block_sums<2>(ss, sh);
+    if (threadIdx.x == 0) {
+        *part(B, P_RR2, pl.gb) = ss[0];
+        *part(B, P_RR1, pl.gb) = ss[1];
+    }
 }
 
 // g = B2^T s, and r = rhs - A (A^T y) on the explicit rows
@@ -487,7 +501,7 @@ k_red_expl(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     });
     block_sums<1>(rr, sh);
     if (threadIdx.x == 0) {
-        *part(B, P_RR1, pl.gb) = rr[0];
+        *part(B, P_RR1, pl.gb) += rr[0];
         *part(B, P_RP, pl.gb) = 0.0;
         *part(B, P_PP, pl.gb) = 0.0;
     }
@@ -575,17 +589,12 @@ k_red_dir(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs
         } else if (sg.kind == RK_MVEC) {
             V.nu1[i] = nu[i];
         } else {
-            // maximal-spin row: (A A^T p) = P^T P p_ms - P^T p_self, and its share
-            // of ||A^T p||^2 beyond ||p_self||^2
+            // maximal-spin row: (A A^T p) = P^T (P p_ms - p_self), the sum of A^T p over its
+            // G2ba entries, and their squares
             const int64_t m0 = R.L.rowoff[RF_MAXSPIN][0][0];
-            const Axpy ps{V.r + m0, V.p0 + m0, ev.beta};
-            const double self = group_sum(ms_row_self(R, sg.sub, (int)i, lane, d, Ptr{V.s}, v, nu), R.lanes);
-            const double gr = group_sum(ms_row_gram(R, sg.sub, (int)i, lane, ps), R.lanes);
-            if (lane == 0) {
-                const int64_t k = sg.sub * (R.nM / 2) + i;
-                V.ams[k] = gr - self;
-                tt[0] += ps[k] * (gr - 2.0 * self);
-            }
+            const Sum m{nu, Axpy{V.r + m0, V.p0 + m0, ev.beta}};
+            const double a = group_sum(ms_row_self(R, sg.sub, (int)i, lane, d, Ptr{V.s}, v, m, tt), R.lanes);
+            if (lane == 0) V.ams[sg.sub * (R.nM / 2) + i] = -a;
         }
     });
     block_sums<1>(tt, sh);
@@ -685,7 +694,7 @@ template <bool FULL>
 __global__ void __launch_bounds__(kNT, 4)
 k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B, int par)
 {
-    __shared__ double sh[3 * kWaves];
+    __shared__ double sh[4 * kWaves];
     const Place pl = place(prob, blk);
     const View V = view(B, *pl.pr, pl.prob, par);
     if (V.scal[RS_A + 6 * par] != 0.0) return;
@@ -694,12 +703,21 @@ k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
     const bool q2 = FULL || R.L.q2, g2 = FULL || R.L.g2;
     const int nd = FULL ? 1 : R.nblk_d;
     const Ptr u{V.u1}, v{V.v1}, mu{V.mu1}, nu{V.nu1};
-    double n[3] = {0.0, 0.0, 0.0};
+    double n[4] = {0.0, 0.0, 0.0, 0.0};
+    const double rr1 = *part(B, P_RR1, pl.gb);   // of the residual pass
     auto self = [&](double s, double ru, double pv) {
         const double r = fma(c, s, ru), p = fma(d, s, pv);
         n[0] = fma(r, r, n[0]);
         n[1] = fma(r, p, n[1]);
         n[2] = fma(p, p, n[2]);
+    };
+    // a G2ba row; ms: a maximal-spin row reads it
+    auto g2ba = [&](bool ms, double s, double ru, double pv) {
+        const double r = fma(c, s, ru), p = fma(d, s, pv), rr = r * r;
+        n[0] += ms ? 0.0 : rr;
+        n[1] += ms ? 0.0 : r * p;
+        n[2] += ms ? 0.0 : p * p;
+        n[3] += ms ? rr : 0.0;
     };
     for_tiles(pl, 3, [&](const Segment &sg, int64_t i, int) {
         if (sg.kind == RK_CELLS) {
@@ -763,7 +781,7 @@ k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
             }
             if (g2) {
                 self(V.s[R.soff[SF_G2AB] + e], su.g1 - x, sv.g1 - z);
-                self(V.s[R.soff[SF_G2BA] + e], su.g2 - x, sv.g2 - z);
+                g2ba(shared_ms(R, a, o), V.s[R.soff[SF_G2BA] + e], su.g2 - x, sv.g2 - z);
                 self(V.s[R.soff[SF_G2A] + e], fma(f, xa, su.g1), fma(f, za, sv.g1));
                 self(V.s[R.soff[SF_G2B] + e], fma(f, xb, su.gb), fma(f, zb, sv.gb));
             }
@@ -774,7 +792,8 @@ k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
             if (q2) one(SF_Q2AB, su.q2(), sv.q2());
             if (g2) {
                 one(SF_G2AB, su.g1(), sv.g1());
-                one(SF_G2BA, su.g2() - (mu[a.m0] + mu[a.m1]), sv.g2() - (nu[a.m0] + nu[a.m1]));
+                g2ba(a.m0 != R.nM || a.m1 != R.nM, V.s[R.soff[SF_G2BA] + a.pos],
+                     su.g2() - (mu[a.m0] + mu[a.m1]), sv.g2() - (nu[a.m0] + nu[a.m1]));
                 one(SF_G2X, su.x0, sv.x0);
                 one(SF_G2Y, su.x0, sv.x0);
                 one(SF_G2A, su.ga(a), sv.ga(a));
@@ -785,11 +804,12 @@ k_red_norm(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBuf
             self(V.s[q1_slot(R, sg, i)], u[sg.start + i], v[sg.start + i]);
         }
     });
-    block_sums<3>(n, sh);
+    block_sums<4>(n, sh);
     if (threadIdx.x == 0) {
         *part(B, P_RR2, pl.gb) = n[0];
         *part(B, P_RP, pl.gb) = n[1];
         *part(B, P_PP, pl.gb) = n[2];
+        *part(B, P_RR1, pl.gb) = rr1 + n[3];
     }
 }
 
@@ -830,7 +850,7 @@ k_red_y(const RedProb *__restrict__ prob, const int *__restrict__ blk, RedBufs B
     const DevLayout &Lo = *pl.pr->full;
     const Ptr w{V.w}, om{V.om};
     for_tiles(pl, 0, [&](const Segment &sg, int64_t i, int lane) {
-        self_slots(R, Lo, sg, i, lane, w, om, [&](int64_t slot, int64_t row, double o) {
+        self_slots(R, Lo, sg, i, lane, w, om, [&](int64_t slot, int64_t row, double o, bool) {
             y[row] += fma(e, V.s[slot], o);
         });
     });

@@ -91,12 +91,14 @@ struct RedBufs {
 // per-problem scalars.  A slots (direction pass) and B slots (residual pass) are
 // ping-pong pairs indexed by the iteration parity; the rest is read by the host
 enum RedSlot : int {
-    RS_A = 0,        // + 6 parity: done, r.z, d, ||p_self||^2, iterations begun
+    RS_A = 0,        // + 6 parity: done, r.z, d, p.p as in kRedParts, iterations begun
     RS_B = 12,       // + 2 parity: c, e
     RS_DONE = 18, RS_NRM = 20, RS_ITER = 21, RS_TOL = 25, RS_MAXIT = 26, RS_NRM0 = 29
 };
 constexpr int kRedScal = 32;
-constexpr int kRedParts = 5;            // ||t||^2, explicit r.r, self r.r, r.p, p.p
+// squares of A^T p; r.r of the explicit rows and the self rows that maximal-spin rows read;
+// r.r, r.p and p.p of the other self rows
+constexpr int kRedParts = 5;
 
 class RedCG {
 public:

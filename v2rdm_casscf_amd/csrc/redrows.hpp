@@ -285,6 +285,9 @@ V2G_HD inline double ms_part(const RedLayout &R, int p, int q, int r, int s, con
     return v;
 }
 
+// whether ms_part has a term
+V2G_HD inline bool ms_reads(const RedLayout &R, int p, int q, int r, int s) { return R.nM && (s == p || q == r); }
+
 // B2^T (B2 x - P m) on a D1 entry: lane-strided share of R.lanes threads
 template <class X, class M>
 V2G_HD inline double gram_d1(const RedLayout &R, int sp, int h, int64_t item, int lane, const X &x,
@@ -392,20 +395,25 @@ V2G_HD inline double ms_row_gram(const RedLayout &R, int o, int item, int lane, 
 }
 
 // maximal-spin row `item` of orientation o (0: G2ba entries (kl, ii), 1: (ii, kl)):
-// lane-strided share of sum_i p_self over its G2ba rows, p_self = d s + B2 x - P m
+// lane-strided share of sum_i p_self over its G2ba rows, p_self = d s + B2 x - P m.  sq
+// (optional): += the squares of those p_self, each G2ba row once over all maximal-spin rows
 template <class S, class X, class M>
 V2G_HD inline double ms_row_self(const RedLayout &R, int o, int item, int lane, double d, const S &s,
-                                 const X &x, const M &m)
+                                 const X &x, const M &m, double *sq = nullptr)
 {
     const DevLayout &L = R.L;
+    const int g0 = L.gems_ab[0];
     const int pr = L.bab[L.bab_off[0] + item], k = P0(pr), l = P1(pr);
-    // the D1b part: its only row with p == r; the P m parts sum to P^T P m
-    double v = lane == 0 ? (o ? x[d1_col(L, XB_D1B, l, k)] : x[d1_col(L, XB_D1B, k, l)]) : 0.0;
-    v -= ms_row_gram(R, o, item, lane, m);
+    const double own = m[o * g0 + item];
+    double v = 0.0;
     for (int i = lane; i < L.amo; i += R.lanes) {
         // the row's pairs are (q, r) and (s, p)
         const int64_t e = o ? ab_pos(R, l, i, i, k) : ab_pos(R, i, k, l, i);
-        v += d * s[R.soff[SF_G2BA] + e] - x[e];
+        double q = d * s[R.soff[SF_G2BA] + e] - x[e] - own;
+        if (k == l) q -= m[(1 - o) * g0 + L.gab[i * L.amo + i]];   // of both orientations
+        if (i == l) q += o ? x[d1_col(L, XB_D1B, l, k)] : x[d1_col(L, XB_D1B, k, l)];   // p == r
+        v += q;
+        if (sq && !(o && k == l)) *sq += q * q;
     }
     return v;
 }
@@ -688,6 +696,13 @@ V2G_HD inline void cell_rows(const Cell &t, double (&a)[3])
 V2G_HD inline int shared_count(const CellRec &c) { return c.flags & CF_TWO ? 2 : 1; }
 // orientation of (ik|jk); (ki|kj), (ki|jk), (ik|kj) are it xor 3, 1, 2
 V2G_HD inline int shared_or(const CellRec &c, int n) { return c.flags >> (2 * n) & 3; }
+
+// whether a maximal-spin row reads the G2ba row of orientation o of the cell
+V2G_HD inline bool shared_ms(const RedLayout &R, const CellRec &c, int o)
+{
+    const int a = o ^ shared_or(c, 0), b = c.flags & CF_TWO ? o ^ shared_or(c, 1) : 0;
+    return R.nM && (a == 1 || a == 2 || b == 1 || b == 2);
+}
 
 // a shared orbital's D1 and maximal-spin numbers
 struct Shared {
